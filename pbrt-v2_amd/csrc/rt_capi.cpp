@@ -132,13 +132,13 @@ struct rt_scene {
   // traversal copy for rayhierarchy: Morton-sorted triangles in clusters of 64
   float* d_v9s = nullptr;
   uint32_t* d_perm = nullptr;
-  uint32_t* d_sperm = nullptr;  // search-BVH position -> triangle id
   float4* d_cbox = nullptr;
   float4* d_tbox = nullptr;  // AABB of every sorted triangle
   float4* d_tmt = nullptr;   // ray-bvh: leaf-test operands v1, e1, e2 (3 float4 per triangle)
-  // per-ray path: search BVH over the sorted triangles and their leaf-test operands
-  float4* d_snode = nullptr;
+  // per-ray path: search tree and the triangles' records in its order (RhItem)
+  uint4* d_snode = nullptr;
   float4* d_tmts = nullptr;
+  SearchFrame sframe{};
   uint32_t* d_tleaf = nullptr;  // ray-bvh: reference BVH leaf of every original triangle
   uint32_t nclusters = 0;
   int clusters_closest = 0, clusters_occluded = 0;  // 0 = built-in choice
@@ -327,16 +327,24 @@ void sort_clusters(const float* v9, uint32_t ntri, std::vector<float>& v9s,
 }
 
 // Leaf-test operands v1, e1 = v2 - v1, e2 = v3 - v1 (FP32, as the device's make_tri) of the
-// triangles of v9, 3 float4 each.
-std::vector<float4> mt_operands(const float* v9, uint32_t ntri) {
-  std::vector<float4> m(3 * (size_t)ntri);
+// triangles of v9, 3 float4 each.  With `order` (position -> triangle) they come in that order,
+// followed by the triangle's index and ~0u as bits, and kSearchPad records of zeros end them
+// (a zero determinant never passes the strict test).
+std::vector<float4> mt_operands(const float* v9, uint32_t ntri, const uint32_t* order = nullptr) {
+  std::vector<float4> m(3 * ((size_t)ntri + (order ? kSearchPad : 0)),
+                        make_float4(0.f, 0.f, 0.f, 0.f));
   for (uint32_t i = 0; i < ntri; ++i) {
-    const float* p = v9 + 9 * (size_t)i;
+    const float* p = v9 + 9 * (size_t)(order ? order[i] : i);
     const float e1[3] = {p[3] - p[0], p[4] - p[1], p[5] - p[2]};
     const float e2[3] = {p[6] - p[0], p[7] - p[1], p[8] - p[2]};
     m[3 * (size_t)i] = make_float4(p[0], p[1], p[2], e1[0]);
     m[3 * (size_t)i + 1] = make_float4(e1[1], e1[2], e2[0], e2[1]);
-    m[3 * (size_t)i + 2] = make_float4(e2[2], 0.f, 0.f, 0.f);
+    float4& last = m[3 * (size_t)i + 2];
+    last = make_float4(e2[2], 0.f, 0.f, 0.f);
+    if (order) {
+      const uint32_t bits[2] = {order[i], 0xffffffffu};
+      std::memcpy(&last.y, bits, sizeof bits);
+    }
   }
   return m;
 }
@@ -390,11 +398,11 @@ int fill_item(const RhJob& jb, RhItem& it) {
   it.uv6 = jb.s->d_uv6;
   it.v9s = jb.s->d_v9s;
   it.perm = jb.s->d_perm;
-  it.sperm = jb.s->d_sperm;
   it.cbox = jb.s->d_cbox;
   it.tbox = jb.s->d_tbox;
   it.tmt = jb.s->d_tmt;
   it.snode = jb.s->d_snode;
+  it.sframe = jb.s->sframe;
   it.tmts = jb.s->d_tmts;
   it.tleaf = jb.s->d_tleaf;
   it.ntri = jb.s->ntri;
@@ -706,16 +714,12 @@ int rt_scene_create(rt_ctx* ctx, const float* v9, const float* uv6, uint32_t ntr
     e = upload(s->d_v9s, v9s.data(), v9s.size());
     if (e == hipSuccess) e = upload(s->d_perm, perm.data(), perm.size());
     if (e == hipSuccess) {
-      std::vector<float4> snode;
+      std::vector<uint4> snode;
       std::vector<uint32_t> sorder;
-      build_search_bvh(v9, ntri, snode, sorder);
+      build_search_bvh(v9, ntri, snode, sorder, s->sframe);
       e = upload(s->d_snode, snode.data(), snode.size());
-      if (e == hipSuccess) e = upload(s->d_sperm, sorder.data(), sorder.size());
       if (e == hipSuccess) {
-        std::vector<float> v9o(9 * (size_t)ntri);
-        for (uint32_t i = 0; i < ntri; ++i)
-          std::memcpy(&v9o[9 * (size_t)i], v9 + 9 * (size_t)sorder[i], 9 * sizeof(float));
-        const std::vector<float4> mts = mt_operands(v9o.data(), ntri);
+        const std::vector<float4> mts = mt_operands(v9, ntri, sorder.data());
         e = upload(s->d_tmts, mts.data(), mts.size());
       }
     }
@@ -884,6 +888,8 @@ int rt_scene_set_bvh(rt_scene* s, const rt_gpu_node* nodes, uint32_t nnodes, con
   RT_TRY(upload(s->d_bvh_parent, parent.data(), parent.size()));
   RT_TRY(upload(s->d_bvh_depth, depth.data(), depth.size()));
   RT_TRY(upload(s->d_tleaf, tleaf.data(), tleaf.size()));
+  RT_TRY(launch_set_tleaf(s->d_tmts, s->d_tleaf, s->ntri, nullptr));
+  RT_TRY(hipStreamSynchronize(nullptr));
   s->nroots = nroots;
   s->has_bvh = true;
   return RT_OK;
@@ -896,7 +902,6 @@ int rt_scene_destroy(rt_scene* s) {
   (void)hipFree(s->d_uv6);
   (void)hipFree(s->d_v9s);
   (void)hipFree(s->d_perm);
-  (void)hipFree(s->d_sperm);
   (void)hipFree(s->d_cbox);
   (void)hipFree(s->d_tbox);
   (void)hipFree(s->d_tmt);

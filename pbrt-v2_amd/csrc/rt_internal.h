@@ -69,6 +69,12 @@ struct HitOut {
   float *t, *u, *v, *dpdu, *dpdv;
 };
 
+// Frame of a search tree's node planes: grid cell c of an axis starts at base + c * unit.
+struct SearchFrame {
+  float base[3];
+  float unit;
+};
+
 // One rayhierarchy traversal job: a resident scene, a ray image and its outputs, with the
 // job's scratch (hierarchy nodes, passing-cluster lists, reduction keys) in device memory.
 // A launch group holds any number of jobs of one mode and node type; the kernels find their
@@ -80,15 +86,16 @@ struct RhItem {
   const float* uv6;      // or null
   const float* v9s;      // Morton-sorted traversal copy, clusters of 64
   const uint32_t* perm;  // sorted slot -> original triangle id
-  const uint32_t* sperm; // search-BVH position -> original triangle id (per-ray path)
   const float4* cbox;    // cluster AABBs (min, max)
   const float4* tbox;    // AABB (min, max) of every sorted triangle
   const float4* tmt;     // ray-bvh: leaf-test operands (v1, e1, e2) of every triangle, original
                          // order (null for rayhierarchy)
-  // per-ray path: padded search BVH over the sorted triangles (4 float4 per node), their
-  // leaf-test operands in sorted order, and for ray-bvh the reference BVH leaf of every
-  // original triangle (bit 31 set: not the first primitive of its leaf; ~0u: in no leaf)
-  const float4* snode;
+  // per-ray path: search tree, its frame, and its triangles' records in search order (3 float4
+  // each: leaf-test operands v1, e1, e2, then as bits the original triangle index and, for
+  // ray-bvh, its tleaf entry).  tleaf: ray-bvh's reference BVH leaf of every original triangle
+  // (bit 31 set: not the first primitive of its leaf; ~0u: in no leaf)
+  const uint4* snode;
+  SearchFrame sframe;
   const float4* tmts;
   const uint32_t* tleaf;
   uint32_t ntri;
@@ -149,27 +156,28 @@ struct RhGroup {
 };
 constexpr int kDefaultWalk = 3;
 
-// Search BVH of the per-ray path over triangles in its own search order (see
-// rt_search_bvh.cpp).  Node = 4 float4: child 0 box (lo.xyz, hi.x), (hi.yz, child 1 lo.xy),
-// (lo.z, hi.xyz), (ref0, ref1 as bits, 0, 0).  A ref with bit 31 clear is an interior node
-// index; with bit 31 set it is a leaf of (bits 27..30) + 1 triangles starting at search
-// position (bits 0..26).
-// Boxes are grown outward by the scene's padding.  The depth is at most kSearchDepth.
-#ifndef RT_SEARCH_DEPTH
-#define RT_SEARCH_DEPTH 26
-#endif
-constexpr int kSearchDepth = RT_SEARCH_DEPTH;
-// Most triangles a leaf holds (the ref's count field allows 16).  One: a leaf test costs
-// about as much as a node visit (52 against 64 bytes, 45 against 24 FLOP), and a lane's leaf
-// is then a single test, so the lanes of a wavefront leave the leaf phase together.  Measured
-// on a batch of 64 cluster scenes against caps of 2, 3 and 4: 8.00-8.03 ms per step against
-// 8.18, 8.31-8.43 and 8.44.
-constexpr int kSearchLeaf = 1;
-// Builds the search BVH of `ntri` triangles (v9 in the caller's order): the node array
-// (4 float4 per node) and the search order (position -> triangle index) whose consecutive
-// positions the leaves reference.
-void build_search_bvh(const float* v9, uint32_t ntri, std::vector<float4>& nodes,
-                      std::vector<uint32_t>& order);
+// Search tree of the per-ray path (see rt_search_bvh.cpp): a 4-wide tree over the triangles in
+// their own search order.  A node is one 64-byte line, 4 uint4:
+//   [0..2]  per axis x, y, z: the children's lower planes, then their upper planes, 4 FP16 each,
+//           in units of SearchFrame::unit above the node's grid cell, rounded outward
+//   [3].x   grid cell of the node, 8 bits per axis from bit 0 (cell c starts at base + c * unit);
+//           bits 24..31: the number of interior children ni (they come first)
+//   [3].y   index of the first interior child; child i < ni is node [3].y + i
+//   [3].z   kSearchLeafBit + position of the first leaf's triangle - ni, so that child i >= ni
+//           is the leaf reference [3].z + i (one triangle per leaf)
+// Absent children have lower planes above their upper planes on every axis; should rounding let
+// a ray into one all the same, its reference is the record of some other triangle (the records
+// end with kSearchPad that no ray hits), whose test is harmless.  A depth-first walk
+// that keeps the unvisited children of every node on its path holds at most kSearchStack of
+// them.
+constexpr uint32_t kSearchLeafBit = 0x80000000u;
+constexpr int kSearchDepth = 26;  // interior levels of the binary tree it is collapsed from
+constexpr int kSearchStack = 26;
+constexpr uint32_t kSearchPad = 4;
+// Builds the search tree of `ntri` triangles (v9 in the caller's order): the nodes (4 uint4
+// each), the search order (position -> triangle index) and the frame of the node planes.
+void build_search_bvh(const float* v9, uint32_t ntri, std::vector<uint4>& nodes,
+                      std::vector<uint32_t>& order, SearchFrame& frame);
 
 // Allocation-free trace: a static device array of kNoAllocScratch bytes per device (defined in
 // rt_kernels.hip).  noalloc_setup looks up its address on `device`, which must be current
@@ -178,6 +186,8 @@ constexpr size_t kNoAllocScratch = (size_t)64 << 20;
 constexpr int kMaxDevices = 64;
 int noalloc_setup(int device);
 void* noalloc_scratch(int device);
+// Writes the tleaf entry of every triangle into its record in search order (RhItem::tmts).
+hipError_t launch_set_tleaf(float4* tmts, const uint32_t* tleaf, uint32_t ntri, hipStream_t s);
 // Writes a job table into device memory through the kernel arguments (no copy, no allocation).
 hipError_t launch_write_table(const RhItem& item, RhItem* dst, hipStream_t s);
 

@@ -63,6 +63,11 @@ __device__ __forceinline__ float4 ld4(RT_GLOBAL const float4* p, size_t i) {
 __device__ __forceinline__ float4 ld4(RT_GLOBAL float4* p, size_t i) {
   return ld4((RT_GLOBAL const float4*)p, i);
 }
+typedef uint32_t rt_u4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint4 ldu4(RT_GLOBAL const uint4* p, size_t i) {
+  const rt_u4 v = ((RT_GLOBAL const rt_u4*)p)[i];
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
 
 template <class P>
 __device__ __forceinline__ V3 ld3(P p) { return {p[0], p[1], p[2]}; }
@@ -1502,19 +1507,33 @@ __global__ __launch_bounds__(256) void bvh_unit_kernel(const RhItem* __restrict_
 // ray.  The (t, id) key, the repair-region key and the occlusion flag are the block path's,
 // so the outcome is the same; every ray of a block is handled by exactly one lane, which
 // writes its results directly.
-constexpr uint32_t kSearchLeafBit = 0x80000000u;
-constexpr float kSlack = 0x1p-16f;  // relative slack of the slab-test parameters
+constexpr float kSlack = 0x1p-16f;   // relative slack of the slab-test parameters
+constexpr float kOffSlack = 0x1p-20f;  // the same of a ray's plane offsets
 
-// Slab test of the ray against a padded box: passes when [tn, tf] (tf widened by kSlack)
-// meets [tlo, thi]; tn is the entry parameter used to order the children.
-__device__ __forceinline__ bool slab(V3 o, V3 inv, V3 lo, V3 hi, float tlo, float thi, float& tn) {
-  const float ax = (lo.x - o.x) * inv.x, bx = (hi.x - o.x) * inv.x;
-  const float ay = (lo.y - o.y) * inv.y, by = (hi.y - o.y) * inv.y;
-  const float az = (lo.z - o.z) * inv.z, bz = (hi.z - o.z) * inv.z;
-  tn = fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fminf(az, bz));
-  float tf = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fmaxf(az, bz));
-  tf = tf + fabsf(tf) * kSlack;
-  return tn <= tf && tn <= thi && tf >= tlo;
+// Ray against the planes of a wide node (SearchFrame units): the parameter of plane g + h of an
+// axis (grid cell g, FP16 offset h) is g * ih + c + h * ih with ih = unit / d and c =
+// (base - o) / d.  c is widened outward (down to cn for near planes, up to cf for far ones) by
+// kOffSlack, which covers its own rounding and that of the sums; the scale h * ih + ... rounds
+// once more, which kSlack covers on the far side.
+struct SlabRay {
+  V3 ih, cn, cf;
+};
+__device__ __forceinline__ void slab_axis(float o, float d, float base, float unit, float& ih,
+                                          float& cn, float& cf) {
+  // zero components become tiny ones, so the slab of that axis is (almost) the whole line when
+  // the origin is inside it and empty otherwise
+  const float inv = 1.0f / (fabsf(d) < 0x1p-80f ? (d < 0.f ? -0x1p-80f : 0x1p-80f) : d);
+  const float c = (base - o) * inv, w = fabsf(c) * kOffSlack;
+  ih = inv * unit;
+  cn = c - w;
+  cf = c + w;
+}
+
+typedef _Float16 rt_h2 __attribute__((ext_vector_type(2)));
+// Child c's FP16 plane of a packed quadruple (two words).
+__device__ __forceinline__ float plane(uint32_t w01, uint32_t w23, int c) {
+  const rt_h2 h = __builtin_bit_cast(rt_h2, c < 2 ? w01 : w23);
+  return (float)h[c & 1];
 }
 
 // Hierarchy node of level l above image position (x, y), from the job's node array.  The
@@ -1570,6 +1589,13 @@ __device__ __forceinline__ bool ray_chain_bvh(const RhItem& it, int x, int y, ui
   return true;
 }
 
+// Compare-exchange of two sort keys.
+__device__ __forceinline__ void key_swap(uint32_t& a, uint32_t& b) {
+  const uint32_t lo = min(a, b);
+  b = max(a, b);
+  a = lo;
+}
+
 // Per-ray kernel: one wavefront per work-group, every lane one ray at a time.  The queue holds
 // 64-ray chunks; a wavefront takes a chunk and deals its rays to lanes without one, and when a
 // lane's ray is done it takes the next ray of the chunk (or of the next chunk) at the next
@@ -1606,7 +1632,7 @@ template <int MODE, int NODE, bool BVH>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void ray_path_kernel(
     const RhItem* __restrict__ items, const uint2* __restrict__ rq, uint32_t* __restrict__ ctr,
     uint32_t nchunks, uint32_t walk) {
-  __shared__ uint32_t sStk[kSearchDepth][64];
+  __shared__ uint32_t sStk[kSearchStack][64];
   constexpr uint32_t kQ = MODE == 2 ? kChainQ : kChainQC;
   __shared__ uint32_t sQIdx[kQ], sQRef[kQ], sQMeta[kQ];
   __shared__ float sQT[MODE == 2 ? 1 : kQ];
@@ -1627,8 +1653,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
   uint32_t jk = 0;
   int x = 0, y = 0;
   size_t idx = 0;
-  V3 o = {0.f, 0.f, 0.f}, d = {0.f, 0.f, 1.f}, inv = {1.f, 1.f, 1.f};
-  float tmin = 0.f, tmax = 0.f, tlo = 0.f;
+  V3 o = {0.f, 0.f, 0.f}, d = {0.f, 0.f, 1.f};
+  SlabRay sr{};
+  // tlo, thi: the interval's ends, widened; thi follows the closest bound (spec or best)
+  float tmin = 0.f, tmax = 0.f, tlo = 0.f, thi = 0.f;
   uint64_t best = kMissKey;
   uint32_t rep = kNoKey32;
   bool occluded = false, track_rep = false;
@@ -1640,6 +1668,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
   int sp = 0;
   uint32_t cur = kDone, pl = kDone;
   auto pop = [&]() { return sp > 0 ? sStk[--sp][lane] : kDone; };
+  const float kInf = __int_as_float(0x7f800000);
+  auto widened = [](float t) { return t + fabsf(t) * kSlack; };
   // occlusion: deferred chain candidates (count sQN), the serial of this lane's ray, and the
   // rounds since the queue was last evaluated (wavefront-uniform)
   uint32_t serial = 0, age = 0;
@@ -1698,6 +1728,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
       if ((sQHit >> lane) & 1ull) {  // a bound failed: trace the ray again
         nospec = true;
         spec = kMissKey;
+        thi = kInf;  // best is unset until this pass finds one
         sp = 0;
         cur = 0u;
         pl = kDone;
@@ -1754,14 +1785,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
           d = {glb(r.dx)[idx], glb(r.dy)[idx], glb(r.dz)[idx]};
           tmin = glb(r.tmin)[idx];
           tmax = glb(r.tmax)[idx];
-          // inverse direction for the slab test; zero components become tiny ones, so the
-          // slab of that axis is (almost) the whole line when the origin is inside it and
-          // empty otherwise
-          auto safe = [](float v) {
-            return fabsf(v) < 0x1p-80f ? (v < 0.f ? -0x1p-80f : 0x1p-80f) : v;
-          };
-          inv = {1.0f / safe(d.x), 1.0f / safe(d.y), 1.0f / safe(d.z)};
+          const SearchFrame& f = it.sframe;
+          slab_axis(o.x, d.x, f.base[0], f.unit, sr.ih.x, sr.cn.x, sr.cf.x);
+          slab_axis(o.y, d.y, f.base[1], f.unit, sr.ih.y, sr.cn.y, sr.cf.y);
+          slab_axis(o.z, d.z, f.base[2], f.unit, sr.ih.z, sr.cn.z, sr.cf.z);
           tlo = tmin - fabsf(tmin) * kSlack;
+          thi = MODE == 2 ? widened(tmax) : kInf;
           best = kMissKey;
           rep = kNoKey32;
           occluded = false;
@@ -1786,29 +1815,60 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     const RhItem& it = items[jk];
     const auto snode = glb(it.snode);
     const auto tmts = glb(it.tmts);
-    const auto perm = glb(it.sperm);
-    // node phase
+    // node phase: a lane visits one 4-wide node a step, four 16-byte loads of one line, its
+    // FP16 planes read by mixed-precision FMAs.  The walk is bound by the chain of dependent
+    // node loads and by VALU issue at part-filled wavefronts; four children a node halve the
+    // steps of the binary walk (FP32 boxes, 64 bytes a node): 1 M random segments against
+    // 200,000 triangles 1,206 -> 1,089 us, room task to path depth 3, closest 855 -> 790 and
+    // occlusion 2,516 -> 2,278 us, camera rays of twelve scenes 1,186 -> 1,049 us.
     for (;;) {
       if (act && cur != kDone && !(cur & kSearchLeafBit) && !(kPause && pend)) {
-        const float4 n0 = ld4(snode, 4 * (size_t)cur), n1 = ld4(snode, 4 * (size_t)cur + 1),
-                     n2 = ld4(snode, 4 * (size_t)cur + 2), n3 = ld4(snode, 4 * (size_t)cur + 3);
-        const uint64_t bound = spec < best ? spec : best;
-        float thi = MODE == 2 ? tmax : (bound == kMissKey ? __int_as_float(0x7f800000)
-                                                          : fkey_inv((uint32_t)(bound >> 32)));
-        thi = thi + fabsf(thi) * kSlack;
-        float tn0, tn1;
-        const bool h0 = slab(o, inv, V3{n0.x, n0.y, n0.z}, V3{n0.w, n1.x, n1.y}, tlo, thi, tn0);
-        const bool h1 = slab(o, inv, V3{n1.z, n1.w, n2.x}, V3{n2.y, n2.z, n2.w}, tlo, thi, tn1);
-        const uint32_t r0 = __float_as_uint(n3.x), r1 = __float_as_uint(n3.y);
-        if (h0 && h1) {
-          const bool first1 = tn1 < tn0;
-          sStk[sp++][lane] = first1 ? r0 : r1;
-          cur = first1 ? r1 : r0;
-        } else if (h0 || h1) {
-          cur = h0 ? r0 : r1;
-        } else {
-          cur = pop();
+        const uint4 nx = ldu4(snode, 4 * (size_t)cur), ny = ldu4(snode, 4 * (size_t)cur + 1),
+                    nz = ldu4(snode, 4 * (size_t)cur + 2), nm = ldu4(snode, 4 * (size_t)cur + 3);
+        const float gx = (float)(nm.x & 255u), gy = (float)((nm.x >> 8) & 255u),
+                    gz = (float)((nm.x >> 16) & 255u);
+        const uint32_t ni = nm.x >> 24;
+        // plane parameters of the cell's corner; near and far plane words by the ray's sign
+        const V3 an = {fmaf(gx, sr.ih.x, sr.cn.x), fmaf(gy, sr.ih.y, sr.cn.y),
+                       fmaf(gz, sr.ih.z, sr.cn.z)};
+        const V3 af = {fmaf(gx, sr.ih.x, sr.cf.x), fmaf(gy, sr.ih.y, sr.cf.y),
+                       fmaf(gz, sr.ih.z, sr.cf.z)};
+        const bool sx = sr.ih.x < 0.f, sy = sr.ih.y < 0.f, sz = sr.ih.z < 0.f;
+        const uint32_t nx0 = sx ? nx.z : nx.x, nx1 = sx ? nx.w : nx.y, fx0 = sx ? nx.x : nx.z,
+                       fx1 = sx ? nx.y : nx.w;
+        const uint32_t ny0 = sy ? ny.z : ny.x, ny1 = sy ? ny.w : ny.y, fy0 = sy ? ny.x : ny.z,
+                       fy1 = sy ? ny.y : ny.w;
+        const uint32_t nz0 = sz ? nz.z : nz.x, nz1 = sz ? nz.w : nz.y, fz0 = sz ? nz.x : nz.z,
+                       fz1 = sz ? nz.y : nz.w;
+        // sort key of a child: its entry parameter, the child in the low two bits; kMiss sorts
+        // last (only the order of the visits depends on the lost bits)
+        constexpr uint32_t kMiss = 0xffffffffu;
+        uint32_t key[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float tn = fmaxf(fmaxf(fmaf(plane(nx0, nx1, c), sr.ih.x, an.x),
+                                       fmaf(plane(ny0, ny1, c), sr.ih.y, an.y)),
+                                 fmaf(plane(nz0, nz1, c), sr.ih.z, an.z));
+          const float tf = fminf(fminf(fmaf(plane(fx0, fx1, c), sr.ih.x, af.x),
+                                       fmaf(plane(fy0, fy1, c), sr.ih.y, af.y)),
+                                 fmaf(plane(fz0, fz1, c), sr.ih.z, af.z));
+          const float en = fmaxf(tn, tlo);
+          const bool hit = en <= fminf(fmaf(fabsf(tf), kSlack, tf), thi);
+          key[c] = hit ? (__float_as_uint(en) & ~3u) | (uint32_t)c : kMiss;
         }
+        auto ref = [&](uint32_t k) {
+          const uint32_t c = k & 3u;
+          return (c < ni ? nm.y : nm.z) + c;
+        };
+        key_swap(key[0], key[1]);
+        key_swap(key[2], key[3]);
+        key_swap(key[0], key[2]);
+        key_swap(key[1], key[3]);
+        key_swap(key[1], key[2]);
+        if (key[3] != kMiss) sStk[sp++][lane] = ref(key[3]);
+        if (key[2] != kMiss) sStk[sp++][lane] = ref(key[2]);
+        if (key[1] != kMiss) sStk[sp++][lane] = ref(key[1]);
+        cur = key[0] != kMiss ? ref(key[0]) : pop();
         if (pl == kDone && cur != kDone && (cur & kSearchLeafBit)) {
           pl = cur;
           cur = pop();
@@ -1822,60 +1882,37 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
           act && pl == kDone && cur != kDone && !(cur & kSearchLeafBit) && !(kPause && pend)));
       if (searching <= ((uint32_t)__popcll(__ballot(act)) >> walk)) break;
     }
-    // leaf phase
-    if constexpr (MODE == 2) {
-      // wavefront-uniform rounds over the leaf's (at most kSearchLeaf) triangles, so the queue
-      // can be evaluated between them
+    // leaf phase: the triangle each lane holds
+    {
       const bool haveleaf = act && pl != kDone && !(kPause && pend);
-      const uint32_t first = pl & ((1u << 27) - 1u);
-      const uint32_t cnt = haveleaf ? ((pl >> 27) & 15u) + 1u : 0u;
-      for (uint32_t f = 0; f < (uint32_t)kSearchLeaf; ++f) {
-        if (!__any(f < cnt)) break;
-        if (f < cnt) {
-          const uint32_t slot = first + f;
-          uint32_t ref = perm[slot];
-          bool ok = true;
-          if constexpr (BVH) {
-            const uint32_t bl = glb(it.tleaf)[ref];
-            ok = bl != 0xffffffffu;
-            ref = bl & 0x7fffffffu;
-          }
-          float t, b1, b2;
-          // intersectAllLeaves.cl:177-179; the chain waits in the queue
-          if (ok && mt_strict(o, d, load_mt(tmts, slot), t, b1, b2) && t > tmin && t < tmax) {
-            const uint32_t e = atomicAdd(&sQN, 1u);  // below kChainQ, see kChainQ
-            sQIdx[e] = (uint32_t)idx;
-            sQRef[e] = ref;
-            sQMeta[e] = (jk << 16) | ((uint32_t)lane << 10) | serial;
-            pend = kPause;
-          }
-        }
-        __syncthreads();
-        const uint32_t cq = __builtin_amdgcn_readfirstlane(sQN);
-        if (cq >= kChainFlush) run_chains(cq);
-      }
-      if (haveleaf) pl = kDone;
-    } else {
-      // wavefront-uniform rounds over the leaf's triangles, as for occlusion
-      const bool haveleaf = act && pl != kDone;
-      const uint32_t first = pl & ((1u << 27) - 1u);
-      const uint32_t cnt = haveleaf ? ((pl >> 27) & 15u) + 1u : 0u;
-      for (uint32_t f = 0; f < (uint32_t)kSearchLeaf; ++f) {
-        if (!__any(f < cnt)) break;
-        if (f < cnt) {
-          const uint32_t slot = first + f;
-          const uint32_t id = perm[slot];
-          bool ok = true;
-          uint32_t bl = 0;
-          if constexpr (BVH) {
-            bl = glb(it.tleaf)[id];
-            // first primitive only (6DB / IA secondary rays)
-            ok = bl != 0xffffffffu && !(MODE == 1 && NODE != 2 && (bl & 0x80000000u));
-            bl &= 0x7fffffffu;
-          }
-          float t, b1, b2;
-          if (ok && mt_strict(o, d, load_mt(tmts, slot), t, b1, b2)) {
-            const bool main = t > tmin && t < __int_as_float(0x7f800000);
+      if (haveleaf) {
+        const uint32_t slot = pl & ~kSearchLeafBit;
+        const float4 ta = ld4(tmts, 3 * (size_t)slot), tb = ld4(tmts, 3 * (size_t)slot + 1),
+                     tc = ld4(tmts, 3 * (size_t)slot + 2);
+        Tri T;
+        T.v1 = {ta.x, ta.y, ta.z};
+        T.e1 = {ta.w, tb.x, tb.y};
+        T.e2 = {tb.z, tb.w, tc.x};
+        T.v2 = T.v3 = T.v1;
+        const uint32_t id = __float_as_uint(tc.y);
+        uint32_t bl = __float_as_uint(tc.z);  // ray-bvh: the triangle's reference BVH leaf
+        // in no leaf; or not its leaf's first primitive (6DB / IA secondary rays)
+        const bool ok = !BVH || (bl != 0xffffffffu &&
+                                 !(MODE == 1 && NODE != 2 && (bl & 0x80000000u)));
+        bl &= 0x7fffffffu;
+        float t, b1, b2;
+        if (ok && mt_strict(o, d, T, t, b1, b2)) {
+          if constexpr (MODE == 2) {
+            // intersectAllLeaves.cl:177-179; the chain waits in the queue
+            if (t > tmin && t < tmax) {
+              const uint32_t e = atomicAdd(&sQN, 1u);  // below kChainQ, see kChainQ
+              sQIdx[e] = (uint32_t)idx;
+              sQRef[e] = BVH ? bl : id;
+              sQMeta[e] = (jk << 16) | ((uint32_t)lane << 10) | serial;
+              pend = kPause;
+            }
+          } else {
+            const bool main = t > tmin && t < kInf;
             const bool rp = track_rep && repair_region(b1, b2) && t >= tmin;
             const uint64_t key = hit_key(t, (int32_t)id);
             const bool um = main && key < best && key < spec, ur = rp && fkey(t) < rep;
@@ -1885,7 +1922,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
                 if constexpr (BVH) pass = ray_chain_bvh<NODE>(it, x, y, bl);
                 else pass = ray_chain_rh<MODE, NODE>(it, x, y, id);
                 if (pass) {
-                  if (um) best = key;
+                  if (um) {
+                    best = key;
+                    thi = widened(t);
+                  }
                   if (ur) rep = fkey(t);
                 }
               } else {
@@ -1894,17 +1934,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
                 sQRef[e] = id;
                 sQT[e] = t;
                 sQMeta[e] = (jk << 16) | ((uint32_t)lane << 10) | (um ? 2u : 0u) | (ur ? 1u : 0u);
-                if (um) spec = key;
+                if (um) {
+                  spec = key;
+                  thi = widened(t);
+                }
                 pend = true;
               }
             }
           }
         }
-        __syncthreads();
-        const uint32_t cq = __builtin_amdgcn_readfirstlane(sQN);
-        if (cq >= kChainFlushC) run_chains(cq);
+        pl = kDone;
       }
-      if (haveleaf) pl = kDone;
+      __syncthreads();
+      const uint32_t cq = __builtin_amdgcn_readfirstlane(sQN);
+      if (cq >= (MODE == 2 ? kChainFlush : kChainFlushC)) run_chains(cq);
     }
     if (act && pl == kDone && cur != kDone && (cur & kSearchLeafBit)) {  // a second leaf waits
       pl = cur;
@@ -2472,6 +2515,16 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
   return hipGetLastError();
 }
 
+// See launch_set_tleaf.
+__global__ __launch_bounds__(256) void set_tleaf_kernel(float4* __restrict__ tmts,
+                                                        const uint32_t* __restrict__ tleaf,
+                                                        uint32_t ntri) {
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+  if (i >= ntri) return;
+  float4& r = tmts[3 * (size_t)i + 2];
+  r.z = __uint_as_float(tleaf[__float_as_uint(r.y)]);
+}
+
 // Copies a job table passed by value (in the kernel arguments) into device memory, so that a
 // launch group can be set up without a host-to-device copy.
 __global__ __launch_bounds__(64) void write_table_kernel(RhItem item, RhItem* __restrict__ dst) {
@@ -2506,6 +2559,12 @@ void* noalloc_scratch(int device) {
   if (device < 0 || device >= kMaxDevices) return nullptr;
   std::lock_guard<std::mutex> lk(g_scratch_mu);
   return g_scratch_ptr[device];
+}
+
+hipError_t launch_set_tleaf(float4* tmts, const uint32_t* tleaf, uint32_t ntri, hipStream_t s) {
+  if (!ntri) return hipSuccess;
+  hipLaunchKernelGGL(set_tleaf_kernel, grid1(ntri), dim3(kThreads), 0, s, tmts, tleaf, ntri);
+  return hipGetLastError();
 }
 
 hipError_t launch_write_table(const RhItem& item, RhItem* dst, hipStream_t s) {
