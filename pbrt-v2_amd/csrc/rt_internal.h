@@ -152,7 +152,7 @@ struct RhGroup {
   // block with a traced ray that way without the cluster scan (job cluster lists unused)
   uint32_t ray_clusters;
   int ray_grid;  // work-groups (one wavefront each) of the per-ray kernel; 0 = resident slots
-  int walk;      // per-ray walk rounds stop at <= 1/2^walk searching lanes (1..7)
+  int walk;      // per-ray walk rounds, RT_PARAM_WALK_* 1..7
 };
 constexpr int kDefaultWalk = 3;
 

@@ -1600,217 +1600,184 @@ __device__ __forceinline__ void key_swap(uint32_t& a, uint32_t& b) {
 // 64-ray chunks; a wavefront takes a chunk and deals its rays to lanes without one, and when a
 // lane's ray is done it takes the next ray of the chunk (or of the next chunk) at the next
 // round, so lanes of long traversals do not leave the others idle.  A round walks interior
-// nodes until every lane holds a leaf or is done (Aila and Laine's while-while), then tests
+// nodes until most lanes hold a leaf or are done (Aila and Laine's while-while), then tests
 // the postponed leaves.
 //
-// Occlusion defers the cull chains: a candidate (strict hit inside the ray's interval) goes to
-// a wavefront queue in LDS as {job, ray, triangle or BVH leaf, lane and ray serial}, and the
-// queue is evaluated 64 candidates at a time, one per lane, once it holds kChainFlush.  A
-// passing chain sets the ray's occlusion flag itself and ends the traversal of its lane if the
-// lane still holds that ray.  The ray is occluded when any of its candidates passes its chain,
-// whatever the order, so the result is the same; the lanes no longer run a chain one or two at
-// a time, and a lane does not wait for its candidates before it takes the next ray.  The queue
-// is also evaluated at least every kChainAge rounds (a lane takes at most one ray per round,
-// so the 10-bit serial cannot wrap while an entry waits) and at the end.
-constexpr uint32_t kChainFlush = 32;
-constexpr uint32_t kChainQ = kChainFlush + 64;  // below kChainFlush, plus one per lane a round
-constexpr uint32_t kChainAge = 512;
-// Closest hits defer their chains the same way.  A candidate (a strict hit that beats the
-// lane's bound) is queued with its t, and the lane goes on pruning with it as a provisional
-// bound.  A passing chain merges the candidate into the ray's global key (atomic min, so the
-// order does not matter); the ray's lane waits at its end until its candidates are evaluated.
-// When a candidate that bounded the search fails its chain, the provisional bound may have
-// pruned the answer, so the lane traces the ray again from the root, evaluating each chain at
-// once (chains pass for most hits, so this is rare).  The queue (four words an entry) is four
-// entries shorter than occlusion's so that five work-groups per SIMD still fit the LDS.
-constexpr uint32_t kChainFlushC = 28;
-constexpr uint32_t kChainQC = kChainFlushC + 64;
+// A ray is first traced as if every cull chain passed, which is what they nearly always do:
+// occlusion ends at its first strict hit inside the interval, a closest hit is the nearest
+// strict hit.  That one candidate goes to a wavefront queue in LDS as {ray, triangle or BVH
+// leaf, job} (a closest hit's key goes to the ray's key in memory) and its lane takes the next
+// ray; whenever the queue holds 64 candidates, their chains are evaluated together, one per
+// lane.  A passing chain confirms the candidate: the nearest strict hit is the answer when its
+// chain passes, and any strict hit with a passing chain occludes.  A ray whose candidate
+// failed goes to a second stack in the same LDS, from which idle lanes take it before new rays
+// and trace it from the root again, evaluating each candidate's chain at once and pruning with
+// verified hits only.  So does a primary ray whose nearest repair-region hit (chains aside) lies
+// low enough to matter to the repair pass, which needs verified repair candidates, and a ray
+// whose candidate finds the queue full.
+//
+// Before, each improvement of a ray's bound and every repair-region hit had its chain evaluated
+// and lanes waited for theirs, a quarter of a wavefront at a time, in a launch's tail one by
+// one.  Measured, every block per-ray, with rounds that walk until half of the lanes hold a leaf
+// (1/8 before): torus 512 x 512 closest 247 -> 142 us, occlusion 318 -> 146; room task to path
+// depth 3, the bounces' closest hits 2,816 -> 1,767, occlusion 2,278 -> 1,251; 1 M segments
+// 1,089 -> 688; camera rays of twelve scenes 1,049 -> 609.
+constexpr uint32_t kChainQ = 127;  // below 64 before a round, one more per lane in it
 // Five wavefronts per SIMD (at most 96 VGPRs; the LDS of 20 work-groups per CU): the walk is
 // latency-bound and gains more from resident wavefronts than it loses to a few spilled
 // registers of the chain evaluation.
 template <int MODE, int NODE, bool BVH>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void ray_path_kernel(
     const RhItem* __restrict__ items, const uint2* __restrict__ rq, uint32_t* __restrict__ ctr,
-    uint32_t nchunks, uint32_t walk) {
+    uint32_t nchunks, uint32_t walk16) {
   __shared__ uint32_t sStk[kSearchStack][64];
-  constexpr uint32_t kQ = MODE == 2 ? kChainQ : kChainQC;
-  __shared__ uint32_t sQIdx[kQ], sQRef[kQ], sQMeta[kQ];
-  __shared__ float sQT[MODE == 2 ? 1 : kQ];
-  __shared__ unsigned long long sQHit;  // occlusion: rays found occluded; closest: failed bounds
-  __shared__ uint32_t sQN;
-  constexpr uint32_t kDone = 0xffffffffu;  // not a node reference (leaves hold < 16 triangles)
-  // Rayhierarchy occlusion pauses a lane that queued a candidate: its chain usually passes,
-  // which ends the ray, so walking on is mostly wasted (7% faster on a batch of 64 scenes).
-  // ray-bvh occlusion walks on (pausing made a 3-bounce frame's passes 1.4% slower).
-  constexpr bool kPause = MODE == 2 && !BVH;
+  // candidates [0, qn) and, from the far end, rays to trace again [kChainQ - nf, kChainQ)
+  __shared__ uint32_t sQIdx[kChainQ], sQRef[kChainQ], sQJob[kChainQ];
+  constexpr uint32_t kDone = 0xffffffffu;  // not a reference (positions are below 2^31)
+  const float kInf = __int_as_float(0x7f800000);
+  auto widened = [](float t) { return t + fabsf(t) * kSlack; };
   const int lane = threadIdx.x;
   const uint64_t lanes_below = (1ull << lane) - 1ull;
-  // wavefront-uniform: the chunk being dealt and its next slot
+  // wavefront-uniform: the chunk being dealt and its next slot, the queue's counts
   uint32_t cjob = 0, cblk = 0, cpart = 0, cslot = 64;
+  uint32_t qn = 0, nf = 0;
   bool more = true;
   // lane state
-  bool act = false;
-  uint32_t jk = 0;
-  int x = 0, y = 0;
-  size_t idx = 0;
+  bool act = false, careful = false;
+  uint32_t jk = 0, idx = 0;
   V3 o = {0.f, 0.f, 0.f}, d = {0.f, 0.f, 1.f};
   SlabRay sr{};
-  // tlo, thi: the interval's ends, widened; thi follows the closest bound (spec or best)
+  // tlo, thi: the interval's ends, widened; thi follows the closest bound
   float tmin = 0.f, tmax = 0.f, tlo = 0.f, thi = 0.f;
-  uint64_t best = kMissKey;
-  uint32_t rep = kNoKey32;
-  bool occluded = false, track_rep = false;
-  // whether the lane has a candidate queued (rayhierarchy occlusion: the lane pauses until it
-  // is evaluated); closest: the provisional bound of queued candidates, and whether the ray is
-  // traced again with its chains evaluated at once
-  uint64_t spec = kMissKey;
-  bool pend = false, nospec = false;
+  uint64_t best = kMissKey;   // closest: the nearest hit (verified when careful)
+  uint32_t rep = kNoKey32;    // primary: the nearest repair-region hit (likewise)
+  uint32_t cand = 0;          // chain operand of the candidate: triangle id or BVH leaf
+  bool track_rep = false;
   int sp = 0;
   uint32_t cur = kDone, pl = kDone;
   auto pop = [&]() { return sp > 0 ? sStk[--sp][lane] : kDone; };
-  const float kInf = __int_as_float(0x7f800000);
-  auto widened = [](float t) { return t + fabsf(t) * kSlack; };
-  // occlusion: deferred chain candidates (count sQN), the serial of this lane's ray, and the
-  // rounds since the queue was last evaluated (wavefront-uniform)
-  uint32_t serial = 0, age = 0;
   // the cluster pass sets ctr[4] when it routed any block here
   if (__builtin_amdgcn_readfirstlane(ctr[4]) == 0u) return;
   UnitClaim claim{blockIdx.x % kClaimQueues, 0u};
-  if (lane == 0) {
-    sQN = 0;
-    sQHit = 0ull;
-  }
-  __syncthreads();
-  // Evaluates the cq queued candidates, 64 per pass (one per lane).  Wavefront-uniform, after
-  // a barrier that made the entries visible.
-  auto run_chains = [&](uint32_t cq) {
-    for (uint32_t base = 0; base < cq; base += 64) {
-      const uint32_t e = base + (uint32_t)lane;
-      const bool have = e < cq;
-      const uint32_t meta = have ? sQMeta[e] : 0u;
-      const uint32_t owner = (meta >> 10) & 63u;
-      const uint32_t owner_serial = (uint32_t)__shfl((int)serial, (int)owner);
-      if (have) {
-        const RhItem& oit = items[meta >> 16];
-        const uint32_t ri = sQIdx[e];
-        const int ox = (int)(ri % (uint32_t)oit.g.W), oy = (int)(ri / (uint32_t)oit.g.W);
-        if constexpr (MODE == 2) {
-          bool ok;
-          if constexpr (BVH) ok = ray_chain_bvh<NODE>(oit, ox, oy, sQRef[e]);
-          else ok = ray_chain_rh<MODE, NODE>(oit, ox, oy, sQRef[e]);
-          if (ok) {
-            glb(oit.occ)[ri] = 1;
-            if ((meta & 1023u) == owner_serial) atomicOr(&sQHit, 1ull << owner);
-          }
-        } else {
-          // closest: sQRef holds the triangle id, meta bit 1 a main candidate, bit 0 a
-          // repair-region one
-          const uint32_t id = sQRef[e];
-          const float t = sQT[e];
-          bool ok;
-          if constexpr (BVH) ok = ray_chain_bvh<NODE>(oit, ox, oy, glb(oit.tleaf)[id] & 0x7fffffffu);
-          else ok = ray_chain_rh<MODE, NODE>(oit, ox, oy, id);
-          if (ok) {
-            if (meta & 2u) atomicMin((unsigned long long*)&oit.keys[ri], hit_key(t, (int32_t)id));
-            if (meta & 1u) atomicMin(&oit.repkeys[ri], fkey(t));
-          } else if (meta & 2u) {
-            atomicOr(&sQHit, 1ull << owner);
-          }
-        }
+  auto chain = [&](const RhItem& it, uint32_t ri, uint32_t ref) {
+    const int x = (int)(ri % (uint32_t)it.g.W), y = (int)(ri / (uint32_t)it.g.W);
+    if constexpr (BVH) return ray_chain_bvh<NODE>(it, x, y, ref);
+    else return ray_chain_rh<MODE, NODE>(it, x, y, ref);
+  };
+  auto restart = [&]() {
+    careful = true;
+    best = kMissKey;
+    rep = kNoKey32;
+    thi = MODE == 2 ? widened(tmax) : kInf;
+    sp = 0;
+    cur = 0u;  // interior node 0 (the root)
+    pl = kDone;
+  };
+  // Evaluates the newest `cnt` (at most 64) candidates, one per lane; wavefront-uniform.
+  auto run_chains = [&](uint32_t cnt) {
+    const uint32_t e = qn - cnt + (uint32_t)lane;
+    const bool have = (uint32_t)lane < cnt;
+    bool failed = false;
+    uint32_t ri = 0, job = 0;
+    if (have) {
+      ri = sQIdx[e];
+      job = sQJob[e];
+      const RhItem& it = items[job];
+      const bool ok = chain(it, ri, sQRef[e]);
+      if constexpr (MODE == 2) {
+        if (ok) glb(it.occ)[ri] = 1;
+      } else {
+        // stores of one wavefront to one address keep their order
+        if (!ok) glb(it.keys)[ri] = kMissKey;
       }
+      failed = !ok;
     }
-    __syncthreads();
-    if constexpr (MODE == 2) {
-      if (act && ((sQHit >> lane) & 1ull)) occluded = true;
-      pend = false;  // every queued candidate has been evaluated
-    } else if (act && pend) {
-      pend = false;
-      if ((sQHit >> lane) & 1ull) {  // a bound failed: trace the ray again
-        nospec = true;
-        spec = kMissKey;
-        thi = kInf;  // best is unset until this pass finds one
-        sp = 0;
-        cur = 0u;
-        pl = kDone;
-      }
+    qn -= cnt;
+    const uint64_t fb = __ballot(failed);
+    if (failed) {
+      const uint32_t p = kChainQ - 1u - nf - (uint32_t)__popcll(fb & lanes_below);
+      sQIdx[p] = ri;
+      sQJob[p] = job;
     }
+    nf += (uint32_t)__popcll(fb);
     __syncthreads();
-    if (lane == 0) {
-      sQN = 0;
-      sQHit = 0ull;
-    }
-    __syncthreads();
-    age = 0;
   };
   for (;;) {
-    // deal rays to the lanes without one
+    // deal rays to the lanes without one: first those to trace again, then the queue's
     for (;;) {
       const uint64_t need = __ballot(!act);
-      if (need == 0 || !more) break;
-      if (cslot >= 64) {
-        uint32_t e = 0;
-        if (lane == 0) e = claim_unit(ctr, nchunks, claim, 1);
-        e = __builtin_amdgcn_readfirstlane(e);
-        if (e >= nchunks) {
-          more = false;
-          break;
-        }
-        const uint2 w = rq[e];
-        if (__builtin_amdgcn_readfirstlane(w.x) == 0xffffffffu) continue;  // a block-path block
-        cjob = __builtin_amdgcn_readfirstlane(w.x);
-        const uint32_t c = __builtin_amdgcn_readfirstlane(w.y);
-        const uint32_t nch = ((uint32_t)items[cjob].g.rb + 63u) / 64u;
-        cblk = c / nch;
-        cpart = c - cblk * nch;
-        cslot = 0;
-      }
-      const uint32_t avail = 64u - cslot;
+      if (need == 0) break;
       const uint32_t rank = (uint32_t)__popcll(need & lanes_below);
-      if (!act && rank < avail) {
-        const RhItem& it = items[cjob];
-        const RHGeom& g = it.g;
-        const int top = g.L - 1;
-        const int K = (int)cblk % g.gw[top], J = (int)cblk / g.gw[top];
-        int leaf = 0;
-        bool have = slot_xy(g, K, J, (int)(cpart * 64u + cslot + rank), x, y, leaf) && it.ntri > 0;
-        if (have) {
-          idx = (size_t)y * g.W + x;
-          const RaysDev& r = it.r;
-          if (MODE != 0 && r.valid != nullptr && glb(r.valid)[idx] == 0) have = false;
+      bool got = false;
+      if (nf > 0) {
+        const uint32_t take = min(nf, (uint32_t)__popcll(need));
+        if (!act && rank < take) {
+          idx = sQIdx[kChainQ - nf + rank];
+          jk = sQJob[kChainQ - nf + rank];
+          careful = true;
+          got = true;
         }
-        if (have) {
-          const RaysDev& r = it.r;
-          jk = cjob;
-          o = {glb(r.ox)[idx], glb(r.oy)[idx], glb(r.oz)[idx]};
-          d = {glb(r.dx)[idx], glb(r.dy)[idx], glb(r.dz)[idx]};
-          tmin = glb(r.tmin)[idx];
-          tmax = glb(r.tmax)[idx];
-          const SearchFrame& f = it.sframe;
-          slab_axis(o.x, d.x, f.base[0], f.unit, sr.ih.x, sr.cn.x, sr.cf.x);
-          slab_axis(o.y, d.y, f.base[1], f.unit, sr.ih.y, sr.cn.y, sr.cf.y);
-          slab_axis(o.z, d.z, f.base[2], f.unit, sr.ih.z, sr.cn.z, sr.cf.z);
-          tlo = tmin - fabsf(tmin) * kSlack;
-          thi = MODE == 2 ? widened(tmax) : kInf;
-          best = kMissKey;
-          rep = kNoKey32;
-          occluded = false;
-          spec = kMissKey;
-          pend = false;
-          nospec = false;
-          track_rep = MODE == 0 && !BVH && it.repkeys != nullptr;
-          sp = 0;
-          cur = 0u;  // interior node 0 (the root)
-          pl = kDone;
-          act = true;
-          serial = (serial + 1u) & 1023u;
+        nf -= take;
+        __syncthreads();
+      } else {
+        if (!more) break;
+        if (cslot >= 64) {
+          uint32_t e = 0;
+          if (lane == 0) e = claim_unit(ctr, nchunks, claim, 1);
+          e = __builtin_amdgcn_readfirstlane(e);
+          if (e >= nchunks) {
+            more = false;
+            break;
+          }
+          const uint2 w = rq[e];
+          if (__builtin_amdgcn_readfirstlane(w.x) == 0xffffffffu) continue;  // a block-path block
+          cjob = __builtin_amdgcn_readfirstlane(w.x);
+          const uint32_t c = __builtin_amdgcn_readfirstlane(w.y);
+          const uint32_t nch = ((uint32_t)items[cjob].g.rb + 63u) / 64u;
+          cblk = c / nch;
+          cpart = c - cblk * nch;
+          cslot = 0;
         }
+        const uint32_t avail = 64u - cslot;
+        if (!act && rank < avail) {
+          const RhItem& it = items[cjob];
+          const RHGeom& g = it.g;
+          const int top = g.L - 1;
+          const int K = (int)cblk % g.gw[top], J = (int)cblk / g.gw[top];
+          int x = 0, y = 0, leaf = 0;
+          got = slot_xy(g, K, J, (int)(cpart * 64u + cslot + rank), x, y, leaf) && it.ntri > 0;
+          if (got) {
+            idx = (uint32_t)y * (uint32_t)g.W + (uint32_t)x;
+            if (MODE != 0 && it.r.valid != nullptr && glb(it.r.valid)[idx] == 0) got = false;
+            jk = cjob;
+            careful = false;
+          }
+        }
+        cslot += min(avail, (uint32_t)__popcll(need));
       }
-      cslot += min(avail, (uint32_t)__popcll(need));
+      if (got) {
+        const RhItem& it = items[jk];
+        const RaysDev& r = it.r;
+        o = {glb(r.ox)[idx], glb(r.oy)[idx], glb(r.oz)[idx]};
+        d = {glb(r.dx)[idx], glb(r.dy)[idx], glb(r.dz)[idx]};
+        tmin = glb(r.tmin)[idx];
+        tmax = glb(r.tmax)[idx];
+        const SearchFrame& f = it.sframe;
+        slab_axis(o.x, d.x, f.base[0], f.unit, sr.ih.x, sr.cn.x, sr.cf.x);
+        slab_axis(o.y, d.y, f.base[1], f.unit, sr.ih.y, sr.cn.y, sr.cf.y);
+        slab_axis(o.z, d.z, f.base[2], f.unit, sr.ih.z, sr.cn.z, sr.cf.z);
+        tlo = tmin - fabsf(tmin) * kSlack;
+        track_rep = MODE == 0 && !BVH && it.repkeys != nullptr;
+        const bool again = careful;
+        restart();
+        careful = again;
+        act = true;
+      }
     }
     if (!__any(act)) {
-      const uint32_t cq = __builtin_amdgcn_readfirstlane(sQN);  // the candidates still queued
-      if (cq > 0u) run_chains(cq);
-      break;
+      if (qn == 0) break;  // nothing to trace again either: the deal takes those first
+      run_chains(min(qn, 64u));
+      continue;
     }
     const RhItem& it = items[jk];
     const auto snode = glb(it.snode);
@@ -1822,7 +1789,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     // 200,000 triangles 1,206 -> 1,089 us, room task to path depth 3, closest 855 -> 790 and
     // occlusion 2,516 -> 2,278 us, camera rays of twelve scenes 1,186 -> 1,049 us.
     for (;;) {
-      if (act && cur != kDone && !(cur & kSearchLeafBit) && !(kPause && pend)) {
+      if (act && cur != kDone && !(cur & kSearchLeafBit)) {
         const uint4 nx = ldu4(snode, 4 * (size_t)cur), ny = ldu4(snode, 4 * (size_t)cur + 1),
                     nz = ldu4(snode, 4 * (size_t)cur + 2), nm = ldu4(snode, 4 * (size_t)cur + 3);
         const float gx = (float)(nm.x & 255u), gy = (float)((nm.x >> 8) & 255u),
@@ -1874,113 +1841,98 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
           cur = pop();
         }
       }
-      // walk on while more than 1/2^walk of the lanes holding a ray have neither a postponed
+      // walk on while more than walk16 / 16 of the lanes holding a ray have neither a postponed
       // leaf nor finished (fewer lanes idle behind the longest walk); the others go on from
       // their node in the next round (every round walks at least one step, so each lane
       // advances)
-      const uint32_t searching = (uint32_t)__popcll(__ballot(
-          act && pl == kDone && cur != kDone && !(cur & kSearchLeafBit) && !(kPause && pend)));
-      if (searching <= ((uint32_t)__popcll(__ballot(act)) >> walk)) break;
+      const uint32_t searching = (uint32_t)__popcll(
+          __ballot(act && pl == kDone && cur != kDone && !(cur & kSearchLeafBit)));
+      if (16u * searching <= walk16 * (uint32_t)__popcll(__ballot(act))) break;
     }
     // leaf phase: the triangle each lane holds
-    {
-      const bool haveleaf = act && pl != kDone && !(kPause && pend);
-      if (haveleaf) {
-        const uint32_t slot = pl & ~kSearchLeafBit;
-        const float4 ta = ld4(tmts, 3 * (size_t)slot), tb = ld4(tmts, 3 * (size_t)slot + 1),
-                     tc = ld4(tmts, 3 * (size_t)slot + 2);
-        Tri T;
-        T.v1 = {ta.x, ta.y, ta.z};
-        T.e1 = {ta.w, tb.x, tb.y};
-        T.e2 = {tb.z, tb.w, tc.x};
-        T.v2 = T.v3 = T.v1;
-        const uint32_t id = __float_as_uint(tc.y);
-        uint32_t bl = __float_as_uint(tc.z);  // ray-bvh: the triangle's reference BVH leaf
-        // in no leaf; or not its leaf's first primitive (6DB / IA secondary rays)
-        const bool ok = !BVH || (bl != 0xffffffffu &&
-                                 !(MODE == 1 && NODE != 2 && (bl & 0x80000000u)));
-        bl &= 0x7fffffffu;
-        float t, b1, b2;
-        if (ok && mt_strict(o, d, T, t, b1, b2)) {
-          if constexpr (MODE == 2) {
-            // intersectAllLeaves.cl:177-179; the chain waits in the queue
-            if (t > tmin && t < tmax) {
-              const uint32_t e = atomicAdd(&sQN, 1u);  // below kChainQ, see kChainQ
-              sQIdx[e] = (uint32_t)idx;
-              sQRef[e] = BVH ? bl : id;
-              sQMeta[e] = (jk << 16) | ((uint32_t)lane << 10) | serial;
-              pend = kPause;
-            }
-          } else {
-            const bool main = t > tmin && t < kInf;
-            const bool rp = track_rep && repair_region(b1, b2) && t >= tmin;
-            const uint64_t key = hit_key(t, (int32_t)id);
-            const bool um = main && key < best && key < spec, ur = rp && fkey(t) < rep;
-            if (um || ur) {
-              if (nospec) {
-                bool pass;
-                if constexpr (BVH) pass = ray_chain_bvh<NODE>(it, x, y, bl);
-                else pass = ray_chain_rh<MODE, NODE>(it, x, y, id);
-                if (pass) {
-                  if (um) {
-                    best = key;
-                    thi = widened(t);
-                  }
-                  if (ur) rep = fkey(t);
-                }
-              } else {
-                const uint32_t e = atomicAdd(&sQN, 1u);  // below kChainQC, see kChainQC
-                sQIdx[e] = (uint32_t)idx;
-                sQRef[e] = id;
-                sQT[e] = t;
-                sQMeta[e] = (jk << 16) | ((uint32_t)lane << 10) | (um ? 2u : 0u) | (ur ? 1u : 0u);
-                if (um) {
-                  spec = key;
-                  thi = widened(t);
-                }
-                pend = true;
-              }
+    bool push = false;
+    if (act && pl != kDone) {
+      const uint32_t slot = pl & ~kSearchLeafBit;
+      const float4 ta = ld4(tmts, 3 * (size_t)slot), tb = ld4(tmts, 3 * (size_t)slot + 1),
+                   tc = ld4(tmts, 3 * (size_t)slot + 2);
+      Tri T;
+      T.v1 = {ta.x, ta.y, ta.z};
+      T.e1 = {ta.w, tb.x, tb.y};
+      T.e2 = {tb.z, tb.w, tc.x};
+      T.v2 = T.v3 = T.v1;
+      const uint32_t id = __float_as_uint(tc.y);
+      const uint32_t bl = __float_as_uint(tc.z);  // ray-bvh: the triangle's reference BVH leaf
+      // in no leaf; or not its leaf's first primitive (6DB / IA secondary rays)
+      const bool ok = !BVH || (bl != 0xffffffffu &&
+                               !(MODE == 1 && NODE != 2 && (bl & 0x80000000u)));
+      const uint32_t ref = BVH ? bl & 0x7fffffffu : id;
+      float t, b1, b2;
+      if (ok && mt_strict(o, d, T, t, b1, b2)) {
+        if constexpr (MODE == 2) {
+          if (t > tmin && t < tmax) {  // intersectAllLeaves.cl:177-179
+            if (!careful) {
+              cand = ref;
+              push = true;
+            } else if (chain(it, idx, ref)) {
+              glb(it.occ)[idx] = 1;
+              act = false;
             }
           }
+        } else {
+          const bool main = t > tmin && t < kInf;
+          const bool rp = track_rep && repair_region(b1, b2) && t >= tmin;
+          const uint64_t key = hit_key(t, (int32_t)id);
+          const bool um = main && key < best, ur = rp && fkey(t) < rep;
+          if ((um || ur) && (!careful || chain(it, idx, ref))) {
+            if (um) {
+              best = key;
+              cand = ref;
+              thi = widened(t);
+            }
+            if (ur) rep = fkey(t);
+          }
         }
-        pl = kDone;
       }
-      __syncthreads();
-      const uint32_t cq = __builtin_amdgcn_readfirstlane(sQN);
-      if (cq >= (MODE == 2 ? kChainFlush : kChainFlushC)) run_chains(cq);
+      pl = kDone;
     }
     if (act && pl == kDone && cur != kDone && (cur & kSearchLeafBit)) {  // a second leaf waits
       pl = cur;
       cur = pop();
     }
-    {
-      // evaluate the queue every kChainAge rounds, and every round once no chunk is left to
-      // deal (idle lanes cannot take new rays, and a ray found occluded or bounded early ends
-      // sooner); also once a quarter of the lanes holding a ray wait: closest-hit lanes at the
-      // ray's end for their candidates, paused occlusion lanes as soon as they queue one (if
-      // the chain fails, the lane walks on from where it paused)
-      bool flush = ++age >= kChainAge || !more;
-      const uint32_t nact = (uint32_t)__popcll(__ballot(act));
-      const uint32_t nwait = (uint32_t)__popcll(
-          __ballot(act && pend && (kPause || (cur == kDone && pl == kDone))));
-      flush = flush || (nwait > 0u && 4u * nwait >= nact);
-      if (flush) {
-        const uint32_t cq = __builtin_amdgcn_readfirstlane(sQN);
-        if (cq > 0u) run_chains(cq);
-        age = 0;
+    // rays that are done: a verified result is written; the others queue their candidate, if
+    // they have one
+    if (act && !push && cur == kDone && pl == kDone) {
+      if constexpr (MODE == 2) {
+        act = false;
+      } else if (careful) {
+        if (best != kMissKey) glb(it.keys)[idx] = best;
+        if (track_rep && rep != kNoKey32) glb(it.repkeys)[idx] = rep;
+        act = false;
+      } else {
+        const float tstar = best == kMissKey ? kInf : fkey_inv((uint32_t)(best >> 32));
+        if (rep != kNoKey32 && !(fkey_inv(rep) > tstar - kEps)) restart();
+        else if (best == kMissKey) act = false;
+        else push = true;
       }
     }
-    if (act && occluded) cur = pl = kDone;
-    if (act && cur == kDone && pl == kDone && !pend) {  // the ray is done: its result, then a new ray
-      if constexpr (MODE == 2) {
-        if (occluded) glb(it.occ)[idx] = 1;
-      } else {
-        // passing queued candidates were merged by the evaluation; chains evaluated at once
-        // (a ray traced again) leave their result here
-        if (best != kMissKey) atomicMin((unsigned long long*)&it.keys[idx], best);
-        if (track_rep && rep != kNoKey32) atomicMin(&it.repkeys[idx], rep);
+    const uint64_t pb = __ballot(push);
+    if (pb != 0) {
+      const uint32_t e = qn + (uint32_t)__popcll(pb & lanes_below);
+      const bool room = e < kChainQ - nf;
+      if (push) {
+        if (room) {
+          sQIdx[e] = idx;
+          sQRef[e] = cand;
+          sQJob[e] = jk;
+          if constexpr (MODE != 2) glb(it.keys)[idx] = best;
+          act = false;
+        } else {
+          restart();
+        }
       }
-      act = false;
+      qn = min(qn + (uint32_t)__popcll(pb), kChainQ - nf);
+      __syncthreads();
+      if (qn >= 64u) run_chains(64u);
     }
   }
 }
@@ -2442,6 +2394,11 @@ unsigned resident_grid(F kernel, uint32_t cap, int threads = kThreads) {
   return std::max(1u, std::min(n, std::max(cap, 1u)));
 }
 
+// RT_PARAM_WALK_* 1..7 as sixteenths of the lanes holding a ray.  The built-in 3 (a half) was the
+// fastest or within 2% of it on every workload measured (1 M segments: 7/8 of the lanes 856 us,
+// 3/4 775, 1/2 688, 1/4 688, 1/8 770).
+constexpr uint32_t kWalk16[7] = {14, 12, 8, 4, 2, 1, 0};
+
 // Launch sequence of one rayhierarchy group with the mode and node type fixed.
 template <int MODE, int NODE>
 hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hipEvent_t tm,
@@ -2493,7 +2450,7 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
     const dim3 grid(G.ray_grid > 0 ? std::max(1u, std::min((unsigned)G.ray_grid, G.max_chunks))
                                    : resident_grid(kernel, G.max_chunks, 64));
     hipLaunchKernelGGL(kernel, grid, dim3(64), 0, s, G.items, G.rq, G.ctr, G.max_chunks,
-                       (uint32_t)std::min(std::max(G.walk, 1), 7));
+                       kWalk16[std::min(std::max(G.walk, 1), 7) - 1]);
   };
   if (G.bvh)
     launch_rays(ray_path_kernel<MODE, NODE, true>);
