@@ -935,14 +935,34 @@ __global__ __launch_bounds__(kPackThreads) void rh_unit_pack_kernel(
 // counter each.  Work-group w starts in range w % kClaimQueues: the hardware deals
 // work-groups to the 8 XCDs in turn, so each XCD works through its own range of blocks in its
 // own L2, and one counter serves an eighth of the claims (claims of one counter serialise).
-// A work-group whose range is used up moves on to the next.  Returns nunits when none is
-// left.  One thread of the work-group calls it and keeps the state.  word 0 selects the unit
-// counters, word 1 those of the per-ray chunk slots.
+// A work-group whose range is used up moves on to the next.  Returns nunits when none is left.
+// One thread of the work-group calls it and keeps the state.  word 0 selects the unit counters,
+// word 1 those of the per-ray chunk slots.
+// A queue that gives every work-group at most one unit is dealt by position, in the same
+// eighths: no atomics, where every work-group otherwise ends with eight failing ones, on
+// counters that all of them visit (~11 ns each, one after another).  Measured per-ray, 4,096
+// chunks: torus 512 x 512 closest 142 -> 125 us, occlusion 148 -> 118; room task path depth 3,
+// secondary 1,750 -> 1,514, occlusion 1,280 -> 1,090.  Dealing only the first units of longer
+// queues by position was slower (1 M segments 680 -> 714 us): a work-group that does not start
+// at once holds its unit until another one has ended.  So was reading all eight counters after
+// a failed claim to go straight to a range with units left (778 us; torus occlusion units 205 ->
+// 267): near the end many work-groups see the same few units, and the reads contend with the
+// claims.
 struct UnitClaim {
   uint32_t q, tried;
 };
+__device__ __forceinline__ UnitClaim claim_start() {
+  return UnitClaim{blockIdx.x % (uint32_t)kClaimQueues, 0u};
+}
 __device__ __forceinline__ uint32_t claim_unit(uint32_t* ctr, uint32_t nunits, UnitClaim& c,
                                                int word = 0) {
+  const uint32_t per = (nunits + (uint32_t)kClaimQueues - 1u) / (uint32_t)kClaimQueues;
+  if (per * (uint32_t)kClaimQueues <= gridDim.x) {
+    const uint32_t k = blockIdx.x / (uint32_t)kClaimQueues;
+    const uint32_t u = c.tried == 0 && k < per ? c.q * per + k : nunits;
+    c.tried = kClaimQueues;
+    return min(u, nunits);
+  }
   while (c.tried < (uint32_t)kClaimQueues) {
     const uint32_t lo = (uint32_t)((uint64_t)nunits * c.q / kClaimQueues);
     const uint32_t hi = (uint32_t)((uint64_t)nunits * (c.q + 1) / kClaimQueues);
@@ -968,7 +988,7 @@ __global__ __launch_bounds__(256) void rh_unit_kernel(const RhItem* __restrict__
   const int tid = threadIdx.x;
   const uint32_t nunits = __builtin_amdgcn_readfirstlane(ctr[0]);
   if (nunits == 0) return;  // every block went to the per-ray path (or had no work)
-  UnitClaim claim{blockIdx.x % kClaimQueues, 0u};
+  UnitClaim claim = claim_start();
   if (tid == 0) {
     const uint32_t u = claim_unit(ctr, nunits, claim);
     sUnit = u < nunits ? units[u] : make_uint4(kNoUnit, 0u, 0u, 0u);
@@ -1334,7 +1354,7 @@ __global__ __launch_bounds__(256) void bvh_unit_kernel(const RhItem* __restrict_
   const int tid = threadIdx.x;
   const uint32_t nunits = __builtin_amdgcn_readfirstlane(ctr[0]);
   if (nunits == 0) return;
-  UnitClaim claim{blockIdx.x % kClaimQueues, 0u};
+  UnitClaim claim = claim_start();
   for (;;) {
     if (tid == 0) sUnit = claim_unit(ctr, nunits, claim);
     __syncthreads();
@@ -1623,16 +1643,18 @@ __device__ __forceinline__ void key_swap(uint32_t& a, uint32_t& b) {
 // depth 3, the bounces' closest hits 2,816 -> 1,767, occlusion 2,278 -> 1,251; 1 M segments
 // 1,089 -> 688; camera rays of twelve scenes 1,049 -> 609.
 constexpr uint32_t kChainQ = 127;  // below 64 before a round, one more per lane in it
-// Five wavefronts per SIMD (at most 96 VGPRs; the LDS of 20 work-groups per CU): the walk is
-// latency-bound and gains more from resident wavefronts than it loses to a few spilled
-// registers of the chain evaluation.
+// Registers for five wavefronts per SIMD (96 VGPRs), ray-bvh for four (its chain spilled 7-15:
+// room task path depth 3, secondary 1,344 -> 1,103 us); see search_stack for the LDS.  Keeping
+// only 24 or 16 stack entries in LDS and the rest in scratch memory, for more work-groups per
+// CU, was 3-6% slower, and six wavefronts per SIMD (80 VGPRs) a quarter to a half.
 template <int MODE, int NODE, bool BVH>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void ray_path_kernel(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5, 8))) void ray_path_kernel(
     const RhItem* __restrict__ items, const uint2* __restrict__ rq, uint32_t* __restrict__ ctr,
     uint32_t nchunks, uint32_t walk16) {
-  __shared__ uint32_t sStk[kSearchStack][64];
+  __shared__ uint32_t sStk[search_stack(BVH)][64];
   // candidates [0, qn) and, from the far end, rays to trace again [kChainQ - nf, kChainQ)
-  __shared__ uint32_t sQIdx[kChainQ], sQRef[kChainQ], sQJob[kChainQ];
+  __shared__ uint32_t sQIdx[kChainQ], sQRef[kChainQ];
+  __shared__ uint16_t sQJob[kChainQ];
   constexpr uint32_t kDone = 0xffffffffu;  // not a reference (positions are below 2^31)
   const float kInf = __int_as_float(0x7f800000);
   auto widened = [](float t) { return t + fabsf(t) * kSlack; };
@@ -1658,7 +1680,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
   auto pop = [&]() { return sp > 0 ? sStk[--sp][lane] : kDone; };
   // the cluster pass sets ctr[4] when it routed any block here
   if (__builtin_amdgcn_readfirstlane(ctr[4]) == 0u) return;
-  UnitClaim claim{blockIdx.x % kClaimQueues, 0u};
+  UnitClaim claim = claim_start();
   auto chain = [&](const RhItem& it, uint32_t ri, uint32_t ref) {
     const int x = (int)(ri % (uint32_t)it.g.W), y = (int)(ri / (uint32_t)it.g.W);
     if constexpr (BVH) return ray_chain_bvh<NODE>(it, x, y, ref);
@@ -1697,7 +1719,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     if (failed) {
       const uint32_t p = kChainQ - 1u - nf - (uint32_t)__popcll(fb & lanes_below);
       sQIdx[p] = ri;
-      sQJob[p] = job;
+      sQJob[p] = (uint16_t)job;
     }
     nf += (uint32_t)__popcll(fb);
     __syncthreads();
@@ -1923,7 +1945,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
         if (room) {
           sQIdx[e] = idx;
           sQRef[e] = cand;
-          sQJob[e] = jk;
+          sQJob[e] = (uint16_t)jk;
           if constexpr (MODE != 2) glb(it.keys)[idx] = best;
           act = false;
         } else {

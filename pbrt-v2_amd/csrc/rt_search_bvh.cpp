@@ -26,8 +26,8 @@
 // many nodes as in the binary tree (counted on the CPU: cluster scene of 200,000 triangles,
 // camera rays 112.6 -> 57.1, random segments 58.8 -> 29.0; room, diffuse bounces 121.2 -> 58.4),
 // and a walk is a chain of dependent loads.  An expansion is only made while the walk's stack
-// stays within kSearchStack: with k siblings left behind, every interior child must have at
-// most (budget - k) binary levels below it, which any binary tree within kSearchStack levels
+// stays within its entries: with k siblings left behind, every interior child must have at most
+// (budget - k) binary levels below it, which any binary tree of no more levels than entries
 // meets by keeping two children per node.
 //
 // Node planes are FP16 in units of the frame above the node's cell of a 256^3 grid over the
@@ -351,7 +351,7 @@ class Collapser {
 
 }  // namespace
 
-void build_search_bvh(const float* v9, uint32_t ntri, std::vector<uint4>& nodes,
+void build_search_bvh(const float* v9, uint32_t ntri, int stack, std::vector<uint4>& nodes,
                       std::vector<uint32_t>& order, SearchFrame& frame) {
   nodes.clear();
   order.clear();
@@ -408,7 +408,7 @@ void build_search_bvh(const float* v9, uint32_t ntri, std::vector<uint4>& nodes,
   b.build(0, ntri, 1, box);
   Collapser::Child c[4] = {Collapser::Child{bin[0].box[0], bin[0].ref[0]},
                            Collapser::Child{bin[0].box[1], bin[0].ref[1]}, {}, {}};
-  w.node(0, c, 2, kSearchStack);
+  w.node(0, c, 2, stack);
 }
 
 }  // namespace rti
