@@ -210,7 +210,7 @@ int rt_make_bounce_rays(rt_scene *scene, const rt_rays *in, const int32_t *id, c
  *   is evaluated for the triangles that pass its strict leaf test -- in place of enumerating
  *   the block's (leaf, triangle) candidate pairs.  1 sends every block with work that way;
  *   2^29 keeps only the direction test; a value above 2^29 (at most 2^30) sends no block.
- *   Built-in (0): 2^29 for closest hits, 256 (rayhierarchy) or 64 (ray-bvh) for occlusion.
+ *   Built-in (0): every block, without looking at its clusters.
  *   RT_PARAM_RAY_GRID_CLOSEST / RT_PARAM_RAY_GRID_OCCLUDED: work-groups (one wavefront each)
  *   of the per-ray kernel (batches only); 0 = one per resident slot.
  *   RT_PARAM_WALK_CLOSEST / RT_PARAM_WALK_OCCLUDED: v in 1..7: a round of the per-ray kernel

@@ -372,14 +372,6 @@ hipError_t timed_launch(Timer& tm, int mode, hipStream_t st, F fn) {
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 constexpr int kDefaultPer[2] = {8, 4};  // passing clusters per unit: closest, occluded
-// Blocks whose root passes at least this many clusters (64 triangles or 64 frontier roots
-// each) in a scene of four times as many, or whose leaves' ray directions spread widely, are
-// traced ray by ray.  2^29 keeps only the direction test.  Built-in choice per accelerator and
-// mode (closest, occluded), measured on the torus, room, uneven-batch and serving workloads:
-// coherent camera blocks are fastest on the block path; shadow blocks that pass many clusters
-// of a large scene are faster ray by ray, more so behind ray-bvh's lockstep block path.
-constexpr int kDefaultRay[2][2] = {{1 << 29, 256}, {1 << 29, 64}};
-int default_ray(bool bvh, int mi) { return kDefaultRay[bvh ? 1 : 0][mi]; }
 constexpr int kDefaultRootClustersPerUnit = 8;  // passing root clusters per ray-bvh unit
 
 // The job-table entry of one job: geometry of its ray image and the scene's resident arrays
@@ -470,7 +462,8 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
     GroupLayout& L = gl[gi];
     // work units: passing clusters of triangles (rayhierarchy) or of frontier roots (ray-bvh)
     L.per = prm.per[mi] > 0 ? prm.per[mi] : (bvh ? kDefaultRootClustersPerUnit : kDefaultPer[mi]);
-    L.ray = (uint32_t)(prm.ray[mi] > 0 ? prm.ray[mi] : default_ray(bvh, mi));
+    L.ray = (uint32_t)prm.ray[mi];
+    const bool direct = L.ray == 0;  // no cluster lists, queues or keys
     L.rgrid = prm.rgrid[mi];
     L.walk = prm.walk[mi] > 0 ? prm.walk[mi] : kDefaultWalk;
     L.max_units = 0;
@@ -503,11 +496,12 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
       off_nodes[j] = total;
       total += align256(sizeof(float4) * 4 * (size_t)it.g.nnodes);
       off_clist[j] = total;
-      total += align256(sizeof(uint32_t) * (size_t)it.g.ntop * std::max<uint32_t>(it.nclusters, 1));
+      if (!direct)
+        total += align256(sizeof(uint32_t) * (size_t)it.g.ntop * std::max<uint32_t>(it.nclusters, 1));
       off_keys[j] = total;
-      if (mode != 2) total += align256(sizeof(uint64_t) * n);
+      if (mode != 2 && !direct) total += align256(sizeof(uint64_t) * n);
       off_rep[j] = total;
-      if (it.repair_run > 0) total += align256(sizeof(uint32_t) * n);
+      if (it.repair_run > 0 && !direct) total += align256(sizeof(uint32_t) * n);
     }
     if (blocks >= (1ull << 31) || rays >= (1ull << 31)) return RT_ERR_UNSUPPORTED;
     L.nblocks = (uint32_t)blocks;
@@ -516,14 +510,16 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
     L.grid = prm.grid[mi] > 0
                  ? (int)std::max<size_t>(1, std::min<size_t>(L.max_units, (size_t)prm.grid[mi]))
                  : 0;
-    L.units = total;
-    total += align256(sizeof(uint4) * std::max<size_t>(L.max_units, 1));
-    L.ustage = total;
-    total += align256(sizeof(uint4) * std::max<size_t>(L.max_units, 1));
-    L.bunits = total;
-    total += align256(sizeof(uint4) * std::max<size_t>(L.nblocks, 1));
-    L.rq = total;
-    total += align256(sizeof(uint2) * std::max<size_t>(L.max_chunks, 1));
+    L.units = L.ustage = L.bunits = L.rq = total;
+    if (!direct) {
+      total += align256(sizeof(uint4) * std::max<size_t>(L.max_units, 1));
+      L.ustage = total;
+      total += align256(sizeof(uint4) * std::max<size_t>(L.max_units, 1));
+      L.bunits = total;
+      total += align256(sizeof(uint4) * std::max<size_t>(L.nblocks, 1));
+      L.rq = total;
+      total += align256(sizeof(uint2) * std::max<size_t>(L.max_chunks, 1));
+    }
     L.ctr = total;
     total += align256(kCounterBytes);
     L.replist = total;
@@ -550,9 +546,10 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
   for (size_t j = 0; j < jobs.size(); ++j) {
     RhItem& it = items[j];
     it.nodes = (float4*)(A + off_nodes[j]);
-    it.clist = (uint32_t*)(A + off_clist[j]);
-    it.keys = jobs[j].mode != 2 ? (uint64_t*)(A + off_keys[j]) : nullptr;
-    it.repkeys = it.repair_run > 0 ? (uint32_t*)(A + off_rep[j]) : nullptr;
+    const bool direct = prm.ray[jobs[j].mode == 2 ? 1 : 0] == 0;
+    it.clist = direct ? nullptr : (uint32_t*)(A + off_clist[j]);
+    it.keys = jobs[j].mode != 2 && !direct ? (uint64_t*)(A + off_keys[j]) : nullptr;
+    it.repkeys = it.repair_run > 0 && !direct ? (uint32_t*)(A + off_rep[j]) : nullptr;
   }
   // tables in group order
   std::vector<RhItem> table;
@@ -1034,14 +1031,17 @@ int rt_trace_closest_noalloc(rt_scene* s, const rt_rays* rays, int32_t mode, con
   };
   RhItem* table = (RhItem*)take(sizeof(RhItem));
   it.nodes = (float4*)take(sizeof(float4) * 4 * (size_t)it.g.nnodes);
-  it.keys = (uint64_t*)take(sizeof(uint64_t) * n);
-  it.repkeys = repair ? (uint32_t*)take(sizeof(uint32_t) * n) : nullptr;
+  // reduction keys and queues, which this form once used and no longer does: the sizes that it
+  // takes and refuses stay the ones its declaration promises
+  take(sizeof(uint64_t) * n);
+  if (repair) take(sizeof(uint32_t) * n);
+  take(sizeof(uint4));
+  take(sizeof(uint4) * (size_t)it.g.ntop);
+  take(sizeof(uint2) * (size_t)it.g.ntop * nch);
+  it.keys = nullptr;
+  it.repkeys = nullptr;
   it.clist = nullptr;
   RhGroup G{};
-  G.units = (uint4*)take(sizeof(uint4));
-  G.ustage = G.units;  // every block takes the per-ray path: no unit is staged
-  G.bunits = (uint4*)take(sizeof(uint4) * (size_t)it.g.ntop);
-  G.rq = (uint2*)take(sizeof(uint2) * (size_t)it.g.ntop * nch);
   G.ctr = (uint32_t*)take(kCounterBytes);
   G.replist = repair ? (uint32_t*)take(sizeof(uint32_t) * n) : nullptr;
   if (off > kNoAllocScratch || n >= (1ull << 31)) return RT_ERR_TOO_LARGE;
@@ -1392,9 +1392,9 @@ int rt_batch_autotune(rt_batch* b, void* stream, int32_t reps) {
   const bool was_graph = b->use_graph;
   b->use_graph = false;
   b->timer.on = true;
-  // stage 1: which blocks take the per-ray path (1: all, 2^30: none) and the per-ray grid
+  // stage 1: which blocks take the per-ray path (0: all, 2^30: none) and the per-ray grid
   // (one wavefront per work-group: 8 or 16 per CU, or every resident slot)
-  static const int kRay[] = {1, 64, 256, 1 << 29, 1 << 30};
+  static const int kRay[] = {0, 64, 256, 1 << 29, 1 << 30};
   static const int kRGrid[] = {0, 2048, 4096};
   auto routing = [&]() {
     return autotune_stage(

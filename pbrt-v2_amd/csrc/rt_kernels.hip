@@ -302,6 +302,18 @@ __device__ __forceinline__ int find_block_item(const RhItem* __restrict__ items,
   }
   return k - 1;
 }
+// Job of a global chunk index, likewise.
+__device__ __forceinline__ int find_chunk_item(const RhItem* __restrict__ items, int n,
+                                               uint32_t gc) {
+  int k = 0;
+  for (int c = 0; c < n; c += 64) {
+    const int j = c + (int)__lane_id();
+    const int m = __popcll(__ballot(j < n && items[j].chunk_base <= gc));
+    k += m;
+    if (m < 64) break;
+  }
+  return k - 1;
+}
 // Job of a global ray index (per lane).
 __device__ __forceinline__ int find_ray_item(const RhItem* __restrict__ items, int n,
                                              uint32_t gr) {
@@ -357,11 +369,23 @@ __device__ void build_block_deep(const RHGeom& g, const RaysDev& r, float4* __re
   }
 }
 
+// Clears a group's counters (thread i of a grid of at least 8 threads).
+__device__ __forceinline__ void clear_counters(uint32_t* __restrict__ ctr, uint32_t i) {
+  if (i < 8) ctr[i] = 0u;
+  if (i < kClaimQueues) {
+    ctr[kClaimBase + kClaimStride * i] = 0u;      // units
+    ctr[kClaimBase + kClaimStride * i + 1] = 0u;  // per-ray chunk slots
+  }
+}
+
+// ctr: the counters to clear for the kernels that follow (null: the init kernel does it).
 template <bool USE_VALID, bool UV>
 __global__ __launch_bounds__(256) void rh_group_build_kernel(const RhItem* __restrict__ items,
-                                                             int nitems) {
+                                                             int nitems,
+                                                             uint32_t* __restrict__ ctr) {
   __shared__ float sBox[kMaxSub][12];
   __shared__ int sVal[kMaxSub];
+  if (ctr != nullptr && blockIdx.x == 0) clear_counters(ctr, threadIdx.x);
   const int k = find_block_item(items, nitems, blockIdx.x);
   const RhItem& it = items[k];
   if (it.g.L > kUnitLevels)
@@ -376,11 +400,7 @@ template <int MODE>
 __global__ __launch_bounds__(256) void rh_init_kernel(const RhItem* __restrict__ items, int nitems,
                                                       uint32_t nrays, uint32_t* __restrict__ ctr) {
   const uint32_t gi = blockIdx.x * kThreads + threadIdx.x;
-  if (gi < 8) ctr[gi] = 0u;
-  if (gi < kClaimQueues) {
-    ctr[kClaimBase + kClaimStride * gi] = 0u;      // units
-    ctr[kClaimBase + kClaimStride * gi + 1] = 0u;  // per-ray chunk slots
-  }
+  clear_counters(ctr, gi);
   if (gi >= nrays) return;
   const RhItem& it = items[find_ray_item(items, nitems, gi)];
   const uint32_t i = gi - it.ray_base;
@@ -1518,6 +1538,71 @@ __global__ __launch_bounds__(256) void bvh_unit_kernel(const RhItem* __restrict_
 }
 
 // ---------------------------------------------------------------------------------------
+// Hit record: id, t, (u, v) and optionally dpdu/dpdv of computeDpTuTv.cl:8-91.
+// Hit record of ray i (computeDpTuTv.cl:8-91).  naive_rule: the naive kernels' inline copy of
+// that code takes the coordinate-system fallback for |det| < EPS (naive.cl:60-61,153-154)
+// where computeDpTuTv.cl:57 takes it for det == 0 only.  write_t: false leaves t as it is.
+__device__ void write_hit(const RaysDev& r, const float* __restrict__ v9,
+                          const float* __restrict__ uv6, size_t i, int32_t id, float t,
+                          const HitOut& out, bool naive_rule = false,
+                          bool write_t = true) {
+  if (id < 0) {
+    out.id[i] = -1;
+    out.t[i] = __int_as_float(0x7f800000);
+    out.u[i] = 0.f;
+    out.v[i] = 0.f;
+    if (out.dpdu)
+      for (int c = 0; c < 3; ++c) out.dpdu[3 * i + c] = 0.f;
+    if (out.dpdv)
+      for (int c = 0; c < 3; ++c) out.dpdv[3 * i + c] = 0.f;
+    return;
+  }
+  const Tri T = load_tri(v9, (uint32_t)id);
+  const V3 o = {r.ox[i], r.oy[i], r.oz[i]};
+  const V3 d = {r.dx[i], r.dy[i], r.dz[i]};
+  float b1, b2;
+  bary(o, d, T, b1, b2);
+  float uv[6] = {0.f, 0.f, 1.f, 0.f, 1.f, 1.f};
+  if (uv6)
+    for (int k = 0; k < 6; ++k) uv[k] = uv6[6 * (size_t)id + k];
+  const float b0 = 1 - b1 - b2;
+  out.id[i] = id;
+  if (write_t) out.t[i] = t;
+  out.u[i] = (b0 * uv[0] + b1 * uv[2]) + b2 * uv[4];
+  out.v[i] = (b0 * uv[1] + b1 * uv[3]) + b2 * uv[5];
+  if (out.dpdu || out.dpdv) {
+    const float du1 = uv[0] - uv[4], du2 = uv[2] - uv[4];
+    const float dv1 = uv[1] - uv[5], dv2 = uv[3] - uv[5];
+    const V3 dp1 = sub(T.v1, T.v3), dp2 = sub(T.v2, T.v3);
+    const float det = du1 * dv2 - dv1 * du2;
+    V3 pu, pv;
+    if (naive_rule ? (det > -kEps && det < kEps) : det == 0.f) {
+      const V3 tn = normalize(cross(T.e2, T.e1));
+      if (fabsf(tn.x) > fabsf(tn.y)) {
+        const float il = 1.0f / sqrtf(tn.x * tn.x + tn.z * tn.z);
+        pu = {-tn.z * il, 0.f, tn.x * il};
+      } else {
+        const float il = 1.0f / sqrtf(tn.y * tn.y + tn.z * tn.z);
+        pu = {0.f, tn.z * il, -tn.y * il};
+      }
+      pv = cross(tn, pu);
+    } else {
+      const float id2 = 1.f / det;
+      pu = {(dv2 * dp1.x - dv1 * dp2.x) * id2, (dv2 * dp1.y - dv1 * dp2.y) * id2,
+            (dv2 * dp1.z - dv1 * dp2.z) * id2};
+      pv = {(-du2 * dp1.x + du1 * dp2.x) * id2, (-du2 * dp1.y + du1 * dp2.y) * id2,
+            (-du2 * dp1.z + du1 * dp2.z) * id2};
+    }
+    if (out.dpdu) {
+      out.dpdu[3 * i] = pu.x; out.dpdu[3 * i + 1] = pu.y; out.dpdu[3 * i + 2] = pu.z;
+    }
+    if (out.dpdv) {
+      out.dpdv[3 * i] = pv.x; out.dpdv[3 * i + 1] = pv.y; out.dpdv[3 * i + 2] = pv.z;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------
 // Per-ray path (blocks the cluster pass queued as incoherent).  A ray's result is the argmin
 // over the triangles that pass its strict leaf test AND the exact cull chain of its leaf (for
 // ray-bvh: that are tested at a (BVH leaf, hierarchy leaf) pair whose lockstep chain passes).
@@ -1626,7 +1711,7 @@ __device__ __forceinline__ void key_swap(uint32_t& a, uint32_t& b) {
 // A ray is first traced as if every cull chain passed, which is what they nearly always do:
 // occlusion ends at its first strict hit inside the interval, a closest hit is the nearest
 // strict hit.  That one candidate goes to a wavefront queue in LDS as {ray, triangle or BVH
-// leaf, job} (a closest hit's key goes to the ray's key in memory) and its lane takes the next
+// leaf, job} (a closest hit's t, or its key, goes to memory) and its lane takes the next
 // ray; whenever the queue holds 64 candidates, their chains are evaluated together, one per
 // lane.  A passing chain confirms the candidate: the nearest strict hit is the answer when its
 // chain passes, and any strict hit with a passing chain occludes.  A ray whose candidate
@@ -1642,15 +1727,23 @@ __device__ __forceinline__ void key_swap(uint32_t& a, uint32_t& b) {
 // (1/8 before): torus 512 x 512 closest 247 -> 142 us, occlusion 318 -> 146; room task to path
 // depth 3, the bounces' closest hits 2,816 -> 1,767, occlusion 2,278 -> 1,251; 1 M segments
 // 1,089 -> 688; camera rays of twelve scenes 1,049 -> 609.
+//
+// Without a queue of chunks (rq null) every block of the group is traced here: chunk e is found
+// from the jobs' chunk prefixes and the results are written here, misses by their lane and hits
+// by the lane that confirms them, so no reduction keys, no init and no finalize launch are
+// needed.  Otherwise the rays of the blocks that the cluster pass sent here leave their keys,
+// repair keys and flags as the block path does.
+// ONE: the group has one job; its table entry and the pointers in it are then uniform.
 constexpr uint32_t kChainQ = 127;  // below 64 before a round, one more per lane in it
 // Registers for five wavefronts per SIMD (96 VGPRs), ray-bvh for four (its chain spilled 7-15:
 // room task path depth 3, secondary 1,344 -> 1,103 us); see search_stack for the LDS.  Keeping
 // only 24 or 16 stack entries in LDS and the rest in scratch memory, for more work-groups per
 // CU, was 3-6% slower, and six wavefronts per SIMD (80 VGPRs) a quarter to a half.
-template <int MODE, int NODE, bool BVH>
+template <int MODE, int NODE, bool BVH, bool ONE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5, 8))) void ray_path_kernel(
-    const RhItem* __restrict__ items, const uint2* __restrict__ rq, uint32_t* __restrict__ ctr,
-    uint32_t nchunks, uint32_t walk16) {
+    const RhItem* __restrict__ items, int nitems, const uint2* __restrict__ rq,
+    uint32_t* __restrict__ ctr, uint32_t* __restrict__ replist, uint32_t nchunks,
+    uint32_t walk16) {
   __shared__ uint32_t sStk[search_stack(BVH)][64];
   // candidates [0, qn) and, from the far end, rays to trace again [kChainQ - nf, kChainQ)
   __shared__ uint32_t sQIdx[kChainQ], sQRef[kChainQ];
@@ -1673,18 +1766,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
   float tmin = 0.f, tmax = 0.f, tlo = 0.f, thi = 0.f;
   uint64_t best = kMissKey;   // closest: the nearest hit (verified when careful)
   uint32_t rep = kNoKey32;    // primary: the nearest repair-region hit (likewise)
-  uint32_t cand = 0;          // chain operand of the candidate: triangle id or BVH leaf
+  uint32_t cand = 0;          // the candidate: triangle id, ray-bvh occlusion its BVH leaf
   bool track_rep = false;
   int sp = 0;
   uint32_t cur = kDone, pl = kDone;
   auto pop = [&]() { return sp > 0 ? sStk[--sp][lane] : kDone; };
+  const bool direct = rq == nullptr;
   // the cluster pass sets ctr[4] when it routed any block here
-  if (__builtin_amdgcn_readfirstlane(ctr[4]) == 0u) return;
+  if (!direct && __builtin_amdgcn_readfirstlane(ctr[4]) == 0u) return;
   UnitClaim claim = claim_start();
+  auto item = [&](uint32_t j) -> const RhItem& { return items[ONE ? 0u : j]; };
+  // the exact chain of ray ri's candidate: a triangle, or for ray-bvh occlusion its BVH leaf
   auto chain = [&](const RhItem& it, uint32_t ri, uint32_t ref) {
     const int x = (int)(ri % (uint32_t)it.g.W), y = (int)(ri / (uint32_t)it.g.W);
-    if constexpr (BVH) return ray_chain_bvh<NODE>(it, x, y, ref);
-    else return ray_chain_rh<MODE, NODE>(it, x, y, ref);
+    if constexpr (BVH)
+      return ray_chain_bvh<NODE>(it, x, y, MODE == 2 ? ref : glb(it.tleaf)[ref] & 0x7fffffffu);
+    else
+      return ray_chain_rh<MODE, NODE>(it, x, y, ref);
+  };
+  // direct: the record of a ray that hits nothing / has hit triangle id (its t is written apart)
+  auto write_miss = [&](const RhItem& it, uint32_t ri) {
+    if constexpr (MODE == 2) glb(it.occ)[ri] = 0;
+    else write_hit(it.r, it.v9, it.uv6, ri, -1, 0.f, it.out);
   };
   auto restart = [&]() {
     careful = true;
@@ -1704,10 +1807,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
     if (have) {
       ri = sQIdx[e];
       job = sQJob[e];
-      const RhItem& it = items[job];
-      const bool ok = chain(it, ri, sQRef[e]);
+      const RhItem& it = item(job);
+      const uint32_t ref = sQRef[e];
+      const bool ok = chain(it, ri, ref);
       if constexpr (MODE == 2) {
         if (ok) glb(it.occ)[ri] = 1;
+      } else if (direct) {
+        if (ok) write_hit(it.r, it.v9, it.uv6, ri, (int32_t)ref, 0.f, it.out, false, false);
       } else {
         // stores of one wavefront to one address keep their order
         if (!ok) glb(it.keys)[ri] = kMissKey;
@@ -1751,34 +1857,41 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
             more = false;
             break;
           }
-          const uint2 w = rq[e];
-          if (__builtin_amdgcn_readfirstlane(w.x) == 0xffffffffu) continue;  // a block-path block
-          cjob = __builtin_amdgcn_readfirstlane(w.x);
-          const uint32_t c = __builtin_amdgcn_readfirstlane(w.y);
-          const uint32_t nch = ((uint32_t)items[cjob].g.rb + 63u) / 64u;
+          uint32_t c;
+          if (direct) {
+            cjob = ONE ? 0u : (uint32_t)find_chunk_item(items, nitems, e);
+            c = e - item(cjob).chunk_base;
+          } else {
+            const uint2 w = rq[e];
+            cjob = __builtin_amdgcn_readfirstlane(w.x);
+            if (cjob == 0xffffffffu) continue;  // a block-path block
+            c = __builtin_amdgcn_readfirstlane(w.y);
+          }
+          const uint32_t nch = ((uint32_t)item(cjob).g.rb + 63u) / 64u;
           cblk = c / nch;
           cpart = c - cblk * nch;
           cslot = 0;
         }
         const uint32_t avail = 64u - cslot;
         if (!act && rank < avail) {
-          const RhItem& it = items[cjob];
+          const RhItem& it = item(cjob);
           const RHGeom& g = it.g;
           const int top = g.L - 1;
           const int K = (int)cblk % g.gw[top], J = (int)cblk / g.gw[top];
           int x = 0, y = 0, leaf = 0;
-          got = slot_xy(g, K, J, (int)(cpart * 64u + cslot + rank), x, y, leaf) && it.ntri > 0;
-          if (got) {
+          if (slot_xy(g, K, J, (int)(cpart * 64u + cslot + rank), x, y, leaf)) {
             idx = (uint32_t)y * (uint32_t)g.W + (uint32_t)x;
-            if (MODE != 0 && it.r.valid != nullptr && glb(it.r.valid)[idx] == 0) got = false;
             jk = cjob;
             careful = false;
+            got = it.ntri > 0 &&
+                  (MODE == 0 || it.r.valid == nullptr || glb(it.r.valid)[idx] != 0);
+            if (direct && !got) write_miss(it, idx);
           }
         }
         cslot += min(avail, (uint32_t)__popcll(need));
       }
       if (got) {
-        const RhItem& it = items[jk];
+        const RhItem& it = item(jk);
         const RaysDev& r = it.r;
         o = {glb(r.ox)[idx], glb(r.oy)[idx], glb(r.oz)[idx]};
         d = {glb(r.dx)[idx], glb(r.dy)[idx], glb(r.dz)[idx]};
@@ -1789,7 +1902,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
         slab_axis(o.y, d.y, f.base[1], f.unit, sr.ih.y, sr.cn.y, sr.cf.y);
         slab_axis(o.z, d.z, f.base[2], f.unit, sr.ih.z, sr.cn.z, sr.cf.z);
         tlo = tmin - fabsf(tmin) * kSlack;
-        track_rep = MODE == 0 && !BVH && it.repkeys != nullptr;
+        track_rep = MODE == 0 && !BVH && it.repair_run > 0;
         const bool again = careful;
         restart();
         careful = again;
@@ -1801,7 +1914,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
       run_chains(min(qn, 64u));
       continue;
     }
-    const RhItem& it = items[jk];
+    const RhItem& it = item(jk);
     const auto snode = glb(it.snode);
     const auto tmts = glb(it.tmts);
     // node phase: a lane visits one 4-wide node a step, four 16-byte loads of one line, its
@@ -1887,7 +2000,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
       // in no leaf; or not its leaf's first primitive (6DB / IA secondary rays)
       const bool ok = !BVH || (bl != 0xffffffffu &&
                                !(MODE == 1 && NODE != 2 && (bl & 0x80000000u)));
-      const uint32_t ref = BVH ? bl & 0x7fffffffu : id;
+      const uint32_t ref = BVH && MODE == 2 ? bl & 0x7fffffffu : id;
       float t, b1, b2;
       if (ok && mt_strict(o, d, T, t, b1, b2)) {
         if constexpr (MODE == 2) {
@@ -1924,17 +2037,29 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
     // rays that are done: a verified result is written; the others queue their candidate, if
     // they have one
     if (act && !push && cur == kDone && pl == kDone) {
+      const float tstar = best == kMissKey ? kInf : fkey_inv((uint32_t)(best >> 32));
       if constexpr (MODE == 2) {
+        if (direct) write_miss(it, idx);
         act = false;
       } else if (careful) {
-        if (best != kMissKey) glb(it.keys)[idx] = best;
-        if (track_rep && rep != kNoKey32) glb(it.repkeys)[idx] = rep;
+        if (direct) {
+          if (best == kMissKey) write_miss(it, idx);
+          else write_hit(it.r, it.v9, it.uv6, idx, (int32_t)(uint32_t)best, tstar, it.out);
+          // as rh_finalize_kernel lists it
+          if (MODE == 0 && rep != kNoKey32 && !(fkey_inv(rep) > tstar - kEps))
+            replist[atomicAdd(&ctr[2], 1u)] = it.ray_base + idx;
+        } else {
+          if (best != kMissKey) glb(it.keys)[idx] = best;
+          if (track_rep && rep != kNoKey32) glb(it.repkeys)[idx] = rep;
+        }
+        act = false;
+      } else if (rep != kNoKey32 && !(fkey_inv(rep) > tstar - kEps)) {
+        restart();
+      } else if (best == kMissKey) {
+        if (direct) write_miss(it, idx);
         act = false;
       } else {
-        const float tstar = best == kMissKey ? kInf : fkey_inv((uint32_t)(best >> 32));
-        if (rep != kNoKey32 && !(fkey_inv(rep) > tstar - kEps)) restart();
-        else if (best == kMissKey) act = false;
-        else push = true;
+        push = true;
       }
     }
     const uint64_t pb = __ballot(push);
@@ -1946,7 +2071,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
           sQIdx[e] = idx;
           sQRef[e] = cand;
           sQJob[e] = (uint16_t)jk;
-          if constexpr (MODE != 2) glb(it.keys)[idx] = best;
+          if constexpr (MODE != 2) {
+            if (direct) glb(it.out.t)[idx] = fkey_inv((uint32_t)(best >> 32));
+            else glb(it.keys)[idx] = best;
+          }
           act = false;
         } else {
           restart();
@@ -2040,69 +2168,6 @@ __global__ __launch_bounds__(256) void naive_kernel(RaysDev r, const float* __re
 }
 
 // ---------------------------------------------------------------------------------------
-// Hit record: id, t, (u, v) and optionally dpdu/dpdv of computeDpTuTv.cl:8-91.
-// Hit record of ray i (computeDpTuTv.cl:8-91).  naive_rule: the naive kernels' inline copy of
-// that code takes the coordinate-system fallback for |det| < EPS (naive.cl:60-61,153-154)
-// where computeDpTuTv.cl:57 takes it for det == 0 only.
-__device__ void write_hit(const RaysDev& r, const float* __restrict__ v9,
-                          const float* __restrict__ uv6, size_t i, int32_t id, float t,
-                          HitOut out, bool naive_rule = false) {
-  if (id < 0) {
-    out.id[i] = -1;
-    out.t[i] = __int_as_float(0x7f800000);
-    out.u[i] = 0.f;
-    out.v[i] = 0.f;
-    if (out.dpdu)
-      for (int c = 0; c < 3; ++c) out.dpdu[3 * i + c] = 0.f;
-    if (out.dpdv)
-      for (int c = 0; c < 3; ++c) out.dpdv[3 * i + c] = 0.f;
-    return;
-  }
-  const Tri T = load_tri(v9, (uint32_t)id);
-  const V3 o = {r.ox[i], r.oy[i], r.oz[i]};
-  const V3 d = {r.dx[i], r.dy[i], r.dz[i]};
-  float b1, b2;
-  bary(o, d, T, b1, b2);
-  float uv[6] = {0.f, 0.f, 1.f, 0.f, 1.f, 1.f};
-  if (uv6)
-    for (int k = 0; k < 6; ++k) uv[k] = uv6[6 * (size_t)id + k];
-  const float b0 = 1 - b1 - b2;
-  out.id[i] = id;
-  out.t[i] = t;
-  out.u[i] = (b0 * uv[0] + b1 * uv[2]) + b2 * uv[4];
-  out.v[i] = (b0 * uv[1] + b1 * uv[3]) + b2 * uv[5];
-  if (out.dpdu || out.dpdv) {
-    const float du1 = uv[0] - uv[4], du2 = uv[2] - uv[4];
-    const float dv1 = uv[1] - uv[5], dv2 = uv[3] - uv[5];
-    const V3 dp1 = sub(T.v1, T.v3), dp2 = sub(T.v2, T.v3);
-    const float det = du1 * dv2 - dv1 * du2;
-    V3 pu, pv;
-    if (naive_rule ? (det > -kEps && det < kEps) : det == 0.f) {
-      const V3 tn = normalize(cross(T.e2, T.e1));
-      if (fabsf(tn.x) > fabsf(tn.y)) {
-        const float il = 1.0f / sqrtf(tn.x * tn.x + tn.z * tn.z);
-        pu = {-tn.z * il, 0.f, tn.x * il};
-      } else {
-        const float il = 1.0f / sqrtf(tn.y * tn.y + tn.z * tn.z);
-        pu = {0.f, tn.z * il, -tn.y * il};
-      }
-      pv = cross(tn, pu);
-    } else {
-      const float id2 = 1.f / det;
-      pu = {(dv2 * dp1.x - dv1 * dp2.x) * id2, (dv2 * dp1.y - dv1 * dp2.y) * id2,
-            (dv2 * dp1.z - dv1 * dp2.z) * id2};
-      pv = {(-du2 * dp1.x + du1 * dp2.x) * id2, (-du2 * dp1.y + du1 * dp2.y) * id2,
-            (-du2 * dp1.z + du1 * dp2.z) * id2};
-    }
-    if (out.dpdu) {
-      out.dpdu[3 * i] = pu.x; out.dpdu[3 * i + 1] = pu.y; out.dpdu[3 * i + 2] = pu.z;
-    }
-    if (out.dpdv) {
-      out.dpdv[3 * i] = pv.x; out.dpdv[3 * i + 1] = pv.y; out.dpdv[3 * i + 2] = pv.z;
-    }
-  }
-}
-
 // Hit record of one ray from its reduction key; returns t (INFINITY on a miss).
 __device__ __forceinline__ float finalize_ray(const RaysDev& r, const float* __restrict__ v9,
                                               const float* __restrict__ uv6, uint64_t key,
@@ -2425,11 +2490,14 @@ constexpr uint32_t kWalk16[7] = {14, 12, 8, 4, 2, 1, 0};
 template <int MODE, int NODE>
 hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hipEvent_t tm,
                              hipEvent_t t1) {
-  hipLaunchKernelGGL((rh_init_kernel<MODE>), grid1(std::max<uint32_t>(G.nrays, 4)),
-                     dim3(kThreads), 0, s, G.items, G.nitems, G.nrays, G.ctr);
+  const bool direct = G.ray_clusters == 0;  // every block ray by ray, results written there
+  if (!direct)
+    hipLaunchKernelGGL((rh_init_kernel<MODE>), grid1(std::max<uint32_t>(G.nrays, kClaimQueues)),
+                       dim3(kThreads), 0, s, G.items, G.nitems, G.nrays, G.ctr);
   hipLaunchKernelGGL((rh_group_build_kernel<MODE != 0, NODE == 2>), dim3(G.nblocks),
-                     dim3(kThreads), 0, s, G.items, G.nitems);
-  if (G.bvh)
+                     dim3(kThreads), 0, s, G.items, G.nitems, direct ? G.ctr : nullptr);
+  if (direct) {
+  } else if (G.bvh)
     hipLaunchKernelGGL((rh_cluster_kernel<MODE, NODE, true>), dim3(G.nblocks), dim3(kThreads), 0,
                        s, G.items, G.nitems, G.ustage, G.bunits, G.rq, G.ctr, G.per_unit,
                        G.ray_clusters);
@@ -2437,7 +2505,7 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
     hipLaunchKernelGGL((rh_cluster_kernel<MODE, NODE, false>), dim3(G.nblocks), dim3(kThreads),
                        0, s, G.items, G.nitems, G.ustage, G.bunits, G.rq, G.ctr, G.per_unit,
                        G.ray_clusters);
-  if (G.ray_clusters > 1) {  // 0 and 1 send every block with work per-ray: no unit
+  if (G.ray_clusters > 1) {  // 1 sends every block with work per-ray: no unit
     hipLaunchKernelGGL(rh_unit_scan_kernel, dim3((G.nblocks + kScanThreads - 1) / kScanThreads),
                        dim3(kScanThreads), 0, s, G.bunits, G.nblocks);
     hipLaunchKernelGGL(rh_unit_pack_kernel, dim3((G.nblocks + kPackThreads / 64 - 1) /
@@ -2454,7 +2522,8 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
     const dim3 grid(G.grid > 0 ? (unsigned)G.grid : resident_grid(kernel, G.max_units));
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, s, G.items, G.units, G.ctr);
   };
-  if (G.bvh && G.big)
+  if (direct) {
+  } else if (G.bvh && G.big)
     launch(bvh_unit_kernel<MODE, NODE, 1024, 4>);
   else if (G.bvh)
     launch(bvh_unit_kernel<MODE, NODE, 256, 3>);
@@ -2471,13 +2540,17 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
   auto launch_rays = [&](auto kernel) {
     const dim3 grid(G.ray_grid > 0 ? std::max(1u, std::min((unsigned)G.ray_grid, G.max_chunks))
                                    : resident_grid(kernel, G.max_chunks, 64));
-    hipLaunchKernelGGL(kernel, grid, dim3(64), 0, s, G.items, G.rq, G.ctr, G.max_chunks,
+    hipLaunchKernelGGL(kernel, grid, dim3(64), 0, s, G.items, G.nitems,
+                       direct ? nullptr : G.rq, G.ctr, G.replist, G.max_chunks,
                        kWalk16[std::min(std::max(G.walk, 1), 7) - 1]);
   };
-  if (G.bvh)
-    launch_rays(ray_path_kernel<MODE, NODE, true>);
-  else
-    launch_rays(ray_path_kernel<MODE, NODE, false>);
+  if (G.nitems == 1) {
+    if (G.bvh) launch_rays(ray_path_kernel<MODE, NODE, true, true>);
+    else launch_rays(ray_path_kernel<MODE, NODE, false, true>);
+  } else {
+    if (G.bvh) launch_rays(ray_path_kernel<MODE, NODE, true, false>);
+    else launch_rays(ray_path_kernel<MODE, NODE, false, false>);
+  }
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (t1) {
@@ -2485,8 +2558,9 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
     if (e != hipSuccess) return e;
   }
   if (MODE != 2) {
-    hipLaunchKernelGGL(rh_finalize_kernel, grid1(G.nrays), dim3(kThreads), 0, s, G.items,
-                       G.nitems, G.nrays, G.ctr, G.replist);
+    if (!direct)
+      hipLaunchKernelGGL(rh_finalize_kernel, grid1(G.nrays), dim3(kThreads), 0, s, G.items,
+                         G.nitems, G.nrays, G.ctr, G.replist);
     if (MODE == 0 && G.replist && !G.bvh)
       hipLaunchKernelGGL((rh_repair_kernel<NODE>), dim3(64), dim3(kThreads), 0, s, G.items,
                          G.nitems, G.ctr, G.replist);
