@@ -713,8 +713,7 @@ int rt_scene_create(rt_ctx* ctx, const float* v9, const float* uv6, uint32_t ntr
     if (e == hipSuccess) {
       std::vector<uint4> snode;
       std::vector<uint32_t> sorder;
-      build_search_bvh(v9, ntri, search_stack(desc->kind == RT_ACCEL_RAYBVH), snode, sorder,
-                       s->sframe);
+      build_search_bvh(v9, ntri, snode, sorder, s->sframe);
       e = upload(s->d_snode, snode.data(), snode.size());
       if (e == hipSuccess) {
         const std::vector<float4> mts = mt_operands(v9, ntri, sorder.data());

@@ -168,22 +168,20 @@ constexpr int kDefaultWalk = 3;
 // Absent children have lower planes above their upper planes on every axis; should rounding let
 // a ray into one all the same, its reference is the record of some other triangle (the records
 // end with kSearchPad that no ray hits), whose test is harmless.  A depth-first walk
-// that keeps the unvisited children of every node on its path holds at most search_stack() of
+// that keeps the unvisited children of every node on its path holds at most kSearchStack of
 // them.
 constexpr uint32_t kSearchLeafBit = 0x80000000u;
 constexpr int kSearchDepth = 26;  // interior levels of the binary tree it is collapsed from
 // Entries of the walk's stack in LDS; the tree's builder keeps narrower nodes where a deeper
-// stack would be needed.  The most that leaves the kernel's work-groups at 18 per CU
-// (rayhierarchy, 5 wavefronts per SIMD by registers) or at 16 (ray-bvh, 4 wavefronts: its chain
-// evaluation needs the registers), LDS being handed out in 1,280-byte pieces.  With 26 entries
-// for both, the nodes were a fifth more on a cluster scene: 1 M segments 673 -> 626 us; ray-bvh
-// room task path depth 3, secondary 1,431 -> 1,080.
-constexpr int search_stack(bool bvh) { return bvh ? 35 : 30; }
+// stack would be needed.  The most that leaves the closest-hit kernel's work-groups (10,240 bytes
+// of LDS each, handed out in 1,280-byte pieces) at 16 per CU, which its registers allow too.
+// With 26 entries the nodes were a fifth more on a cluster scene (1 M segments 673 us, 626 with
+// 30).
+constexpr int kSearchStack = 32;
 constexpr uint32_t kSearchPad = 4;
-// Builds the search tree of `ntri` triangles (v9 in the caller's order) for a walk with `stack`
-// entries (at least kSearchDepth): the nodes (4 uint4 each), the search order (position ->
-// triangle index) and the frame of the node planes.
-void build_search_bvh(const float* v9, uint32_t ntri, int stack, std::vector<uint4>& nodes,
+// Builds the search tree of `ntri` triangles (v9 in the caller's order): the nodes (4 uint4
+// each), the search order (position -> triangle index) and the frame of the node planes.
+void build_search_bvh(const float* v9, uint32_t ntri, std::vector<uint4>& nodes,
                       std::vector<uint32_t>& order, SearchFrame& frame);
 
 // Allocation-free trace: a static device array of kNoAllocScratch bytes per device (defined in

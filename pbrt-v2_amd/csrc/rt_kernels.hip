@@ -1734,29 +1734,48 @@ __device__ __forceinline__ void key_swap(uint32_t& a, uint32_t& b) {
 // needed.  Otherwise the rays of the blocks that the cluster pass sent here leave their keys,
 // repair keys and flags as the block path does.
 // ONE: the group has one job; its table entry and the pointers in it are then uniform.
+//
+// Once the wavefront has no ray left to deal, its lanes run dry one after another while its
+// longest rays go on (a chunk's longest walk is 2-3 times its mean).  From then on it splits
+// rays: whenever at most kSplitLanes lanes hold one, each of those with unvisited nodes on its
+// stack gives the oldest of them, with a copy of the ray, to an idle lane.  The lanes of a ray
+// share its bound (or the news of its candidate) through LDS, and the last of them to finish
+// decides the ray.  Launches of few rays deal a wavefront fewer than 64 (nsub), so that more
+// wavefronts share them.  Measured: 1 M segments 596 -> 455 us, room task path depth 3, secondary
+// 1,104 -> 813 and occlusion 953 -> 629, twelve scenes' segments 398 -> 290, 100x4 leaves closest
+// 249 -> 114, box_uv clusters 164 -> 82, preview 64 x 64 41 -> 31 (44 with 64 rays a wavefront).
+// Splitting from 32 busy lanes was up to 10% slower than from 48, from 16 up to 50%; every second
+// round up to 20%, every fourth up to 70%.
+
 constexpr uint32_t kChainQ = 127;  // below 64 before a round, one more per lane in it
-// Registers for five wavefronts per SIMD (96 VGPRs), ray-bvh for four (its chain spilled 7-15:
-// room task path depth 3, secondary 1,344 -> 1,103 us); see search_stack for the LDS.  Keeping
-// only 24 or 16 stack entries in LDS and the rest in scratch memory, for more work-groups per
-// CU, was 3-6% slower, and six wavefronts per SIMD (80 VGPRs) a quarter to a half.
+constexpr uint32_t kSplitLanes = 48, kSplitRounds = 1;
+// State of a split ray (sRay): lanes at work in bits 0..7, then a hit at exactly tmin that the
+// repair pass must see (primary), or the candidate found (occlusion).
+constexpr uint32_t kRayLanes = 255u, kRayMark = 256u;
+// Registers for four wavefronts per SIMD (128 VGPRs) and LDS for as many, see kSearchStack; with
+// registers for five (96, 15-30 spilled) the room task's secondary rays took 1,315 us, the torus
+// closest hits 134 us (94).  Keeping only 24 or 16 stack entries in LDS and the rest in scratch
+// memory, for more work-groups per CU, was 3-6% slower.
 template <int MODE, int NODE, bool BVH, bool ONE>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5, 8))) void ray_path_kernel(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void ray_path_kernel(
     const RhItem* __restrict__ items, int nitems, const uint2* __restrict__ rq,
-    uint32_t* __restrict__ ctr, uint32_t* __restrict__ replist, uint32_t nchunks,
+    uint32_t* __restrict__ ctr, uint32_t* __restrict__ replist, uint32_t nchunks, uint32_t nsub,
     uint32_t walk16) {
-  __shared__ uint32_t sStk[search_stack(BVH)][64];
+  __shared__ uint32_t sStk[kSearchStack][64];
   // candidates [0, qn) and, from the far end, rays to trace again [kChainQ - nf, kChainQ)
   __shared__ uint32_t sQIdx[kChainQ], sQRef[kChainQ];
   __shared__ uint16_t sQJob[kChainQ];
+  __shared__ unsigned long long sBest[MODE == 2 ? 1 : 64];  // split rays, by the lane that had it
+  __shared__ uint32_t sRay[64];
   constexpr uint32_t kDone = 0xffffffffu;  // not a reference (positions are below 2^31)
   const float kInf = __int_as_float(0x7f800000);
   auto widened = [](float t) { return t + fabsf(t) * kSlack; };
   const int lane = threadIdx.x;
   const uint64_t lanes_below = (1ull << lane) - 1ull;
   // wavefront-uniform: the chunk being dealt and its next slot, the queue's counts
-  uint32_t cjob = 0, cblk = 0, cpart = 0, cslot = 64;
-  uint32_t qn = 0, nf = 0;
-  bool more = true;
+  uint32_t cjob = 0, cblk = 0, cpart = 0, cslot = 64, cend = 64;
+  uint32_t qn = 0, nf = 0, rounds = 0;
+  bool more = true, split = false;
   // lane state
   bool act = false, careful = false;
   uint32_t jk = 0, idx = 0;
@@ -1765,12 +1784,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
   // tlo, thi: the interval's ends, widened; thi follows the closest bound
   float tmin = 0.f, tmax = 0.f, tlo = 0.f, thi = 0.f;
   uint64_t best = kMissKey;   // closest: the nearest hit (verified when careful)
-  uint32_t rep = kNoKey32;    // primary: the nearest repair-region hit (likewise)
-  uint32_t cand = 0;          // the candidate: triangle id, ray-bvh occlusion its BVH leaf
+  bool mark = false;          // primary: a repair-region hit at exactly tmin (likewise)
+  uint32_t cand = 0;          // occlusion: the candidate triangle, for ray-bvh its BVH leaf
   bool track_rep = false;
-  int sp = 0;
+  int sp = 0, sb = 0;         // the lane's stack entries [sb, sp)
+  uint32_t own = 0;           // the lane whose sRay / sBest a split ray uses
   uint32_t cur = kDone, pl = kDone;
-  auto pop = [&]() { return sp > 0 ? sStk[--sp][lane] : kDone; };
+  auto pop = [&]() { return sp > sb ? sStk[--sp][lane] : kDone; };
   const bool direct = rq == nullptr;
   // the cluster pass sets ctr[4] when it routed any block here
   if (!direct && __builtin_amdgcn_readfirstlane(ctr[4]) == 0u) return;
@@ -1792,9 +1812,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
   auto restart = [&]() {
     careful = true;
     best = kMissKey;
-    rep = kNoKey32;
+    mark = false;
     thi = MODE == 2 ? widened(tmax) : kInf;
-    sp = 0;
+    sp = sb = 0;
     cur = 0u;  // interior node 0 (the root)
     pl = kDone;
   };
@@ -1849,14 +1869,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
         __syncthreads();
       } else {
         if (!more) break;
-        if (cslot >= 64) {
+        if (cslot >= cend) {
           uint32_t e = 0;
-          if (lane == 0) e = claim_unit(ctr, nchunks, claim, 1);
+          if (lane == 0) e = claim_unit(ctr, nchunks * nsub, claim, 1);
           e = __builtin_amdgcn_readfirstlane(e);
-          if (e >= nchunks) {
+          if (e >= nchunks * nsub) {
             more = false;
             break;
           }
+          const uint32_t sub = e % nsub;
+          e /= nsub;
           uint32_t c;
           if (direct) {
             cjob = ONE ? 0u : (uint32_t)find_chunk_item(items, nitems, e);
@@ -1870,9 +1892,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
           const uint32_t nch = ((uint32_t)item(cjob).g.rb + 63u) / 64u;
           cblk = c / nch;
           cpart = c - cblk * nch;
-          cslot = 0;
+          cslot = 64u / nsub * sub;
+          cend = cslot + 64u / nsub;
         }
-        const uint32_t avail = 64u - cslot;
+        const uint32_t avail = cend - cslot;
         if (!act && rank < avail) {
           const RhItem& it = item(cjob);
           const RHGeom& g = it.g;
@@ -1913,6 +1936,64 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
       if (qn == 0) break;  // nothing to trace again either: the deal takes those first
       run_chains(min(qn, 64u));
       continue;
+    }
+    if (!more && nf == 0 && ++rounds >= kSplitRounds) {
+      const uint64_t am = __ballot(act);
+      if ((uint32_t)__popcll(am) <= kSplitLanes) {
+        rounds = 0;
+        if (!split) {
+          split = true;
+          own = (uint32_t)lane;
+          sRay[lane] = 1u | (mark ? kRayMark : 0u);
+          if constexpr (MODE != 2) sBest[lane] = best;
+          __syncthreads();
+        }
+        const bool gives = act && !careful && sp > sb;
+        const uint64_t gm = __ballot(gives);
+        const uint32_t n = min((uint32_t)__popcll(gm), (uint32_t)__popcll(~am));
+        if (n > 0) {
+          // the r-th giving lane and the r-th idle lane meet in entry 64 + r of the queue, which
+          // holds less than 64 candidates here and nothing to trace again
+          const uint32_t gr = (uint32_t)__popcll(gm & lanes_below);
+          const uint32_t ir = (uint32_t)__popcll(~am & lanes_below);
+          if (gives && gr < n) {
+            sQIdx[64 + gr] = sStk[sb++][lane];
+            sQRef[64 + gr] = (uint32_t)lane;
+            atomicAdd(&sRay[own], 1u);
+          }
+          __syncthreads();
+          const bool takes = !act && ir < n;
+          const int from = takes ? (int)sQRef[64 + ir] : lane;
+          auto copy = [&](auto& v) { v = __shfl(v, from); };
+          copy(o.x); copy(o.y); copy(o.z);
+          copy(d.x); copy(d.y); copy(d.z);
+          copy(sr.ih.x); copy(sr.ih.y); copy(sr.ih.z);
+          copy(sr.cn.x); copy(sr.cn.y); copy(sr.cn.z);
+          copy(sr.cf.x); copy(sr.cf.y); copy(sr.cf.z);
+          copy(tmin); copy(tmax); copy(tlo); copy(thi);
+          copy(idx); copy(jk); copy(own);
+          const bool tr = __shfl((int)track_rep, from) != 0;
+          if constexpr (MODE != 2) {
+            const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(best >> 32), from),
+                           lo = (uint32_t)__shfl((int)(uint32_t)best, from);
+            best = ((uint64_t)hi << 32) | lo;
+          }
+          if (takes) {
+            act = true;
+            careful = false;
+            mark = false;
+            track_rep = tr;
+            sp = sb = 0;
+            pl = kDone;
+            cur = sQIdx[64 + ir];
+            if (cur & kSearchLeafBit) {
+              pl = cur;
+              cur = kDone;
+            }
+          }
+          __syncthreads();
+        }
+      }
     }
     const RhItem& it = item(jk);
     const auto snode = glb(it.snode);
@@ -2007,7 +2088,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
           if (t > tmin && t < tmax) {  // intersectAllLeaves.cl:177-179
             if (!careful) {
               cand = ref;
-              push = true;
+              push = !split || !(atomicOr(&sRay[own], kRayMark) & kRayMark);
+              act = push;  // false: another lane of the split ray has its candidate
             } else if (chain(it, idx, ref)) {
               glb(it.occ)[idx] = 1;
               act = false;
@@ -2015,16 +2097,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
           }
         } else {
           const bool main = t > tmin && t < kInf;
-          const bool rp = track_rep && repair_region(b1, b2) && t >= tmin;
+          // A repair-region hit beyond tmin is a main hit too, so the nearest of them is never
+          // below the answer; only one at tmin is kept apart.
+          const bool rp = track_rep && t == tmin && repair_region(b1, b2);
           const uint64_t key = hit_key(t, (int32_t)id);
-          const bool um = main && key < best, ur = rp && fkey(t) < rep;
-          if ((um || ur) && (!careful || chain(it, idx, ref))) {
+          const bool um = main && key < best;
+          if ((um || (rp && !mark)) && (!careful || chain(it, idx, id))) {
             if (um) {
               best = key;
-              cand = ref;
               thi = widened(t);
+              if (split && !careful) atomicMin(&sBest[own], (unsigned long long)key);
             }
-            if (ur) rep = fkey(t);
+            if (rp) mark = true;
           }
         }
       }
@@ -2035,25 +2119,40 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
       cur = pop();
     }
     // rays that are done: a verified result is written; the others queue their candidate, if
-    // they have one
+    // they have one (a split ray's last lane for all of them)
     if (act && !push && cur == kDone && pl == kDone) {
+      bool last = true;
+      if (split && !careful) {
+        if (MODE != 2 && mark) atomicOr(&sRay[own], kRayMark);
+        const uint32_t was = atomicAdd(&sRay[own], 0xffffffffu);
+        last = (was & kRayLanes) == 1u && !(MODE == 2 && (was & kRayMark));
+        if constexpr (MODE != 2) {
+          best = sBest[own];
+          mark = (was & kRayMark) != 0u;
+        }
+      }
       const float tstar = best == kMissKey ? kInf : fkey_inv((uint32_t)(best >> 32));
-      if constexpr (MODE == 2) {
+      // whether the repair pass can change the ray (rh_finalize_kernel's rule; where t - EPS
+      // rounds to t it is not asked which hit lies in the repair region)
+      const bool repairs = MODE == 0 && track_rep &&
+                           ((mark && !(tmin > tstar - kEps)) ||
+                            (best != kMissKey && !(tstar > tstar - kEps)));
+      if (!last) {
+        act = false;
+      } else if constexpr (MODE == 2) {
         if (direct) write_miss(it, idx);
         act = false;
       } else if (careful) {
         if (direct) {
           if (best == kMissKey) write_miss(it, idx);
           else write_hit(it.r, it.v9, it.uv6, idx, (int32_t)(uint32_t)best, tstar, it.out);
-          // as rh_finalize_kernel lists it
-          if (MODE == 0 && rep != kNoKey32 && !(fkey_inv(rep) > tstar - kEps))
-            replist[atomicAdd(&ctr[2], 1u)] = it.ray_base + idx;
+          if (repairs) replist[atomicAdd(&ctr[2], 1u)] = it.ray_base + idx;
         } else {
           if (best != kMissKey) glb(it.keys)[idx] = best;
-          if (track_rep && rep != kNoKey32) glb(it.repkeys)[idx] = rep;
+          if (repairs) glb(it.repkeys)[idx] = fkey(mark ? tmin : tstar);
         }
         act = false;
-      } else if (rep != kNoKey32 && !(fkey_inv(rep) > tstar - kEps)) {
+      } else if (repairs) {
         restart();
       } else if (best == kMissKey) {
         if (direct) write_miss(it, idx);
@@ -2069,7 +2168,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
       if (push) {
         if (room) {
           sQIdx[e] = idx;
-          sQRef[e] = cand;
+          sQRef[e] = MODE == 2 ? cand : (uint32_t)best;
           sQJob[e] = (uint16_t)jk;
           if constexpr (MODE != 2) {
             if (direct) glb(it.out.t)[idx] = fkey_inv((uint32_t)(best >> 32));
@@ -2083,6 +2182,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(BVH ? 4 : 5,
       qn = min(qn + (uint32_t)__popcll(pb), kChainQ - nf);
       __syncthreads();
       if (qn >= 64u) run_chains(64u);
+    }
+    // the other lanes' news of a split ray
+    if (split && act && !careful) {
+      if constexpr (MODE == 2) {
+        if (sRay[own] & kRayMark) act = false;
+      } else {
+        const uint64_t b = sBest[own];
+        if (b < best) {
+          best = b;
+          thi = widened(fkey_inv((uint32_t)(b >> 32)));
+        }
+      }
     }
   }
 }
@@ -2538,10 +2649,16 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
     if (e != hipSuccess) return e;
   }
   auto launch_rays = [&](auto kernel) {
-    const dim3 grid(G.ray_grid > 0 ? std::max(1u, std::min((unsigned)G.ray_grid, G.max_chunks))
-                                   : resident_grid(kernel, G.max_chunks, 64));
+    const unsigned slots = resident_grid(kernel, 0x7fffffffu, 64);
+    // a launch that would leave slots empty deals 64 / nsub rays a wavefront, at least 4 (64
+    // wavefronts of 64 rays against 1,024 of 4: 44 -> 31 us); more wavefronts than slots would
+    // run one after another (torus 333 x 251 69 -> 124 us)
+    unsigned nsub = 1;
+    while (nsub < 16 && G.max_chunks * 2 * nsub <= slots) nsub *= 2;
+    const unsigned most = G.ray_grid > 0 ? (unsigned)G.ray_grid : slots;
+    const dim3 grid(std::max(1u, std::min(most, G.max_chunks * nsub)));
     hipLaunchKernelGGL(kernel, grid, dim3(64), 0, s, G.items, G.nitems,
-                       direct ? nullptr : G.rq, G.ctr, G.replist, G.max_chunks,
+                       direct ? nullptr : G.rq, G.ctr, G.replist, G.max_chunks, nsub,
                        kWalk16[std::min(std::max(G.walk, 1), 7) - 1]);
   };
   if (G.nitems == 1) {

@@ -351,7 +351,7 @@ class Collapser {
 
 }  // namespace
 
-void build_search_bvh(const float* v9, uint32_t ntri, int stack, std::vector<uint4>& nodes,
+void build_search_bvh(const float* v9, uint32_t ntri, std::vector<uint4>& nodes,
                       std::vector<uint32_t>& order, SearchFrame& frame) {
   nodes.clear();
   order.clear();
@@ -408,7 +408,7 @@ void build_search_bvh(const float* v9, uint32_t ntri, int stack, std::vector<uin
   b.build(0, ntri, 1, box);
   Collapser::Child c[4] = {Collapser::Child{bin[0].box[0], bin[0].ref[0]},
                            Collapser::Child{bin[0].box[1], bin[0].ref[1]}, {}, {}};
-  w.node(0, c, 2, stack);
+  w.node(0, c, 2, kSearchStack);
 }
 
 }  // namespace rti
