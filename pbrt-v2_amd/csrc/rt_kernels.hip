@@ -314,6 +314,17 @@ __device__ __forceinline__ int find_chunk_item(const RhItem* __restrict__ items,
   }
   return k - 1;
 }
+// The same per lane.
+__device__ __forceinline__ uint32_t find_chunk_item_lane(const RhItem* __restrict__ items, int n,
+                                                         uint32_t gc) {
+  int lo = 0, hi = n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (items[mid].chunk_base <= gc) lo = mid;
+    else hi = mid - 1;
+  }
+  return (uint32_t)lo;
+}
 // Job of a global ray index (per lane).
 __device__ __forceinline__ int find_ray_item(const RhItem* __restrict__ items, int n,
                                              uint32_t gr) {
@@ -1740,15 +1751,25 @@ __device__ __forceinline__ void key_swap(uint32_t& a, uint32_t& b) {
 // rays: whenever at most kSplitLanes lanes hold one, each of those with unvisited nodes on its
 // stack gives the oldest of them, with a copy of the ray, to an idle lane.  The lanes of a ray
 // share its bound (or the news of its candidate) through LDS, and the last of them to finish
-// decides the ray.  Launches of few rays deal a wavefront fewer than 64 (nsub), so that more
-// wavefronts share them.  Measured: 1 M segments 596 -> 455 us, room task path depth 3, secondary
+// decides the ray.  Measured: 1 M segments 596 -> 455 us, room task path depth 3, secondary
 // 1,104 -> 813 and occlusion 953 -> 629, twelve scenes' segments 398 -> 290, 100x4 leaves closest
-// 249 -> 114, box_uv clusters 164 -> 82, preview 64 x 64 41 -> 31 (44 with 64 rays a wavefront).
-// Splitting from 32 busy lanes was up to 10% slower than from 48, from 16 up to 50%; every second
-// round up to 20%, every fourth up to 70%.
-
+// 249 -> 114, box_uv clusters 164 -> 82.  Splitting from 32 busy lanes was up to 10% slower than
+// from 48, from 16 up to 50%; every second round up to 20%, every fourth up to 70%.
+//
+// A launch of at most one chunk per resident wavefront deals each its rays at once (`spread` of
+// them), in runs of 16 taken from distant parts of the launch: neighbouring rays are long
+// together, and the launch lasts as long as its longest wavefront.  With whole chunks the mean
+// wavefront of the torus 512 x 512 occlusion ended after 18 us, the last after 114; now 31 and
+// 69 (119 -> 70 us, closest 93 -> 85; 333 x 251 ia 72 -> 53 and 69 -> 57).  Fewer rays than that
+// are spread over more wavefronts, at least four each (64 wavefronts of 64 rays 44 us, 1,024 of
+// 4 31 us); more wavefronts than are resident run one after another (333 x 251: 69 -> 124).
 constexpr uint32_t kChainQ = 127;  // below 64 before a round, one more per lane in it
-constexpr uint32_t kSplitLanes = 48, kSplitRounds = 1;
+constexpr uint32_t kSplitLanes = 48;
+// Idle lanes from which a wavefront deals new rays.  A deal is a chain of loads that every lane
+// waits for; one for each idle lane took 18-25% of a long launch (1 M camera rays, 200,000
+// triangles: any idle lane 801 us, 4 lanes 769, 8 765, 16 761, 24 781; twelve scenes 561, 523,
+// 507, 499, 494).
+constexpr uint32_t kDealLanes = 16;
 // State of a split ray (sRay): lanes at work in bits 0..7, then a hit at exactly tmin that the
 // repair pass must see (primary), or the candidate found (occlusion).
 constexpr uint32_t kRayLanes = 255u, kRayMark = 256u;
@@ -1759,7 +1780,7 @@ constexpr uint32_t kRayLanes = 255u, kRayMark = 256u;
 template <int MODE, int NODE, bool BVH, bool ONE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void ray_path_kernel(
     const RhItem* __restrict__ items, int nitems, const uint2* __restrict__ rq,
-    uint32_t* __restrict__ ctr, uint32_t* __restrict__ replist, uint32_t nchunks, uint32_t nsub,
+    uint32_t* __restrict__ ctr, uint32_t* __restrict__ replist, uint32_t nchunks, uint32_t spread,
     uint32_t walk16) {
   __shared__ uint32_t sStk[kSearchStack][64];
   // candidates [0, qn) and, from the far end, rays to trace again [kChainQ - nf, kChainQ)
@@ -1773,8 +1794,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
   const int lane = threadIdx.x;
   const uint64_t lanes_below = (1ull << lane) - 1ull;
   // wavefront-uniform: the chunk being dealt and its next slot, the queue's counts
-  uint32_t cjob = 0, cblk = 0, cpart = 0, cslot = 64, cend = 64;
-  uint32_t qn = 0, nf = 0, rounds = 0;
+  uint32_t cjob = 0, cblk = 0, cpart = 0, cslot = 64;
+  uint32_t qn = 0, nf = 0;
   bool more = true, split = false;
   // lane state
   bool act = false, careful = false;
@@ -1854,7 +1875,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     // deal rays to the lanes without one: first those to trace again, then the queue's
     for (;;) {
       const uint64_t need = __ballot(!act);
-      if (need == 0) break;
+      if (need == 0 || (more && nf == 0 && (uint32_t)__popcll(need) < kDealLanes)) break;
       const uint32_t rank = (uint32_t)__popcll(need & lanes_below);
       bool got = false;
       if (nf > 0) {
@@ -1869,49 +1890,78 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
         __syncthreads();
       } else {
         if (!more) break;
-        if (cslot >= cend) {
-          uint32_t e = 0;
-          if (lane == 0) e = claim_unit(ctr, nchunks * nsub, claim, 1);
-          e = __builtin_amdgcn_readfirstlane(e);
-          if (e >= nchunks * nsub) {
-            more = false;
-            break;
+        // the lane's job, block, chunk of the block and slot in it
+        uint32_t job = 0xffffffffu, blk = 0, part = 0, q = 0;
+        if (spread != 0) {
+          // the wavefront's only rays: `spread` of them in runs of at most 16, one run in each
+          // of the launch's equal parts; consecutive wavefronts of an XCD take neighbouring runs
+          more = false;
+          const uint32_t run = min(spread, 16u);
+          const uint32_t w = (blockIdx.x % (uint32_t)kClaimQueues) * (gridDim.x / kClaimQueues) +
+                             blockIdx.x / (uint32_t)kClaimQueues;
+          const uint32_t slot = ((uint32_t)lane / run * gridDim.x + w) * run + (uint32_t)lane % run;
+          uint32_t c = slot / 64u;
+          q = slot % 64u;
+          if ((uint32_t)lane < spread && c < nchunks) {
+            if (direct) {
+              job = ONE ? 0u : find_chunk_item_lane(items, nitems, c);
+              c -= item(job).chunk_base;
+            } else {
+              const uint2 v = rq[c];
+              job = v.x;  // ~0u: a block-path block
+              c = v.y;
+            }
+            if (job != 0xffffffffu) {
+              const uint32_t nch = ((uint32_t)item(job).g.rb + 63u) / 64u;
+              blk = c / nch;
+              part = c - blk * nch;
+            }
           }
-          const uint32_t sub = e % nsub;
-          e /= nsub;
-          uint32_t c;
-          if (direct) {
-            cjob = ONE ? 0u : (uint32_t)find_chunk_item(items, nitems, e);
-            c = e - item(cjob).chunk_base;
-          } else {
-            const uint2 w = rq[e];
-            cjob = __builtin_amdgcn_readfirstlane(w.x);
-            if (cjob == 0xffffffffu) continue;  // a block-path block
-            c = __builtin_amdgcn_readfirstlane(w.y);
+        } else {
+          if (cslot >= 64u) {
+            uint32_t e = 0;
+            if (lane == 0) e = claim_unit(ctr, nchunks, claim, 1);
+            e = __builtin_amdgcn_readfirstlane(e);
+            if (e >= nchunks) {
+              more = false;
+              break;
+            }
+            uint32_t c;
+            if (direct) {
+              cjob = ONE ? 0u : (uint32_t)find_chunk_item(items, nitems, e);
+              c = e - item(cjob).chunk_base;
+            } else {
+              const uint2 w = rq[e];
+              cjob = __builtin_amdgcn_readfirstlane(w.x);
+              if (cjob == 0xffffffffu) continue;  // a block-path block
+              c = __builtin_amdgcn_readfirstlane(w.y);
+            }
+            const uint32_t nch = ((uint32_t)item(cjob).g.rb + 63u) / 64u;
+            cblk = c / nch;
+            cpart = c - cblk * nch;
+            cslot = 0;
           }
-          const uint32_t nch = ((uint32_t)item(cjob).g.rb + 63u) / 64u;
-          cblk = c / nch;
-          cpart = c - cblk * nch;
-          cslot = 64u / nsub * sub;
-          cend = cslot + 64u / nsub;
+          q = cslot + rank;
+          if (q < 64u) job = cjob;
+          blk = cblk;
+          part = cpart;
+          cslot += min(64u - cslot, (uint32_t)__popcll(need));
         }
-        const uint32_t avail = cend - cslot;
-        if (!act && rank < avail) {
-          const RhItem& it = item(cjob);
+        if (!act && job != 0xffffffffu) {
+          const RhItem& it = item(job);
           const RHGeom& g = it.g;
-          const int top = g.L - 1;
-          const int K = (int)cblk % g.gw[top], J = (int)cblk / g.gw[top];
+          const int gwt = g.gw[g.L - 1];
+          const int J = (int)blk / gwt, K = (int)blk - J * gwt;
           int x = 0, y = 0, leaf = 0;
-          if (slot_xy(g, K, J, (int)(cpart * 64u + cslot + rank), x, y, leaf)) {
+          if (slot_xy(g, K, J, (int)(part * 64u + q), x, y, leaf)) {
             idx = (uint32_t)y * (uint32_t)g.W + (uint32_t)x;
-            jk = cjob;
+            jk = job;
             careful = false;
             got = it.ntri > 0 &&
                   (MODE == 0 || it.r.valid == nullptr || glb(it.r.valid)[idx] != 0);
             if (direct && !got) write_miss(it, idx);
           }
         }
-        cslot += min(avail, (uint32_t)__popcll(need));
       }
       if (got) {
         const RhItem& it = item(jk);
@@ -1937,10 +1987,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
       run_chains(min(qn, 64u));
       continue;
     }
-    if (!more && nf == 0 && ++rounds >= kSplitRounds) {
+    if (!more && nf == 0) {
       const uint64_t am = __ballot(act);
       if ((uint32_t)__popcll(am) <= kSplitLanes) {
-        rounds = 0;
         if (!split) {
           split = true;
           own = (uint32_t)lane;
@@ -2592,10 +2641,11 @@ unsigned resident_grid(F kernel, uint32_t cap, int threads = kThreads) {
   return std::max(1u, std::min(n, std::max(cap, 1u)));
 }
 
-// RT_PARAM_WALK_* 1..7 as sixteenths of the lanes holding a ray.  The built-in 3 (a half) was the
+// RT_PARAM_WALK_* 1..7 as sixteenths of the lanes holding a ray.  The built-in 3 was the
 // fastest or within 2% of it on every workload measured (1 M segments: 7/8 of the lanes 856 us,
-// 3/4 775, 1/2 688, 1/4 688, 1/8 770).
-constexpr uint32_t kWalk16[7] = {14, 12, 8, 4, 2, 1, 0};
+// 3/4 775, 1/2 688, 1/4 688, 1/8 770; with the lanes of a wavefront better filled, camera rays of
+// twelve scenes 555 us at 1/2, 538 at 3/8, 527 at 1/4).
+constexpr uint32_t kWalk16[7] = {14, 12, 6, 4, 2, 1, 0};
 
 // Launch sequence of one rayhierarchy group with the mode and node type fixed.
 template <int MODE, int NODE>
@@ -2649,16 +2699,18 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
     if (e != hipSuccess) return e;
   }
   auto launch_rays = [&](auto kernel) {
+    unsigned spread = 0;
     const unsigned slots = resident_grid(kernel, 0x7fffffffu, 64);
-    // a launch that would leave slots empty deals 64 / nsub rays a wavefront, at least 4 (64
-    // wavefronts of 64 rays against 1,024 of 4: 44 -> 31 us); more wavefronts than slots would
-    // run one after another (torus 333 x 251 69 -> 124 us)
-    unsigned nsub = 1;
-    while (nsub < 16 && G.max_chunks * 2 * nsub <= slots) nsub *= 2;
-    const unsigned most = G.ray_grid > 0 ? (unsigned)G.ray_grid : slots;
-    const dim3 grid(std::max(1u, std::min(most, G.max_chunks * nsub)));
+    const dim3 grid = [&]() {
+      if (G.ray_grid > 0) return std::max(1u, std::min((unsigned)G.ray_grid, G.max_chunks));
+      if (G.max_chunks > slots) return slots;
+      const unsigned rays = G.max_chunks * 64u;
+      spread = (rays + slots - 1) / slots;
+      spread = spread > 16 ? (spread + 15) / 16 * 16 : spread > 8 ? 16 : spread > 4 ? 8 : 4;
+      return ((rays + spread - 1) / spread + kClaimQueues - 1) / kClaimQueues * kClaimQueues;
+    }();
     hipLaunchKernelGGL(kernel, grid, dim3(64), 0, s, G.items, G.nitems,
-                       direct ? nullptr : G.rq, G.ctr, G.replist, G.max_chunks, nsub,
+                       direct ? nullptr : G.rq, G.ctr, G.replist, G.max_chunks, spread,
                        kWalk16[std::min(std::max(G.walk, 1), 7) - 1]);
   };
   if (G.nitems == 1) {
