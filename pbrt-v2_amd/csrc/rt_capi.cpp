@@ -451,7 +451,7 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
     uint32_t ray;
     int rgrid, walk;
     uint32_t nblocks, nrays;
-    bool big, repair;
+    bool big, repair, one_ray;
     int per, grid;
   };
   std::vector<GroupLayout> gl(keys.size());
@@ -472,6 +472,7 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
     L.nrays = 0;
     L.big = prm.tile[mi] == 1;
     L.repair = false;
+    L.one_ray = true;
     uint64_t blocks = 0, rays = 0;
     for (int j : members[gi]) {
       const RhJob& jb = jobs[j];
@@ -491,6 +492,7 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
       if (it.g.rb <= kMaxBlockRays && it.g.L <= kUnitLevels && (it.g.rb > 256 || it.g.L > 3))
         L.big = true;
       if (it.repair_run > 0) L.repair = true;
+      if (!one_ray_leaves(it.g)) L.one_ray = false;
       L.max_units += (size_t)it.g.ntop * ((it.nclusters + L.per - 1) / L.per);
       L.max_chunks += (size_t)it.g.ntop * (size_t)((it.g.rb + 63) / 64);
       off_nodes[j] = total;
@@ -563,6 +565,7 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
     G.node = keys[gi].second & 3;
     G.bvh = keys[gi].second >> 2;
     G.big = gl[gi].big ? 1 : 0;
+    G.one_ray = gl[gi].one_ray ? 1 : 0;
     G.nblocks = gl[gi].nblocks;
     G.nrays = gl[gi].nrays;
     G.units = (uint4*)(A + gl[gi].units);
@@ -1053,6 +1056,7 @@ int rt_trace_closest_noalloc(rt_scene* s, const rt_rays* rays, int32_t mode, con
   G.node = s->desc.node;
   G.bvh = kind == RT_ACCEL_RAYBVH ? 1 : 0;
   G.big = (it.g.rb > 256 || it.g.L > 3) ? 1 : 0;
+  G.one_ray = one_ray_leaves(it.g) ? 1 : 0;
   G.nblocks = (uint32_t)it.g.ntop;
   G.nrays = (uint32_t)n;
   G.per_unit = 1;
@@ -1197,12 +1201,19 @@ static int batch_launch(rt_batch* b, const std::vector<RhGroup>& groups, hipStre
 // kernels (build, cluster pass, finalize) overlap another's traversal.  The side streams and
 // events exist before the capture begins (see ensure_side).
 constexpr size_t kSideStreams = 3;  // with the caller's stream, the device's 4 hardware queues
+constexpr uint32_t kForkLateChunks = 4096;  // 64-ray chunks: 16 wavefronts on each of 256 CUs
 static int batch_launch_forked(rt_batch* b, const std::vector<RhGroup>& groups, hipStream_t hs) {
   const size_t nside = std::min(groups.size() - 1, b->side.size());
   if (groups.size() < 2 || nside == 0) return batch_launch(b, groups, hs, false);
-  RT_TRY(hipEventRecord(b->forks[0], hs));
+  // A first group that fills the device forks after its build (the point of the event that
+  // launch_rh_group records before the traversal), so that its traversal takes the device first
+  // and the others' fill in behind it; forked at the start, two such traversals split the
+  // device between them (twelve scenes: 838 us a step against 738).
+  const bool late = groups[0].max_chunks > kForkLateChunks;
+  if (!late) RT_TRY(hipEventRecord(b->forks[0], hs));
+  else RT_TRY(launch_rh_group(groups[0], hs, b->forks[0], nullptr, nullptr));
   for (size_t k = 0; k < nside; ++k) RT_TRY(hipStreamWaitEvent(b->side[k], b->forks[0], 0));
-  for (size_t gi = 0; gi < groups.size(); ++gi)
+  for (size_t gi = late ? 1 : 0; gi < groups.size(); ++gi)
     RT_TRY(launch_rh_group(groups[gi], gi == 0 ? hs : b->side[(gi - 1) % nside], nullptr,
                            nullptr, nullptr));
   for (size_t k = 0; k < nside; ++k) {

@@ -64,6 +64,9 @@ struct RHGeom {
 // Returns 0 on success, nonzero when the shape is not supported.
 int rh_geometry(int W, int H, int cx, int cy, int height, RHGeom* g);
 
+// Whether the leaf build has at most one ray for each of a leaf's lanes.
+inline bool one_ray_leaves(const RHGeom& g) { return g.g <= 64 && (g.g & (g.g - 1)) == 0; }
+
 struct HitOut {
   int32_t* id;
   float *t, *u, *v, *dpdu, *dpdv;
@@ -132,6 +135,7 @@ struct RhGroup {
   int node;  // 0 box_dir, 1 ia
   int big;   // some job has more than 256 rays per block or 4 levels
   int bvh;   // ray-bvh jobs (product traversal with the scene's BVH)
+  int one_ray;  // every job's leaves hold a power of two of at most 64 rays (one_ray_leaves)
   uint32_t nblocks, nrays;
   uint4* units;       // {item, block, first cluster, count}, compacted from ustage
   uint4* ustage;      // the units of every block at fixed slots (job unit_base + block * stride)

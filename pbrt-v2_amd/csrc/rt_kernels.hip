@@ -110,7 +110,7 @@ __device__ __forceinline__ bool slot_xy(const RHGeom& g, int K, int J, int rl, i
   if (rl >= g.rb) return false;
   leaf = rl / g.g;
   int q = rl - leaf * g.g;
-  int lk = leaf % g.nlx, lj = leaf / g.nlx;
+  int lk = leaf & (g.nlx - 1), lj = leaf >> (g.L - 1);  // nlx is 2^(L-1)
   x = K * g.bw + lk * g.cx + q % g.cx;
   y = J * g.bh + lj * g.cy + q / g.cx;
   return x < g.W && y < g.H;
@@ -135,27 +135,26 @@ __device__ __forceinline__ void box_combine(float* a, bool& ha, const float* b, 
 // [-1, 1] and marks it as a restart: the kernel assigns that interval, dropping what the
 // leaf's earlier rays gave, and later rays widen it again.
 template <bool USE_VALID, bool UV>
-__device__ __forceinline__ void ray_box(const RaysDev& r, size_t i, float* v, bool& restart) {
-  const float dx = r.dx[i], dy = r.dy[i], dz = r.dz[i];
+__device__ __forceinline__ void ray_box(V3 o, V3 d, float* v, bool& restart) {
   restart = false;
   if constexpr (UV) {
-    const bool flat = dx == 0.f;
-    v[0] = v[3] = flat ? 0.f : dy / dx;
+    const bool flat = d.x == 0.f;
+    v[0] = v[3] = flat ? 0.f : d.y / d.x;
     if (USE_VALID && flat) {
       v[0] = -1.f;
       v[3] = 1.f;
       restart = true;
     }
-    v[1] = v[4] = dz;
+    v[1] = v[4] = d.z;
     v[2] = v[5] = 0.f;
   } else {
-    v[0] = v[3] = dx;
-    v[1] = v[4] = dy;
-    v[2] = v[5] = dz;
+    v[0] = v[3] = d.x;
+    v[1] = v[4] = d.y;
+    v[2] = v[5] = d.z;
   }
-  v[6] = v[9] = r.ox[i];
-  v[7] = v[10] = r.oy[i];
-  v[8] = v[11] = r.oz[i];
+  v[6] = v[9] = o.x;
+  v[7] = v[10] = o.y;
+  v[8] = v[11] = o.z;
 }
 
 // Merge of the rays of one leaf in the reference's read order, a before b: the component-wise
@@ -177,34 +176,114 @@ __device__ __forceinline__ void leaf_merge(float* a, bool& ha, bool& ra, const f
   ra = ra || rb;
 }
 
-// Box of the leaf whose first ray is (x0, y0): its rays merged one by one in the reference's
-// read order (row by row, left to right); zeros and false when no ray is traced.
-template <bool USE_VALID, bool UV>
-__device__ bool leaf_box(const RHGeom& g, const RaysDev& r, int x0, int y0, float* v) {
-  bool have = false, restart = false;
-  for (int y = y0; y < min(g.H, y0 + g.cy); ++y)
-    for (int x = x0; x < min(g.W, x0 + g.cx); ++x) {
-      const size_t i = (size_t)y * g.W + x;
-      if (USE_VALID && r.valid != nullptr && r.valid[i] == 0) continue;
+// Value of the lane that lane ^ m names, for a value that is the same in each group of m lanes
+// (so any lane of the neighbouring group will do): DPP moves within a row of 16, a permute beyond.
+template <int M>
+__device__ __forceinline__ int from_group(int v) {
+  if constexpr (M == 1) return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, false);
+  if constexpr (M == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, false);
+  if constexpr (M == 4) return __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, false);
+  if constexpr (M == 8) return __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, false);
+  return __shfl_xor(v, M);
+}
+// Merges the boxes of neighbouring groups of M lanes, the lower group's rays first, when a leaf
+// has more than M lanes.
+template <int M, bool RESTART>
+__device__ __forceinline__ void merge_groups(float* v, bool& have, bool& restart, int lanes,
+                                             int tid) {
+  if (M >= lanes) return;  // uniform
+  float o[12];
+  for (int k = 0; k < 12; ++k) o[k] = __int_as_float(from_group<M>(__float_as_int(v[k])));
+  bool ho = from_group<M>((int)have) != 0;
+  bool ro = RESTART && from_group<M>((int)restart) != 0;
+  if (tid & M) {  // the neighbours' rays come first: ours are merged after them
+    leaf_merge(o, ho, ro, v, have, restart);
+    for (int k = 0; k < 12; ++k) v[k] = o[k];
+    have = ho;
+    restart = ro;
+  } else {
+    leaf_merge(v, have, restart, o, ho, ro);
+  }
+}
+
+// Boxes of the leaves of block (K, J): `store(leaf, box, have)` is called by one lane for each.
+// A leaf's rays are merged in the reference's read order (row by row, left to right).  A leaf of
+// g.g rays is shared by the largest power of two of at most 64 lanes that it fills: each lane
+// merges g.g / lanes consecutive rays, four loads in flight, then groups of lanes merge at
+// distances 1, 2, 4, ... with the lower group first, which equals the sequential read.
+// One lane a leaf, as leaves of other sizes than powers of two up to 64 had it, left a 100 x 4
+// leaf's 400 rays to one lane: 400 x 300 image, 86 us (primary) and 149 us (with validity), now
+// 11 and 12.  The build of 4 x 4 leaves over 1024 x 1024 rays went from 28 to 24 us with the DPP
+// merges; it waits for its loads (the rays once, 33.6 MB: 7 us at the rate of a large copy).
+// ONE: every lane has at most one ray (leaves of a power of two of at most 64 rays).
+template <bool USE_VALID, bool UV, bool ONE, class F>
+__device__ __forceinline__ void build_leaves(const RHGeom& g, const RaysDev& r, int K, int J,
+                                             F store) {
+  const int tid = threadIdx.x;
+  const int lanes = 1 << (31 - __clz(min(g.g, 64)));  // uniform
+  const int each = (g.g + lanes - 1) / lanes;
+  const int nleaf = g.nlx * g.nlx, top = g.L - 1;
+  const int lane = tid & (lanes - 1), group = tid / lanes, groups = kThreads / lanes;
+  for (int base = 0; base < nleaf; base += groups) {
+    const int li = base + group;
+    const int x0 = K * g.bw + (li & (g.nlx - 1)) * g.cx, y0 = J * g.bh + (li >> top) * g.cy;
+    float v[12];
+    bool have = false, restart = false;
+    const int q0 = lane * each, qn = li < nleaf ? min(each, g.g - q0) : 0;
+    int dy = q0 / g.cx, dx = q0 - dy * g.cx;
+    V3 o[4], d[4];
+    bool h[4];
+    auto load = [&](int n, int k) {  // the lane's ray n
+      const int x = x0 + dx, y = y0 + dy;
+      h[k] = n < qn && x < g.W && y < g.H;
+      if (h[k]) {
+        const size_t i = (size_t)y * g.W + x;
+        if (USE_VALID && r.valid != nullptr) h[k] = glb(r.valid)[i] != 0;
+        d[k] = {glb(r.dx)[i], glb(r.dy)[i], glb(r.dz)[i]};
+        o[k] = {glb(r.ox)[i], glb(r.oy)[i], glb(r.oz)[i]};
+      }
+      if (++dx == g.cx) {
+        dx = 0;
+        ++dy;
+      }
+    };
+    auto merge = [&](int k) {
+      if (!h[k]) return;
       float b[12];
       bool rb;
-      ray_box<USE_VALID, UV>(r, i, b, rb);
+      ray_box<USE_VALID, UV>(o[k], d[k], b, rb);
       leaf_merge(v, have, restart, b, true, rb);
+    };
+    if constexpr (ONE) {
+      load(0, 0);
+      merge(0);
+    } else {
+      for (int n = 0; n < each; n += 4) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) load(n + k, k);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) merge(k);
+      }
     }
-  if (!have)
-    for (int k = 0; k < 12; ++k) v[k] = 0.f;
-  return have;
+    if (!have)
+      for (int k = 0; k < 12; ++k) v[k] = 0.f;
+    constexpr bool R = USE_VALID && UV;
+    merge_groups<1, R>(v, have, restart, lanes, tid);
+    merge_groups<2, R>(v, have, restart, lanes, tid);
+    merge_groups<4, R>(v, have, restart, lanes, tid);
+    merge_groups<8, R>(v, have, restart, lanes, tid);
+    merge_groups<16, R>(v, have, restart, lanes, tid);
+    merge_groups<32, R>(v, have, restart, lanes, tid);
+    if (lane == 0 && li < nleaf) store(li, v, have);
+  }
 }
 
 // ---------------------------------------------------------------------------------------
 // Fused hierarchy build: one work-group builds the leaves and every level of one block
 // (rayhconstruct6DB.cl / rayhconstructP6DB.cl / rayhconstruct(P)5DB.cl + levelConstruct6DB.cl /
 // levelConstructP6DB.cl / levelConstruct(P)5DB.cl folded into one launch instead of
-// 1 + (height-1) launches with host waits, rayhierarchy.cpp:375-549).  A leaf's rays are
-// merged in the reference's read order (row by row, left to right): lane pairs at distance
-// 1, 2, 4, ... combine the lower lane's part first, so every lane ends with the in-order
-// merge.
-template <bool USE_VALID, bool UV>
+// 1 + (height-1) launches with host waits, rayhierarchy.cpp:375-549).
+template <bool USE_VALID, bool UV, bool ONE>
 __device__ void build_block(const RHGeom& g, const RaysDev& r, float4* __restrict__ nodes, int b,
                             float (*sBox)[12], int* sVal) {
   const int tid = threadIdx.x;
@@ -213,53 +292,13 @@ __device__ void build_block(const RHGeom& g, const RaysDev& r, float4* __restric
   const int nleaf = g.nlx * g.nlx;
   const int leaf_off = g.nsub - nleaf;
 
-  const bool pow2 = g.g <= 64 && (g.g & (g.g - 1)) == 0;
-  if (pow2) {
-    for (int base = 0; base < g.rb; base += kThreads) {
-      int rl = base + tid;
-      int x = 0, y = 0, leaf = 0;
-      float v[12];
-      bool have = false, restart = false;
-      bool in_block = rl < g.rb;
-      if (slot_xy(g, K, J, rl, x, y, leaf)) {
-        size_t i = (size_t)y * g.W + x;
-        have = !USE_VALID || r.valid == nullptr || r.valid[i] != 0;
-        if (have) ray_box<USE_VALID, UV>(r, i, v, restart);
-      }
-      if (!have)
-        for (int k = 0; k < 12; ++k) v[k] = 0.f;
-      for (int m = 1; m < g.g; m <<= 1) {
-        float o[12];
-        for (int k = 0; k < 12; ++k) o[k] = __shfl_xor(v[k], m);
-        bool ho = __shfl_xor((int)have, m) != 0;
-        bool ro = __shfl_xor((int)restart, m) != 0;
-        if (tid & m) {  // the partner's rays come first: ours are merged after them
-          leaf_merge(o, ho, ro, v, have, restart);
-          for (int k = 0; k < 12; ++k) v[k] = o[k];
-          have = ho;
-          restart = ro;
-        } else {
-          leaf_merge(v, have, restart, o, ho, ro);
-        }
-      }
-      if (in_block && (rl % g.g) == 0) {
-        int li = rl / g.g;
-        for (int k = 0; k < 12; ++k) sBox[leaf_off + li][k] = v[k];
-        sVal[leaf_off + li] = have ? 1 : 0;
-      }
-    }
-  } else {
-    for (int li = tid; li < nleaf; li += kThreads) {
-      float v[12];
-      const bool have = leaf_box<USE_VALID, UV>(g, r, K * g.bw + (li % g.nlx) * g.cx,
-                                                J * g.bh + (li / g.nlx) * g.cy, v);
-      for (int k = 0; k < 12; ++k) sBox[leaf_off + li][k] = v[k];
-      sVal[leaf_off + li] = have ? 1 : 0;
-    }
-  }
+  build_leaves<USE_VALID, UV, ONE>(g, r, K, J, [&](int li, const float* v, bool have) {
+    for (int k = 0; k < 12; ++k) sBox[leaf_off + li][k] = v[k];
+    sVal[leaf_off + li] = have ? 1 : 0;
+  });
   __syncthreads();
   for (int li = tid; li < nleaf; li += kThreads) {
-    int gk = K * g.nlx + li % g.nlx, gj = J * g.nlx + li / g.nlx;
+    int gk = K * g.nlx + (li & (g.nlx - 1)), gj = J * g.nlx + (li >> top);
     if (gk < g.gw[0] && gj < g.gh[0])
       node_store(nodes, (size_t)g.off[0] + (size_t)gj * g.gw[0] + gk, sBox[leaf_off + li],
                  sVal[leaf_off + li] != 0);
@@ -268,7 +307,7 @@ __device__ void build_block(const RHGeom& g, const RaysDev& r, float4* __restric
     const int s = top - l, nl = 1 << s, cnl = nl * 2;
     const int soff = pow4_off(s), coff = pow4_off(s + 1);
     for (int i = tid; i < nl * nl; i += kThreads) {
-      int dk = i % nl, dj = i / nl;
+      int dk = i & (nl - 1), dj = i >> s;
       float v[12];
       bool have = false;
       for (int a = 0; a < 4; ++a) {
@@ -342,24 +381,22 @@ __device__ __forceinline__ int find_ray_item(const RhItem* __restrict__ items, i
 // go straight to the node array, and each level reads its four children back from it (the
 // work-group's own writes, ordered by the barrier between levels).  Children outside a level's
 // grid are skipped, as build_block skips the invalid ones; the merge order is the same.
-template <bool USE_VALID, bool UV>
+template <bool USE_VALID, bool UV, bool ONE>
 __device__ void build_block_deep(const RHGeom& g, const RaysDev& r, float4* __restrict__ nodes,
                                  int b) {
   const int tid = threadIdx.x;
   const int top = g.L - 1;
   const int K = b % g.gw[top], J = b / g.gw[top];
-  for (int li = tid; li < g.nlx * g.nlx; li += kThreads) {
-    const int gk = K * g.nlx + li % g.nlx, gj = J * g.nlx + li / g.nlx;
-    if (gk >= g.gw[0] || gj >= g.gh[0]) continue;
-    float v[12];
-    const bool have = leaf_box<USE_VALID, UV>(g, r, gk * g.cx, gj * g.cy, v);
-    node_store(nodes, (size_t)g.off[0] + (size_t)gj * g.gw[0] + gk, v, have);
-  }
+  build_leaves<USE_VALID, UV, ONE>(g, r, K, J, [&](int li, const float* v, bool have) {
+    const int gk = K * g.nlx + (li & (g.nlx - 1)), gj = J * g.nlx + (li >> top);
+    if (gk < g.gw[0] && gj < g.gh[0])
+      node_store(nodes, (size_t)g.off[0] + (size_t)gj * g.gw[0] + gk, v, have);
+  });
   __syncthreads();
   for (int l = 1; l < g.L; ++l) {
     const int nl = g.nlx >> l;
     for (int i = tid; i < nl * nl; i += kThreads) {
-      const int gk = K * nl + i % nl, gj = J * nl + i / nl;
+      const int gk = K * nl + (i & (nl - 1)), gj = J * nl + (i >> (top - l));
       if (gk >= g.gw[l] || gj >= g.gh[l]) continue;
       float v[12];
       bool have = false;
@@ -390,7 +427,7 @@ __device__ __forceinline__ void clear_counters(uint32_t* __restrict__ ctr, uint3
 }
 
 // ctr: the counters to clear for the kernels that follow (null: the init kernel does it).
-template <bool USE_VALID, bool UV>
+template <bool USE_VALID, bool UV, bool ONE>
 __global__ __launch_bounds__(256) void rh_group_build_kernel(const RhItem* __restrict__ items,
                                                              int nitems,
                                                              uint32_t* __restrict__ ctr) {
@@ -400,9 +437,9 @@ __global__ __launch_bounds__(256) void rh_group_build_kernel(const RhItem* __res
   const int k = find_block_item(items, nitems, blockIdx.x);
   const RhItem& it = items[k];
   if (it.g.L > kUnitLevels)
-    build_block_deep<USE_VALID, UV>(it.g, it.r, it.nodes, (int)(blockIdx.x - it.block_base));
+    build_block_deep<USE_VALID, UV, ONE>(it.g, it.r, it.nodes, (int)(blockIdx.x - it.block_base));
   else
-    build_block<USE_VALID, UV>(it.g, it.r, it.nodes, (int)(blockIdx.x - it.block_base), sBox,
+    build_block<USE_VALID, UV, ONE>(it.g, it.r, it.nodes, (int)(blockIdx.x - it.block_base), sBox,
                                sVal);
 }
 
@@ -2655,8 +2692,12 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
   if (!direct)
     hipLaunchKernelGGL((rh_init_kernel<MODE>), grid1(std::max<uint32_t>(G.nrays, kClaimQueues)),
                        dim3(kThreads), 0, s, G.items, G.nitems, G.nrays, G.ctr);
-  hipLaunchKernelGGL((rh_group_build_kernel<MODE != 0, NODE == 2>), dim3(G.nblocks),
-                     dim3(kThreads), 0, s, G.items, G.nitems, direct ? G.ctr : nullptr);
+  if (G.one_ray)
+    hipLaunchKernelGGL((rh_group_build_kernel<MODE != 0, NODE == 2, true>), dim3(G.nblocks),
+                       dim3(kThreads), 0, s, G.items, G.nitems, direct ? G.ctr : nullptr);
+  else
+    hipLaunchKernelGGL((rh_group_build_kernel<MODE != 0, NODE == 2, false>), dim3(G.nblocks),
+                       dim3(kThreads), 0, s, G.items, G.nitems, direct ? G.ctr : nullptr);
   if (direct) {
   } else if (G.bvh)
     hipLaunchKernelGGL((rh_cluster_kernel<MODE, NODE, true>), dim3(G.nblocks), dim3(kThreads), 0,
