@@ -417,9 +417,12 @@ int fill_item(const RhJob& jb, RhItem& it) {
 
 // Lays out the jobs as launch groups (one per mode and node type, in job order) in the
 // workspace arena, fills the job tables and uploads them when they changed.  `changed` tells
-// whether the device tables or arena were rewritten.
+// whether the device tables or arena were rewritten.  `single`: for one job whose blocks are all
+// traced per-ray, the table entry is left there for the launch (RhGroup::single) and nothing is
+// uploaded.
 int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& prm,
-               hipStream_t st, std::vector<RhGroup>& groups, bool* changed) {
+               hipStream_t st, std::vector<RhGroup>& groups, bool* changed,
+               RhItem* single = nullptr) {
   groups.clear();
   *changed = false;
   // group membership in job order
@@ -582,6 +585,13 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
     G.grid = gl[gi].grid;
     G.max_units = (uint32_t)std::min<size_t>(gl[gi].max_units, 0xffffffffu);
     groups.push_back(G);
+  }
+  if (single && table.size() == 1 && gl[0].ray == 0) {
+    *single = table[0];
+    groups[0].single = single;
+    ws.last_arena = nullptr;  // the launch overwrites the entry that the arena holds
+    *changed = true;
+    return RT_OK;
   }
   const bool same = ws.last_arena == A && ws.last.size() == table.size() &&
                     (table.empty() ||
@@ -948,7 +958,8 @@ static int trace_impl(rt_scene* s, const rt_rays* rays, int mode, const rt_hits*
     prm.walk[1] = s->walk_occluded;
     prm.tile[0] = s->tile_closest;
     prm.tile[1] = s->tile_occluded;
-    st = rh_prepare(s->ws[mode], jobs, prm, hs, groups, &changed);
+    RhItem single;
+    st = rh_prepare(s->ws[mode], jobs, prm, hs, groups, &changed, &single);
     if (st) return st;
     Timer::Slot* t = s->timer.next(mode, true);
     RT_TRY(launch_rh_group(groups[0], hs, t ? t->a : nullptr, t ? t->m : nullptr,
@@ -1066,7 +1077,7 @@ int rt_trace_closest_noalloc(rt_scene* s, const rt_rays* rays, int32_t mode, con
   G.ray_clusters = 0;
   G.ray_grid = 0;
   G.walk = kDefaultWalk;
-  RT_TRY(launch_write_table(it, table, hs));
+  G.single = &it;
   RT_TRY(launch_rh_group(G, hs, nullptr, nullptr, nullptr));
   return RT_OK;
 }

@@ -130,6 +130,9 @@ struct RhItem {
 // repair list are shared by the group's jobs.
 struct RhGroup {
   const RhItem* items;
+  // one job, every block per-ray: its table entry (host memory), which the build kernel takes as
+  // an argument and writes to items; null: items is on the device already
+  const RhItem* single;
   int nitems;
   int mode;  // 0 closest primary, 1 closest secondary, 2 occluded
   int node;  // 0 box_dir, 1 ia
@@ -197,8 +200,6 @@ int noalloc_setup(int device);
 void* noalloc_scratch(int device);
 // Writes the tleaf entry of every triangle into its record in search order (RhItem::tmts).
 hipError_t launch_set_tleaf(float4* tmts, const uint32_t* tleaf, uint32_t ntri, hipStream_t s);
-// Writes a job table into device memory through the kernel arguments (no copy, no allocation).
-hipError_t launch_write_table(const RhItem& item, RhItem* dst, hipStream_t s);
 
 // Launchers (all asynchronous on `s`).
 hipError_t launch_fill_u64(uint64_t* p, uint64_t v, size_t n, hipStream_t s);

@@ -428,19 +428,35 @@ __device__ __forceinline__ void clear_counters(uint32_t* __restrict__ ctr, uint3
 
 // ctr: the counters to clear for the kernels that follow (null: the init kernel does it).
 template <bool USE_VALID, bool UV, bool ONE>
-__global__ __launch_bounds__(256) void rh_group_build_kernel(const RhItem* __restrict__ items,
-                                                             int nitems,
-                                                             uint32_t* __restrict__ ctr) {
+__device__ __forceinline__ void group_build(const RhItem& it, uint32_t* __restrict__ ctr) {
   __shared__ float sBox[kMaxSub][12];
   __shared__ int sVal[kMaxSub];
   if (ctr != nullptr && blockIdx.x == 0) clear_counters(ctr, threadIdx.x);
-  const int k = find_block_item(items, nitems, blockIdx.x);
-  const RhItem& it = items[k];
+  const int b = (int)(blockIdx.x - it.block_base);
   if (it.g.L > kUnitLevels)
-    build_block_deep<USE_VALID, UV, ONE>(it.g, it.r, it.nodes, (int)(blockIdx.x - it.block_base));
+    build_block_deep<USE_VALID, UV, ONE>(it.g, it.r, it.nodes, b);
   else
-    build_block<USE_VALID, UV, ONE>(it.g, it.r, it.nodes, (int)(blockIdx.x - it.block_base), sBox,
-                               sVal);
+    build_block<USE_VALID, UV, ONE>(it.g, it.r, it.nodes, b, sBox, sVal);
+}
+template <bool USE_VALID, bool UV, bool ONE>
+__global__ __launch_bounds__(256) void rh_group_build_kernel(const RhItem* __restrict__ items,
+                                                             int nitems,
+                                                             uint32_t* __restrict__ ctr) {
+  group_build<USE_VALID, UV, ONE>(items[find_block_item(items, nitems, blockIdx.x)], ctr);
+}
+// The same for a single job whose table entry comes with the launch; the first work-group leaves
+// it in `table` for the kernels that follow.  A renderer whose buffers change from call to call
+// thus uploads nothing: the copy (3.5 us), its event and the wait for the one before are gone.
+template <bool USE_VALID, bool UV, bool ONE>
+__global__ __launch_bounds__(256) void rh_single_build_kernel(const RhItem it,
+                                                              RhItem* __restrict__ table,
+                                                              uint32_t* __restrict__ ctr) {
+  if (blockIdx.x == 0) {
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(&it);
+    for (uint32_t i = threadIdx.x; i < sizeof(RhItem) / 4; i += kThreads)
+      reinterpret_cast<uint32_t*>(table)[i] = src[i];
+  }
+  group_build<USE_VALID, UV, ONE>(it, ctr);
 }
 
 // Clears the reduction state of every job: keys, repair keys, occlusion flags, counters.
@@ -2692,12 +2708,20 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
   if (!direct)
     hipLaunchKernelGGL((rh_init_kernel<MODE>), grid1(std::max<uint32_t>(G.nrays, kClaimQueues)),
                        dim3(kThreads), 0, s, G.items, G.nitems, G.nrays, G.ctr);
+  uint32_t* const clear = direct ? G.ctr : nullptr;
+  auto build = [&](auto group, auto single) {
+    if (G.single)
+      hipLaunchKernelGGL(single, dim3(G.nblocks), dim3(kThreads), 0, s, *G.single,
+                         const_cast<RhItem*>(G.items), clear);
+    else
+      hipLaunchKernelGGL(group, dim3(G.nblocks), dim3(kThreads), 0, s, G.items, G.nitems, clear);
+  };
   if (G.one_ray)
-    hipLaunchKernelGGL((rh_group_build_kernel<MODE != 0, NODE == 2, true>), dim3(G.nblocks),
-                       dim3(kThreads), 0, s, G.items, G.nitems, direct ? G.ctr : nullptr);
+    build(rh_group_build_kernel<MODE != 0, NODE == 2, true>,
+          rh_single_build_kernel<MODE != 0, NODE == 2, true>);
   else
-    hipLaunchKernelGGL((rh_group_build_kernel<MODE != 0, NODE == 2, false>), dim3(G.nblocks),
-                       dim3(kThreads), 0, s, G.items, G.nitems, direct ? G.ctr : nullptr);
+    build(rh_group_build_kernel<MODE != 0, NODE == 2, false>,
+          rh_single_build_kernel<MODE != 0, NODE == 2, false>);
   if (direct) {
   } else if (G.bvh)
     hipLaunchKernelGGL((rh_cluster_kernel<MODE, NODE, true>), dim3(G.nblocks), dim3(kThreads), 0,
@@ -2788,14 +2812,6 @@ __global__ __launch_bounds__(256) void set_tleaf_kernel(float4* __restrict__ tmt
   r.z = __uint_as_float(tleaf[__float_as_uint(r.y)]);
 }
 
-// Copies a job table passed by value (in the kernel arguments) into device memory, so that a
-// launch group can be set up without a host-to-device copy.
-__global__ __launch_bounds__(64) void write_table_kernel(RhItem item, RhItem* __restrict__ dst) {
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(&item);
-  uint32_t* out = reinterpret_cast<uint32_t*>(dst);
-  for (uint32_t i = threadIdx.x; i < sizeof(RhItem) / 4; i += 64) out[i] = src[i];
-}
-
 // Scratch of the allocation-free trace (rt_trace_closest_noalloc): one array per device, held
 // until the process ends.  Its device address is looked up in this file, once per device.
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratch];
@@ -2827,11 +2843,6 @@ void* noalloc_scratch(int device) {
 hipError_t launch_set_tleaf(float4* tmts, const uint32_t* tleaf, uint32_t ntri, hipStream_t s) {
   if (!ntri) return hipSuccess;
   hipLaunchKernelGGL(set_tleaf_kernel, grid1(ntri), dim3(kThreads), 0, s, tmts, tleaf, ntri);
-  return hipGetLastError();
-}
-
-hipError_t launch_write_table(const RhItem& item, RhItem* dst, hipStream_t s) {
-  hipLaunchKernelGGL(write_table_kernel, dim3(1), dim3(64), 0, s, item, dst);
   return hipGetLastError();
 }
 
