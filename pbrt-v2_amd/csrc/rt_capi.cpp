@@ -156,9 +156,6 @@ struct rt_scene {
   uint32_t nroots = 0;
   int roots_per_unit = 0;  // root clusters per ray-bvh unit; 0 = built-in choice
   bool has_bvh = false;
-  // scratch of the naive path, grown on demand
-  uint64_t* d_keys = nullptr;
-  size_t keys_cap = 0;
   // scratch of the rayhierarchy and ray-bvh paths (a launch group of one job), one per trace
   // mode, so that a renderer alternating camera, shadow and bounce calls on the same buffers
   // finds its job table already on the device
@@ -212,25 +209,6 @@ int hip_status(hipError_t e) {
     if (_e != hipSuccess) return hip_status(_e); \
   } while (0)
 
-template <class T>
-int grow(T*& p, size_t& cap, size_t need) {
-  if (need <= cap && p) return RT_OK;
-  if (p) {
-    hipError_t e = hipFree(p);
-    p = nullptr;
-    cap = 0;
-    if (e != hipSuccess) return hip_status(e);
-  }
-  size_t n = std::max<size_t>(need, 1);
-  hipError_t e = hipMalloc((void**)&p, n * sizeof(T));
-  if (e != hipSuccess) {
-    p = nullptr;
-    return hip_status(e);
-  }
-  cap = n;
-  return RT_OK;
-}
-
 int check_rays(const rt_rays* r, bool need_valid_ok) {
   (void)need_valid_ok;
   if (!r || !r->ox || !r->oy || !r->oz || !r->dx || !r->dy || !r->dz || !r->tmin || !r->tmax)
@@ -243,13 +221,6 @@ int check_rays(const rt_rays* r, bool need_valid_ok) {
 RaysDev to_dev(const rt_rays* r) {
   return RaysDev{r->ox, r->oy, r->oz, r->dx, r->dy, r->dz, r->tmin, r->tmax, r->valid,
                  r->width, r->height};
-}
-
-// Triangle chunks per block so that a launch has >= ~1024 work-groups (4 per CU).
-int pick_tchunks(int nblocks, uint32_t nwork, uint32_t per_tile) {
-  int want = (2048 + nblocks - 1) / std::max(nblocks, 1);  // ~8 work-groups per CU
-  int maxc = (int)std::max<uint32_t>(1, nwork / std::max<uint32_t>(per_tile, 1));
-  return std::max(1, std::min(want, maxc));
 }
 
 int desc_ok(const rt_accel_desc* d) {
@@ -924,7 +895,6 @@ int rt_scene_destroy(rt_scene* s) {
   (void)hipFree(s->d_bvh_parent);
   (void)hipFree(s->d_bvh_depth);
   (void)hipFree(s->d_rcbox);
-  (void)hipFree(s->d_keys);
   delete s;
   return RT_OK;
 }
@@ -936,7 +906,6 @@ static int trace_impl(rt_scene* s, const rt_rays* rays, int mode, const rt_hits*
   std::lock_guard<std::mutex> lk(s->mu);
   RT_TRY(hipSetDevice(s->ctx->device));
   hipStream_t hs = (hipStream_t)stream;
-  const size_t n = (size_t)rays->width * rays->height;
   const RaysDev r = to_dev(rays);
   const bool closest = mode != 2;
   const HitOut out = closest ? HitOut{hits->id, hits->t, hits->u, hits->v, hits->dpdu, hits->dpdv}
@@ -966,27 +935,12 @@ static int trace_impl(rt_scene* s, const rt_rays* rays, int mode, const rt_hits*
                            t ? t->b : nullptr));
     return RT_OK;
   }
-  if (closest) {
-    st = grow(s->d_keys, s->keys_cap, n);
-    if (st) return st;
-  }
-  if (ntri == 0) {
-    // empty scene: everything misses
-    if (closest) RT_TRY(launch_fill_u64(s->d_keys, ~0ull, n, hs));
-    else RT_TRY(launch_fill_u8(occ, 0, n, hs));
-  } else if (kind == RT_ACCEL_NAIVE) {
-    const int nblk = (int)((n + 255) / 256);
-    const int tchunks = pick_tchunks(nblk, ntri, 64);
-    if (tchunks > 1) {
-      if (closest) RT_TRY(launch_fill_u64(s->d_keys, ~0ull, n, hs));
-      else RT_TRY(launch_fill_u8(occ, 0, n, hs));
-    }
-    RT_TRY(timed_launch(s->timer, mode, hs, [&] {
-      return launch_naive_trace(r, mode, s->d_v9, ntri, tchunks, s->d_keys, occ, hs);
-    }));
-  }
-  if (closest)
-    RT_TRY(launch_finalize(r, s->d_v9, s->d_uv6, s->d_keys, out, kind == RT_ACCEL_NAIVE, hs));
+  // naive brute force, or an empty scene, where every ray misses
+  const auto launch = [&] {
+    return launch_naive_trace(r, mode, s->d_v9, s->d_uv6, ntri, kind == RT_ACCEL_NAIVE, out, occ,
+                              hs);
+  };
+  RT_TRY(ntri > 0 ? timed_launch(s->timer, mode, hs, launch) : launch());
   return RT_OK;
 }
 
@@ -1017,16 +971,10 @@ int rt_trace_closest_noalloc(rt_scene* s, const rt_rays* rays, int32_t mode, con
   const HitOut out{hits->id, hits->t, hits->u, hits->v, hits->dpdu, hits->dpdv};
   const int kind = s->desc.kind;
   if (kind == RT_ACCEL_NAIVE || s->ntri == 0) {
-    // naive brute force (or an empty scene): the reduction keys are the only scratch
+    // naive brute force (or an empty scene) needs no scratch; the bound is the call's own
     if (align256(sizeof(uint64_t) * n) > kNoAllocScratch) return RT_ERR_TOO_LARGE;
-    uint64_t* keys = (uint64_t*)base;
-    RT_TRY(launch_fill_u64(keys, ~0ull, n, hs));
-    if (s->ntri > 0) {
-      const int nblk = (int)((n + 255) / 256);
-      const int tchunks = pick_tchunks(nblk, s->ntri, 64);
-      RT_TRY(launch_naive_trace(r, mode, s->d_v9, s->ntri, tchunks, keys, nullptr, hs));
-    }
-    RT_TRY(launch_finalize(r, s->d_v9, s->d_uv6, keys, out, kind == RT_ACCEL_NAIVE, hs));
+    RT_TRY(launch_naive_trace(r, mode, s->d_v9, s->d_uv6, s->ntri, kind == RT_ACCEL_NAIVE, out,
+                              nullptr, hs));
     return RT_OK;
   }
   // rayhierarchy / ray-bvh: one job whose blocks all take the per-ray path (the same result as

@@ -86,34 +86,27 @@ __device__ __forceinline__ bool repair_region(float b1, float b2) {
   return !(b1 < kEps || b1 > kRepHi1) && !(b2 < kEps || (b1 + b2) > kRepHi2);
 }
 
-// naive.cl:30-46 (TriRay closest).
-__device__ __forceinline__ bool mt_naive(V3 o, V3 d, const Tri& T, float& t, float& b1, float& b2) {
-  V3 s1 = cross(d, T.e2);
-  float div = dot(s1, T.e1);
-  if (div < kEps && div > -kEps) return false;
-  float inv = 1.0f / div;
-  V3 dd = sub(o, T.v1);
-  b1 = dot(dd, s1) * inv;
-  if (b1 < kNaiveLo || b1 > kNaiveHi) return false;
-  V3 s2 = cross(dd, T.e1);
-  b2 = dot(d, s2) * inv;
-  if (b2 < kNaiveLo || (b1 + b2) > kNaiveHi) return false;
-  t = dot(T.e2, s2) * inv;
-  return true;
+// Half the width of the leaf test's interval of b1, which lies around 1/2, with a margin for the
+// roundings of b1 = fl(n1 * fl(1 / div)) (2^-22 of it at most).
+template <bool P>
+constexpr float naive_half() {
+  return (0.5f - (P ? kNaivePLo : kNaiveLo)) * (1.0f + 0x1p-18f);
 }
-
-// naive.cl:211-227 (IntersectionP).
-__device__ __forceinline__ bool mt_naive_p(V3 o, V3 d, const Tri& T, float& t) {
-  V3 s1 = cross(d, T.e2);
-  float div = dot(s1, T.e1);
-  if (div == 0.0f) return false;
-  float inv = 1.0f / div;
-  V3 dd = sub(o, T.v1);
-  float b1 = dot(dd, s1) * inv;
-  if (b1 < kNaivePLo || b1 > kNaivePHi) return false;
-  V3 s2 = cross(dd, T.e1);
-  float b2 = dot(d, s2) * inv;
-  if (b2 < kNaivePLo || (b1 + b2) > kNaivePHi) return false;
+// Leaf test of the naive kernels: naive.cl:30-46 (TriRay closest) and, with P, naive.cl:211-227
+// (IntersectionP).
+template <bool P>
+__device__ __forceinline__ bool mt_naive(V3 o, V3 d, const Tri& T, float& t) {
+  constexpr float lo = P ? kNaivePLo : kNaiveLo, hi = P ? kNaivePHi : kNaiveHi;
+  const V3 s1 = cross(d, T.e2);
+  const float div = dot(s1, T.e1);
+  if (P ? div == 0.0f : (div < kEps && div > -kEps)) return false;
+  const float inv = 1.0f / div;
+  const V3 dd = sub(o, T.v1);
+  const float b1 = dot(dd, s1) * inv;
+  if (b1 < lo || b1 > hi) return false;
+  const V3 s2 = cross(dd, T.e1);
+  const float b2 = dot(d, s2) * inv;
+  if (b2 < lo || (b1 + b2) > hi) return false;
   t = dot(T.e2, s2) * inv;
   return true;
 }

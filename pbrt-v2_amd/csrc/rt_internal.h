@@ -202,7 +202,6 @@ void* noalloc_scratch(int device);
 hipError_t launch_set_tleaf(float4* tmts, const uint32_t* tleaf, uint32_t ntri, hipStream_t s);
 
 // Launchers (all asynchronous on `s`).
-hipError_t launch_fill_u64(uint64_t* p, uint64_t v, size_t n, hipStream_t s);
 hipError_t launch_fill_u8(uint8_t* p, uint8_t v, size_t n, hipStream_t s);
 // rayhierarchy / ray-bvh group: init, fused build, cluster (root) pass, persistent unit
 // kernel, per-ray kernel and, for closest hits, finalize and (rayhierarchy) repair.  When
@@ -210,11 +209,11 @@ hipError_t launch_fill_u8(uint8_t* p, uint8_t v, size_t n, hipStream_t s);
 // t1 after the per-ray kernel.
 hipError_t launch_rh_group(const RhGroup& G, hipStream_t s, hipEvent_t t0, hipEvent_t tm,
                            hipEvent_t t1);
-hipError_t launch_naive_trace(const RaysDev& r, int mode, const float* v9, uint32_t ntri,
-                              int tchunks, uint64_t* keys, uint8_t* occ, hipStream_t s);
-// Hit records of the naive path from the reduction keys.
-hipError_t launch_finalize(const RaysDev& r, const float* v9, const float* uv6,
-                           const uint64_t* keys, HitOut out, bool naive_rule, hipStream_t s);
+// Naive brute force from rays to hit records (mode 0, 1) or occlusion flags (mode 2); without
+// triangles every ray misses.  naive_rule: shading frames as the naive kernels take them.
+hipError_t launch_naive_trace(const RaysDev& r, int mode, const float* v9, const float* uv6,
+                              uint32_t ntri, bool naive_rule, HitOut out, uint8_t* occ,
+                              hipStream_t s);
 hipError_t launch_camera_rays(int W, int H, int spp, const float origin[3], float tan_half,
                               float aspect, uint32_t seed, float* ox, float* oy, float* oz,
                               float* dx, float* dy, float* dz, float* tmin, float* tmax,

@@ -2317,70 +2317,6 @@ __device__ __forceinline__ Tri staged_tri(const float4 (*sT)[3], int slot) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Naive brute force (naive.cl "TriRay" semantics, ray-parallel): every ray of the block tests
-// every triangle of its chunk, triangles staged through LDS.
-template <int MODE>
-__global__ __launch_bounds__(256) void naive_kernel(RaysDev r, const float* __restrict__ v9,
-                                                    uint32_t ntri, uint32_t chunk,
-                                                    uint64_t* __restrict__ keys,
-                                                    uint8_t* __restrict__ occ_out, int tchunks) {
-  __shared__ float4 sT[kThreads][3];
-  const int tid = threadIdx.x;
-  const size_t n = (size_t)r.W * r.H;
-  const size_t i = (size_t)blockIdx.x * kThreads + tid;
-  const bool exists = i < n;
-  const bool valid = exists && (MODE == 0 || r.valid == nullptr || r.valid[i] != 0);
-  V3 o{}, d{};
-  float tmin = 0.f, tmax = 0.f;
-  if (valid) {
-    o = {r.ox[i], r.oy[i], r.oz[i]};
-    d = {r.dx[i], r.dy[i], r.dz[i]};
-    tmin = r.tmin[i];
-    tmax = r.tmax[i];
-  }
-  uint64_t best = kMissKey;
-  bool occ = false;
-  const uint32_t t0 = blockIdx.y * chunk;
-  const uint32_t t1 = min(ntri, t0 + chunk);
-  for (uint32_t base = t0; base < t1; base += kThreads) {
-    const uint32_t ti = base + tid;
-    if (ti < t1) stage_tri(sT, tid, load_tri(v9, ti));
-    __syncthreads();
-    const int cnt = (int)min((uint32_t)kThreads, t1 - base);
-    if (valid && !(MODE == 2 && occ)) {
-      for (int k = 0; k < cnt; ++k) {
-        const Tri T = staged_tri(sT, k);
-        float t, b1, b2;
-        if (MODE == 2) {
-          if (!mt_naive_p(o, d, T, t)) continue;
-          if (t < tmin || t > tmax) continue;
-          occ = true;
-          break;
-        } else {
-          if (!mt_naive(o, d, T, t, b1, b2)) continue;
-          if (t < tmin) continue;
-          uint64_t kk = hit_key(t, (int32_t)(base + k));
-          if (kk < best) best = kk;
-        }
-      }
-    }
-    if (MODE == 2) {
-      if (__syncthreads_and(!valid || occ)) break;
-    } else {
-      __syncthreads();
-    }
-  }
-  if (!exists) return;
-  if (MODE == 2) {
-    if (tchunks == 1) occ_out[i] = occ ? 1 : 0;
-    else if (occ) occ_out[i] = 1;
-  } else {
-    if (tchunks == 1) keys[i] = best;
-    else if (best != kMissKey) atomicMin((unsigned long long*)&keys[i], (unsigned long long)best);
-  }
-}
-
-// ---------------------------------------------------------------------------------------
 // Hit record of one ray from its reduction key; returns t (INFINITY on a miss).
 __device__ __forceinline__ float finalize_ray(const RaysDev& r, const float* __restrict__ v9,
                                               const float* __restrict__ uv6, uint64_t key,
@@ -2395,15 +2331,158 @@ __device__ __forceinline__ float finalize_ray(const RaysDev& r, const float* __r
   return t;
 }
 
-// Hit records of the naive accelerator (and of an empty scene's misses).
-__global__ __launch_bounds__(256) void finalize_kernel(RaysDev r, const float* __restrict__ v9,
-                                                       const float* __restrict__ uv6,
-                                                       const uint64_t* __restrict__ keys,
-                                                       HitOut out, int naive_rule) {
+// ---------------------------------------------------------------------------------------
+// Naive brute force (naive.cl "TriRay" semantics, ray-parallel).
+constexpr int kNaiveThreads = 512;
+constexpr int kNaiveTris = 512;          // triangles staged at a time
+constexpr int kNaiveShift = 6;           // 1 << kNaiveShift lanes test one triangle
+constexpr int kNaiveRays = 2 << kNaiveShift;  // rays of a work-group: two to a lane
+
+// A triangle as the naive kernel stages it.  With m = o x d the leaf test's numerators and
+// determinant are linear in (d, m), so a ray is rejected by fused multiply-adds alone:
+//   div = d.(e2 x e1), n1 = m.e2 - d.(e2 x v1), n2 = d.(e1 x v1) - m.e1.
+// q[0] = e2 x e1 and the bound's factor (below), q[1] and q[2] = e2 and e2 x v1 + (e2 x e1) / 2,
+// then e1 and e1 x v1; q[4] = v1.
+struct NaiveTri {
+  float4 q[5];
+};
+// |.|1 is the sum of magnitudes, u = 2^-24.  The rounding errors of n1 - div / 2 and |div| / 2 as
+// the leaf test and as the filter compute them come to less than
+// 20 u |d|1 (|e1|1 + |e2|1) (|o|1 + |v1|1 + |e1|1 + |e2|1), those of n2, n1 + n2 likewise to less
+// than 28 u of it; the bound is 64 u.  Every norm counts as 2^-40 at least, which covers what
+// underflow takes away (2^-150 times one of the factors), and where a factor exceeds 2^40, so
+// that products could overflow, or is not a number, the bound is infinite: nothing is rejected.
+constexpr float kNormMin = 0x1p-40f, kNormMax = 0x1p40f, kNaiveErr = 0x1p-18f;
+__device__ __forceinline__ float norm1(V3 a) { return fabsf(a.x) + fabsf(a.y) + fabsf(a.z); }
+__device__ __forceinline__ float norm_bound(float x) {
+  return x <= kNormMax ? (x < kNormMin ? kNormMin : x) : __int_as_float(0x7f800000);
+}
+
+__device__ __forceinline__ void stage_naive(NaiveTri& s, const Tri& T, float omax) {
+  const V3 n = cross(T.e2, T.e1), c1 = cross(T.e2, T.v1), c2 = cross(T.e1, T.v1);
+  const float edges = norm1(T.e1) + norm1(T.e2), e = edges < kNormMin ? kNormMin : edges;
+  const float f = norm_bound(e * (omax + norm1(T.v1) + e)) * kNaiveErr;
+  s.q[0] = make_float4(n.x, n.y, n.z, f);
+  s.q[1] = make_float4(T.e2.x, T.e2.y, T.e2.z, c1.x + 0.5f * n.x);
+  s.q[2] = make_float4(c1.y + 0.5f * n.y, c1.z + 0.5f * n.z, T.e1.x, T.e1.y);
+  s.q[3] = make_float4(T.e1.z, c2.x, c2.y, c2.z);
+  s.q[4] = make_float4(T.v1.x, T.v1.y, T.v1.z, 0.f);
+}
+__device__ __forceinline__ float dot_fma(float x, float y, float z, V3 v, float c) {
+  return __builtin_fmaf(x, v.x, __builtin_fmaf(y, v.y, __builtin_fmaf(z, v.z, c)));
+}
+// First part of the filter: false if b1 is certainly outside the leaf test's interval.
+__device__ __forceinline__ bool naive_b1(const float4 (&q)[3], V3 d, V3 m, float dn, float half,
+                                         float& div, float& err, float& x) {
+  div = dot_fma(q[0].x, q[0].y, q[0].z, d, 0.f);
+  x = dot_fma(q[1].x, q[1].y, q[1].z, m, -dot_fma(q[1].w, q[2].x, q[2].y, d, 0.f));
+  err = dn * q[0].w;
+  return !(fabsf(x) > __builtin_fmaf(half, fabsf(div), err));
+}
+
+// A work-group has the whole answer of its rays, two to a lane (a triangle's LDS reads serve two
+// tests).  1 << shift lanes test one triangle; the parts of that many lanes share out the
+// triangles, staged through LDS.  So a call is one launch, without keys in memory to clear,
+// reduce by atomics and turn into hit records by launches of their own.
+// Bound by vector issue: the leaf test alone takes 26 instructions to its first reject, the
+// filter 12.  1,024 triangles, 128 x 128 rays: closest 24.5 -> 21 us and occlusion 27.6 -> 22 us
+// (without the launches saved), 4,096 triangles, 250 x 200 rays: 392 -> 266 us for both.
+template <int MODE>
+__global__ __launch_bounds__(kNaiveThreads) void naive_kernel(RaysDev r,
+                                                              const float* __restrict__ v9,
+                                                              const float* __restrict__ uv6,
+                                                              uint32_t ntri, int shift,
+                                                              HitOut out, bool naive_rule,
+                                                              uint8_t* __restrict__ occ_out) {
+  constexpr bool P = MODE == 2;
+  constexpr float half = naive_half<P>();
+  __shared__ NaiveTri sT[kNaiveTris];
+  __shared__ uint64_t sBest[kNaiveRays];  // closest: reduction key; occlusion: 0 when occluded
+  __shared__ uint32_t sFar;               // largest |o|1 of the work-group's rays
+  const int tid = threadIdx.x;
   const size_t n = (size_t)r.W * r.H;
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  finalize_ray(r, v9, uv6, keys[i], i, out, naive_rule != 0);
+  const int lanes = 1 << shift;
+  const int slot = tid & (lanes - 1);
+  const uint32_t part = (uint32_t)tid >> shift, parts = (uint32_t)kNaiveThreads >> shift;
+  const size_t first = (size_t)blockIdx.x * (2 * lanes);
+  if (tid < 2 * lanes) sBest[tid] = kMissKey;
+  if (tid == 0) sFar = __float_as_uint(kNormMin);
+  __syncthreads();
+  V3 o[2], d[2], m[2];
+  float tmin[2], tmax[2], dn[2];
+  uint64_t best[2] = {kMissKey, kMissKey};
+  bool live[2];
+  for (int j = 0; j < 2; ++j) {
+    const size_t i = first + slot + j * lanes;
+    live[j] = i < n && (MODE == 0 || r.valid == nullptr || r.valid[i] != 0);
+    o[j] = d[j] = {0.f, 0.f, 0.f};
+    tmin[j] = tmax[j] = 0.f;
+    if (live[j]) {
+      o[j] = {r.ox[i], r.oy[i], r.oz[i]};
+      d[j] = {r.dx[i], r.dy[i], r.dz[i]};
+      tmin[j] = r.tmin[i];
+      if (P) tmax[j] = r.tmax[i];
+      // magnitudes order as their bit patterns do, NaN above all
+      if (part == 0) atomicMax(&sFar, __float_as_uint(norm1(o[j])));
+    }
+    m[j] = cross(o[j], d[j]);
+    dn[j] = norm_bound(norm1(d[j]));
+  }
+  for (uint32_t base = 0; base < ntri; base += kNaiveTris) {
+    const uint32_t cnt = min(ntri - base, (uint32_t)kNaiveTris);
+    __syncthreads();
+    const float omax = __uint_as_float(sFar);
+    for (uint32_t k = tid; k < cnt; k += kNaiveThreads)
+      stage_naive(sT[k], load_tri(v9, base + k), omax);
+    __syncthreads();
+    if (part >= cnt) continue;
+    float4 q[3] = {sT[part].q[0], sT[part].q[1], sT[part].q[2]};
+    for (uint32_t k = part; k < cnt; k += parts) {
+      if (P && !__any(live[0] || live[1])) break;
+      const uint32_t kn = k + parts < cnt ? k + parts : k;
+      const float4 next[3] = {sT[kn].q[0], sT[kn].q[1], sT[kn].q[2]};
+      for (int j = 0; j < 2; ++j) {
+        float div, err, x;
+        if (!naive_b1(q, d[j], m[j], dn[j], half, div, err, x) || !live[j]) continue;
+        const float4 q3 = sT[k].q[3], q4 = sT[k].q[4];
+        Tri T;
+        T.v1 = T.v2 = T.v3 = {q4.x, q4.y, q4.z};
+        T.e1 = {q[2].z, q[2].w, q3.x};
+        T.e2 = {q[1].x, q[1].y, q[1].z};
+        // b2 and b1 + b2, from x = n1 - div / 2; a determinant within the bound may have the
+        // other sign or, without an inverse, make b1 NaN, after which no sum is rejected
+        const float n2 = dot_fma(q3.y, q3.z, q3.w, d[j], -dot_fma(T.e1.x, T.e1.y, T.e1.z, m[j], 0.f));
+        const float n12 = x + n2;
+        const bool neg = div < 0.f;
+        if (fabsf(div) > err &&
+            ((neg ? -n2 : n2) < -__builtin_fmaf(half - 0.5f, fabsf(div), err) ||
+             (neg ? -n12 : n12) > __builtin_fmaf(half, fabsf(div), err) + err))
+          continue;
+        float t;
+        if (!mt_naive<P>(o[j], d[j], T, t) || t < tmin[j]) continue;
+        if (P) {
+          if (t > tmax[j]) continue;
+          live[j] = false;
+          best[j] = 0;
+        } else {
+          const uint64_t key = hit_key(t, (int32_t)(base + k));
+          if (key < best[j]) best[j] = key;
+        }
+      }
+      for (int c = 0; c < 3; ++c) q[c] = next[c];
+    }
+  }
+  __syncthreads();
+  for (int j = 0; j < 2; ++j)
+    if (best[j] != kMissKey)
+      atomicMin((unsigned long long*)&sBest[slot + j * lanes], (unsigned long long)best[j]);
+  __syncthreads();
+  const size_t i = first + tid;
+  if (tid >= 2 * lanes || i >= n) return;
+  if (P)
+    occ_out[i] = sBest[tid] == 0 ? 1 : 0;
+  else
+    finalize_ray(r, v9, uv6, sBest[tid], i, out, naive_rule);
 }
 
 // Hit records of every job of a closest-hit group.  Rays whose nearest repair-region
@@ -2893,11 +2972,6 @@ int rh_geometry(int W, int H, int cx, int cy, int height, RHGeom* g) {
   return 0;
 }
 
-hipError_t launch_fill_u64(uint64_t* p, uint64_t v, size_t n, hipStream_t s) {
-  if (!n) return hipSuccess;
-  hipLaunchKernelGGL(fill_kernel<uint64_t>, grid1(n), dim3(kThreads), 0, s, p, v, n);
-  return hipGetLastError();
-}
 hipError_t launch_fill_u8(uint8_t* p, uint8_t v, size_t n, hipStream_t s) {
   if (!n) return hipSuccess;
   hipLaunchKernelGGL(fill_kernel<uint8_t>, grid1(n), dim3(kThreads), 0, s, p, v, n);
@@ -2924,25 +2998,23 @@ hipError_t launch_rh_group(const RhGroup& G, hipStream_t s, hipEvent_t t0, hipEv
 #undef RT_CALL
 }
 
-hipError_t launch_naive_trace(const RaysDev& r, int mode, const float* v9, uint32_t ntri,
-                              int tchunks, uint64_t* keys, uint8_t* occ, hipStream_t s) {
+hipError_t launch_naive_trace(const RaysDev& r, int mode, const float* v9, const float* uv6,
+                              uint32_t ntri, bool naive_rule, HitOut out, uint8_t* occ,
+                              hipStream_t s) {
   const size_t n = (size_t)r.W * r.H;
-  const uint32_t chunk = (uint32_t)((ntri + tchunks - 1) / tchunks);
-  dim3 grid((unsigned)((n + kThreads - 1) / kThreads), tchunks);
-  if (mode == 0)
-    hipLaunchKernelGGL(naive_kernel<0>, grid, dim3(kThreads), 0, s, r, v9, ntri, chunk, keys, occ, tchunks);
-  else if (mode == 1)
-    hipLaunchKernelGGL(naive_kernel<1>, grid, dim3(kThreads), 0, s, r, v9, ntri, chunk, keys, occ, tchunks);
-  else
-    hipLaunchKernelGGL(naive_kernel<2>, grid, dim3(kThreads), 0, s, r, v9, ntri, chunk, keys, occ, tchunks);
-  return hipGetLastError();
-}
-
-hipError_t launch_finalize(const RaysDev& r, const float* v9, const float* uv6,
-                           const uint64_t* keys, HitOut out, bool naive_rule, hipStream_t s) {
-  const size_t n = (size_t)r.W * r.H;
-  hipLaunchKernelGGL(finalize_kernel, grid1(n), dim3(kThreads), 0, s, r, v9, uv6, keys, out,
-                     naive_rule ? 1 : 0);
+  // Rays to a work-group: as many as leave 512 work-groups, two to a CU, and 8 at least.  With
+  // work-groups of 1,024 threads, one to a CU, 4,096 triangles and 250 x 200 rays take 352 us in
+  // place of 266 (128 x 128 rays: equal); with 128 rays always, 33 x 40 rays leave 245 CUs idle.
+  int shift = kNaiveShift;
+  while (shift > 2 && ((n - 1) >> (shift + 1)) + 1 < 512) --shift;
+  const dim3 grid((unsigned)(((n - 1) >> (shift + 1)) + 1));
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kNaiveThreads), 0, s, r, v9, uv6, ntri, shift, out,
+                       naive_rule, occ);
+  };
+  if (mode == 0) run(naive_kernel<0>);
+  else if (mode == 1) run(naive_kernel<1>);
+  else run(naive_kernel<2>);
   return hipGetLastError();
 }
 
