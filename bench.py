@@ -13,8 +13,8 @@ box_dir nodes, repairRun 1).  One step traces every scene's closest hits and occ
 All three must give the same bits; sampled ray blocks are checked against the oracle, with
 near ties, ulp-marginal rays and differences to the exact pbrt predicate counted.
 
-Also reported: the roofline of the dominant traversal kernel (algorithmic bytes from the
-oracle's restatement of its work, HIP-event time of the kernel), pbrt's CPU BVH on a bounded
+Also reported: the roofline of the dominant traversal kernel (the bytes a trace cannot do
+without, HIP-event time of the kernel, profiled traffic and VALU share), pbrt's CPU BVH on a bounded
 sample of the same rays, the plain rayhierarchy torus workload, and the serving form at
 Poisson request rates.
 """
@@ -107,36 +107,37 @@ def bound_of(facts, hbm_meas, hbm_alg, valu_frac):
     return "hbm" if hbm_alg >= valu_frac else "valu"
 
 
-def per_ray_roofline(name, t_ms, st, mode, workload):
-    """Roofline of a per-ray kernel launch from the oracle's restatement of its work: per
-    traced ray 32 B (o, d, tmin, tmax) + 1 B valid + the result (16 B id/t/u/v, 1 B occlusion),
-    64 B per search-BVH node loaded, 52 B per strict leaf test (v1, e1, e2 and the triangle
-    id), 64 B per chain cull (one hierarchy node) and 36 B per chain (the triangle's
-    vertices).  Arithmetic: 24 FLOP per node (two slab tests), 45 per leaf test, 60 per cull."""
-    out_b = 1 if mode == 2 else 16
-    b = (st.rays * (33 + out_b) + st.visits * 64 + st.tests * 52 + st.culls * 64
-         + st.chains * 36)
+def per_ray_roofline(name, t_ms, rays, ntri, mode, workload, st=None):
+    """Roofline of a per-ray kernel launch.  Bytes: what it cannot do without, each ray read once
+    (32 B o, d, tmin, tmax + 1 B valid), its result written once (16 B id/t/u/v, 1 B occlusion)
+    and each triangle read once (36 B).  The walk's node and leaf loads are served by the caches
+    many times over, so they are no floor; `traffic`, `busy_measured` and
+    `lane_utilisation_measured` are what the counters saw.  st: the oracle's counts of the walk
+    of each ray through the binary tree (the kernel's four-wide tree is that one collapsed), with
+    24 FLOP per node (two slab tests), 45 per leaf test and 60 per cull."""
+    b = rays * (33 + (1 if mode == 2 else 16)) + ntri * 36
     achieved = b / (t_ms * 1e-3) / 1e9
-    flops = 24 * st.visits + 45 * st.tests + 60 * st.culls
-    tflops = flops / (t_ms * 1e-3) / 1e12
     facts = profile_facts(workload, name)
     traffic = facts.get("traffic-per-launch")
     hbm_meas = None if traffic is None else traffic / (t_ms * 1e-3) / 1e9 / HBM_PEAK_GBS
-    return {"bound": bound_of(facts, hbm_meas, achieved / HBM_PEAK_GBS,
-                              tflops / FP32_UNPACKED_TFLOPS), "kernel": name,
-            "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4),
-            "traffic": None if traffic is None else int(traffic),
-            "bytes_per_launch": int(b), "ms_per_launch": round(t_ms, 4),
-            "counts": {"rays": int(st.rays), "node_loads": int(st.visits),
-                       "leaf_tests": int(st.tests), "chain_culls": int(st.culls),
-                       "chains": int(st.chains)},
-            "valu": {"flops_per_launch": int(flops), "achieved": round(tflops, 3),
+    valu = {"busy_measured": facts.get("valu-busy"),
+            "lane_utilisation_measured": facts.get("lane-utilisation")}
+    out = {"bound": bound_of(facts, hbm_meas, achieved / HBM_PEAK_GBS, 1.0), "kernel": name,
+           "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+           "frac": round(achieved / HBM_PEAK_GBS, 4),
+           "traffic": None if traffic is None else int(traffic),
+           "bytes_per_launch": int(b), "ms_per_launch": round(t_ms, 4), "valu": valu}
+    if st is not None:
+        flops = 24 * st.visits + 45 * st.tests + 60 * st.culls
+        tflops = flops / (t_ms * 1e-3) / 1e12
+        out["counts_binary_tree"] = {"rays": int(st.rays), "node_loads": int(st.visits),
+                                     "leaf_tests": int(st.tests), "chain_culls": int(st.culls),
+                                     "chains": int(st.chains)}
+        valu.update({"flops_per_launch": int(flops), "achieved": round(tflops, 3),
                      "unit": "TFLOP/s", "peak": FP32_PEAK_TFLOPS,
                      "frac": round(tflops / FP32_PEAK_TFLOPS, 4),
-                     "peak_unpacked": FP32_UNPACKED_TFLOPS,
-                     "busy_measured": facts.get("valu-busy"),
-                     "lane_utilisation_measured": facts.get("lane-utilisation")}}
+                     "peak_unpacked": FP32_UNPACKED_TFLOPS})
+    return out
 
 
 def _window(r, x0, y0, w, h):
@@ -275,8 +276,8 @@ def bench_uneven(args, rt, scenes, torch, orc):
         ex.close()
 
     # rooflines of both per-ray kernels: a kernel's work is every ray it traces, so each is timed
-    # with every block of its mode sent to it (median of 3 eager runs), and the oracle's
-    # restatement counts that work; the line's roofline is the one whose kernel takes longer
+    # with every block of its mode sent to it (median of 3 eager runs), and the oracle
+    # counts the walks; the line's roofline is the one whose kernel takes longer
     # in the step, the other is reported beside it
     b.set_param(rt.RT_PARAM_GRAPH, 0)
     rooflines = {}
@@ -305,8 +306,10 @@ def bench_uneven(args, rt, scenes, torch, orc):
             else:
                 for f in ("rays", "visits", "tests", "culls", "chains"):
                     setattr(tot, f, getattr(tot, f) + getattr(st, f))
-        kname = f"ray_path_kernel<{hm},0,false>"
-        rooflines[mname] = per_ray_roofline(kname, t_kernel, tot, hm, "uneven_batch_64")
+        kname = f"ray_path_kernel<{hm},0,false,false>"
+        rooflines[mname] = per_ray_roofline(kname, t_kernel, int(tot.rays),
+                                            sum(j["v9"].size // 9 for j in jobs), hm,
+                                            "uneven_batch_64", tot)
         rooflines[mname]["measured_as"] = (
             f"the {mname} jobs of the batch with every block sent to the per-ray kernel, "
             f"median of 3 eager runs")
@@ -560,7 +563,8 @@ def bench_frame(args, rt, scenes, torch, orc, wl):
 def bench_plain(args, rt, scenes, torch, orc, name):
     """One plain per-scene workload (a scene of WORKLOADS): the primary trace, shadow rays and
     occlusion trace (and path bounces to its depth) on the device; the dominant traversal
-    kernel against the HBM roofline by the reference candidate set's algorithmic bytes."""
+    kernel against the HBM roofline (block path, if its parameters ask for it: by the reference
+    candidate set's algorithmic bytes)."""
     wl = scenes.WORKLOADS[name]
     log(f"workload {name}: building scene")
     v9 = scenes.make_scene(wl["scene"])
@@ -664,7 +668,15 @@ def bench_plain(args, rt, scenes, torch, orc, name):
                             "near_ties": int((ref["flags"] & orc.NEAR_TIE != 0).sum()),
                             "ulp_marginal": int((ref["flags"] & orc.ULP_MARGINAL != 0).sum()
                                                 + (oref["flags"] & orc.ULP_MARGINAL != 0).sum())}
-        if accel != "naive":
+        if accel != "naive" and not (args.ray_closest or args.ray_occluded):
+            # every block is traced ray by ray
+            tc, to = km.get("closest_per_ray", 0.0), km.get("occlusion_per_ray", 0.0)
+            bvh_s = "true" if accel == "ray-bvh" else "false"
+            m, t, k = (2, to, n_shadow) if to >= tc else (0, tc, n)
+            if t > 0:
+                roofline = per_ray_roofline(f"ray_path_kernel<{m},0,{bvh_s},true>", t, k,
+                                            v9.size // 9, m, name)
+        elif accel != "naive":
             # the block path's work: rays 32 B + hit 16 B (closest) or 1 B (occlusion), 36 B per
             # (leaf, triangle) pair reaching the leaf test, 24 B per (hierarchy node, triangle)
             # cull evaluation (+ 32 B per BVH node for ray-bvh) of the reference candidate set
