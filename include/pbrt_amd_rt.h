@@ -163,10 +163,10 @@ int rt_trace_occluded(rt_scene *scene, const rt_rays *rays, uint8_t *occluded, v
  * that forbid hipMalloc).  Same arguments and the same results as rt_trace_closest; its
  * scratch (hierarchy, reduction keys, work queue, job table) lives in a static device array of
  * 64 MiB per device, set up by rt_ctx_create and held until the process ends.  A call needs
- * at most about 22 bytes per ray, its hierarchy included (naive: 8 bytes per ray), so up to
- * about 3 million rays; a larger one returns RT_ERR_TOO_LARGE.  Every call on a device shares that array, which keeps
- * the last call's contents: calls that overlap in time on one device race (serialize them,
- * e.g. on one stream). */
+ * at most about 22 bytes per ray, its hierarchy included, so up to about 3 million rays; a
+ * larger one returns RT_ERR_TOO_LARGE (naive, which uses none of it: beyond 8 bytes per ray).
+ * Every call on a device shares that array, which keeps the last call's contents: calls that
+ * overlap in time on one device race (serialize them, e.g. on one stream). */
 int rt_trace_closest_noalloc(rt_scene *scene, const rt_rays *rays, int32_t mode,
                              const rt_hits *hits, void *stream);
 

@@ -4,24 +4,29 @@
 //   triangles  v9[9*ntri] (p1, p2, p3), resident per scene; uv6[6*ntri] optional
 //   rays       structure of arrays ox..dz, tmin, tmax (+ valid bytes), row-major ray image
 //   hierarchy  4 float4 per node {dmin|valid, dmax, omin, omax}, level-major, row-major
-//   keys       one uint64 per ray: (order-preserving t bits << 32) | triangle id
+//   keys       one uint64 per ray: (order-preserving t bits << 32) | triangle id (block path)
+//   search     64-byte four-wide nodes of FP16 planes in a grid cell's units (per-ray path)
 //   bvh        2 float4 per node {ax ay az bx}{by bz primOffset nPrimitives}
 //
 // Work decomposition of a rayhierarchy / ray-bvh trace (a launch group of one or more jobs):
-//   init      clears the per-ray keys / occlusion flags and the group counters;
 //   build     one 256-thread work-group per top-level hierarchy node ("block") builds the
-//             block's leaves and levels from its rays;
+//             block's leaves and levels from its rays and clears the group's counters;
+//   ray path  wavefronts take 64-ray chunks of every block, walk each ray through a search tree
+//             of the triangles and write its hit record or occlusion flag;
+//   repair    the reference's repairRun pass for the rays that were listed for it.
+// With RT_PARAM_RAY_CLUSTERS_* above 0, coherent blocks take the block path instead:
+//   init      clears the per-ray keys / occlusion flags and the group counters;
 //   cluster   one work-group per block bounds every cluster of 64 triangles (or of 64 ray-bvh
 //             frontier roots) against the block root and queues work units of a few passing
-//             clusters;
+//             clusters, or the block's chunks for the ray path;
 //   unit      a persistent grid (one work-group per resident slot) takes units from the queue
 //             with an atomic counter, stages the unit's block of rays and subtree in LDS and
 //             traverses (phases below); per-ray results are reduced in LDS and merged with
 //             global atomics;
-//   finalize  turns each ray's (t, id) key into id / t / u / v (+ dpdu, dpdv);
-//   repair    the reference's repairRun pass for the rays finalize flagged.
-// The nearest hit is reduced as a (t, id) key with atomic min, so the result is
-// deterministic (ties -> smallest id).
+//   finalize  turns each ray's (t, id) key into id / t / u / v (+ dpdu, dpdv).
+// naive is one launch: a work-group has its rays' whole answer.
+// The nearest hit is the smallest (t, id) key, so the result is deterministic (ties -> smallest
+// id).
 #include <algorithm>
 #include <atomic>
 #include <map>
@@ -1667,7 +1672,7 @@ __device__ void write_hit(const RaysDev& r, const float* __restrict__ v9,
 }
 
 // ---------------------------------------------------------------------------------------
-// Per-ray path (blocks the cluster pass queued as incoherent).  A ray's result is the argmin
+// Per-ray path (every block, or those the cluster pass queued).  A ray's result is the argmin
 // over the triangles that pass its strict leaf test AND the exact cull chain of its leaf (for
 // ray-bvh: that are tested at a (BVH leaf, hierarchy leaf) pair whose lockstep chain passes).
 // Every such triangle passes the strict leaf test, so each ray walks the scene's search BVH
