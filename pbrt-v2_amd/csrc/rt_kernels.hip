@@ -2391,7 +2391,7 @@ __device__ __forceinline__ bool naive_b1(const float4 (&q)[3], V3 d, V3 m, float
 // reduce by atomics and turn into hit records by launches of their own.
 // Bound by vector issue: the leaf test alone takes 26 instructions to its first reject, the
 // filter 12.  1,024 triangles, 128 x 128 rays: closest 24.5 -> 21 us and occlusion 27.6 -> 22 us
-// (without the launches saved), 4,096 triangles, 250 x 200 rays: 392 -> 266 us for both.
+// (without the launches saved), 4,096 triangles, 250 x 200 rays: 392 -> 240 us for both.
 template <int MODE>
 __global__ __launch_bounds__(kNaiveThreads) void naive_kernel(RaysDev r,
                                                               const float* __restrict__ v9,
@@ -3007,11 +3007,12 @@ hipError_t launch_naive_trace(const RaysDev& r, int mode, const float* v9, const
                               uint32_t ntri, bool naive_rule, HitOut out, uint8_t* occ,
                               hipStream_t s) {
   const size_t n = (size_t)r.W * r.H;
-  // Rays to a work-group: as many as leave 512 work-groups, two to a CU, and 8 at least.  With
-  // work-groups of 1,024 threads, one to a CU, 4,096 triangles and 250 x 200 rays take 352 us in
-  // place of 266 (128 x 128 rays: equal); with 128 rays always, 33 x 40 rays leave 245 CUs idle.
+  // Rays to a work-group: as many as leave 1,024 work-groups, four to a CU (three are resident
+  // at once), and 8 at least.  4,096 triangles, 250 x 200 rays, both kernels: 512 work-groups
+  // 266 us, 1,024 240, 2,048 254, 4,096 335 (every work-group stages all triangles); 128 x 128
+  // rays equal.  With 128 rays always, 33 x 40 rays would leave 245 CUs idle.
   int shift = kNaiveShift;
-  while (shift > 2 && ((n - 1) >> (shift + 1)) + 1 < 512) --shift;
+  while (shift > 2 && ((n - 1) >> (shift + 1)) + 1 < 1024) --shift;
   const dim3 grid((unsigned)(((n - 1) >> (shift + 1)) + 1));
   auto run = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(kNaiveThreads), 0, s, r, v9, uv6, ntri, shift, out,

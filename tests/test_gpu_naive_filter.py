@@ -38,7 +38,7 @@ def _rays(rng, v9, w, h, scale):
 
 @pytest.mark.parametrize("ntri,w,h,scale", [(1, 1, 1, 1.0), (5, 31, 7, 1.0), (511, 64, 33, 1.0),
                                             (513, 40, 9, 1e4), (1025, 129, 65, 1.0),
-                                            (70, 300, 220, 0.01), (300, 50, 20, 1e18),
+                                            (70, 300, 220, 0.01), (9, 400, 330, 1.0), (300, 50, 20, 1e18),
                                             (300, 50, 20, 1e-18), (200, 37, 11, 1e12)])
 def test_naive_equals_oracle(rt, orc, gpu_ctx, ntri, w, h, scale):
     rng = np.random.default_rng(ntri * 1000 + w)
