@@ -172,11 +172,12 @@ constexpr int kDefaultWalk = 3;
 //   [3].y   index of the first interior child; child i < ni is node [3].y + i
 //   [3].z   kSearchLeafBit + position of the first leaf's triangle - ni, so that child i >= ni
 //           is the leaf reference [3].z + i (one triangle per leaf)
-// Absent children have lower planes above their upper planes on every axis; should rounding let
-// a ray into one all the same, its reference is the record of some other triangle (the records
-// end with kSearchPad that no ray hits), whose test is harmless.  A depth-first walk
-// that keeps the unvisited children of every node on its path holds at most kSearchStack of
-// them.
+//   [3].w   the number of children n (1..4): a walk enters children below n only
+// A depth-first walk that keeps the unvisited children of every node on its path holds at most
+// kSearchStack of them, whatever the ray: the builder counts n - 1 for a node, and the count, not
+// the planes of the absent children, keeps a ray out of those (a direction or origin that is not
+// finite, or an origin so far out that its slack exceeds the planes' range, passes every plane
+// test).
 constexpr uint32_t kSearchLeafBit = 0x80000000u;
 constexpr int kSearchDepth = 26;  // interior levels of the binary tree it is collapsed from
 // Entries of the walk's stack in LDS; the tree's builder keeps narrower nodes where a deeper
@@ -185,7 +186,7 @@ constexpr int kSearchDepth = 26;  // interior levels of the binary tree it is co
 // With 26 entries the nodes were a fifth more on a cluster scene (1 M segments 673 us, 626 with
 // 30).
 constexpr int kSearchStack = 32;
-constexpr uint32_t kSearchPad = 4;
+constexpr uint32_t kSearchPad = 4;  // records of zeros after the triangles'
 // Builds the search tree of `ntri` triangles (v9 in the caller's order): the nodes (4 uint4
 // each), the search order (position -> triangle index) and the frame of the node planes.
 void build_search_bvh(const float* v9, uint32_t ntri, std::vector<uint4>& nodes,

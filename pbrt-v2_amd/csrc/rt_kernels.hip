@@ -37,6 +37,7 @@
 #include "../../include/pbrt_amd_rt.h"
 #include "rt_device.h"
 #include "rt_internal.h"
+#include "rt_search.h"
 
 using namespace rtd;
 
@@ -1681,35 +1682,6 @@ __device__ void write_hit(const RaysDev& r, const float* __restrict__ v9,
 // ray.  The (t, id) key, the repair-region key and the occlusion flag are the block path's,
 // so the outcome is the same; every ray of a block is handled by exactly one lane, which
 // writes its results directly.
-constexpr float kSlack = 0x1p-16f;   // relative slack of the slab-test parameters
-constexpr float kOffSlack = 0x1p-20f;  // the same of a ray's plane offsets
-
-// Ray against the planes of a wide node (SearchFrame units): the parameter of plane g + h of an
-// axis (grid cell g, FP16 offset h) is g * ih + c + h * ih with ih = unit / d and c =
-// (base - o) / d.  c is widened outward (down to cn for near planes, up to cf for far ones) by
-// kOffSlack, which covers its own rounding and that of the sums; the scale h * ih + ... rounds
-// once more, which kSlack covers on the far side.
-struct SlabRay {
-  V3 ih, cn, cf;
-};
-__device__ __forceinline__ void slab_axis(float o, float d, float base, float unit, float& ih,
-                                          float& cn, float& cf) {
-  // zero components become tiny ones, so the slab of that axis is (almost) the whole line when
-  // the origin is inside it and empty otherwise
-  const float inv = 1.0f / (fabsf(d) < 0x1p-80f ? (d < 0.f ? -0x1p-80f : 0x1p-80f) : d);
-  const float c = (base - o) * inv, w = fabsf(c) * kOffSlack;
-  ih = inv * unit;
-  cn = c - w;
-  cf = c + w;
-}
-
-typedef _Float16 rt_h2 __attribute__((ext_vector_type(2)));
-// Child c's FP16 plane of a packed quadruple (two words).
-__device__ __forceinline__ float plane(uint32_t w01, uint32_t w23, int c) {
-  const rt_h2 h = __builtin_bit_cast(rt_h2, c < 2 ? w01 : w23);
-  return (float)h[c & 1];
-}
-
 // Hierarchy node of level l above image position (x, y), from the job's node array.  The
 // job (and so g) may differ between the lanes of a wavefront: the level's table entries are
 // read with the lane's own index, two loads instead of a select over every level.
@@ -2115,37 +2087,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
       if (act && cur != kDone && !(cur & kSearchLeafBit)) {
         const uint4 nx = ldu4(snode, 4 * (size_t)cur), ny = ldu4(snode, 4 * (size_t)cur + 1),
                     nz = ldu4(snode, 4 * (size_t)cur + 2), nm = ldu4(snode, 4 * (size_t)cur + 3);
-        const float gx = (float)(nm.x & 255u), gy = (float)((nm.x >> 8) & 255u),
-                    gz = (float)((nm.x >> 16) & 255u);
-        const uint32_t ni = nm.x >> 24;
-        // plane parameters of the cell's corner; near and far plane words by the ray's sign
-        const V3 an = {fmaf(gx, sr.ih.x, sr.cn.x), fmaf(gy, sr.ih.y, sr.cn.y),
-                       fmaf(gz, sr.ih.z, sr.cn.z)};
-        const V3 af = {fmaf(gx, sr.ih.x, sr.cf.x), fmaf(gy, sr.ih.y, sr.cf.y),
-                       fmaf(gz, sr.ih.z, sr.cf.z)};
-        const bool sx = sr.ih.x < 0.f, sy = sr.ih.y < 0.f, sz = sr.ih.z < 0.f;
-        const uint32_t nx0 = sx ? nx.z : nx.x, nx1 = sx ? nx.w : nx.y, fx0 = sx ? nx.x : nx.z,
-                       fx1 = sx ? nx.y : nx.w;
-        const uint32_t ny0 = sy ? ny.z : ny.x, ny1 = sy ? ny.w : ny.y, fy0 = sy ? ny.x : ny.z,
-                       fy1 = sy ? ny.y : ny.w;
-        const uint32_t nz0 = sz ? nz.z : nz.x, nz1 = sz ? nz.w : nz.y, fz0 = sz ? nz.x : nz.z,
-                       fz1 = sz ? nz.y : nz.w;
-        // sort key of a child: its entry parameter, the child in the low two bits; kMiss sorts
-        // last (only the order of the visits depends on the lost bits)
-        constexpr uint32_t kMiss = 0xffffffffu;
         uint32_t key[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const float tn = fmaxf(fmaxf(fmaf(plane(nx0, nx1, c), sr.ih.x, an.x),
-                                       fmaf(plane(ny0, ny1, c), sr.ih.y, an.y)),
-                                 fmaf(plane(nz0, nz1, c), sr.ih.z, an.z));
-          const float tf = fminf(fminf(fmaf(plane(fx0, fx1, c), sr.ih.x, af.x),
-                                       fmaf(plane(fy0, fy1, c), sr.ih.y, af.y)),
-                                 fmaf(plane(fz0, fz1, c), sr.ih.z, af.z));
-          const float en = fmaxf(tn, tlo);
-          const bool hit = en <= fminf(fmaf(fabsf(tf), kSlack, tf), thi);
-          key[c] = hit ? (__float_as_uint(en) & ~3u) | (uint32_t)c : kMiss;
-        }
+        node_keys(nx, ny, nz, nm, sr, tlo, thi, key);
+        const uint32_t ni = nm.x >> 24;
         auto ref = [&](uint32_t k) {
           const uint32_t c = k & 3u;
           return (c < ni ? nm.y : nm.z) + c;
@@ -2155,10 +2099,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
         key_swap(key[0], key[2]);
         key_swap(key[1], key[3]);
         key_swap(key[1], key[2]);
-        if (key[3] != kMiss) sStk[sp++][lane] = ref(key[3]);
-        if (key[2] != kMiss) sStk[sp++][lane] = ref(key[2]);
-        if (key[1] != kMiss) sStk[sp++][lane] = ref(key[1]);
-        cur = key[0] != kMiss ? ref(key[0]) : pop();
+        if (key[3] != kNoChild) sStk[sp++][lane] = ref(key[3]);
+        if (key[2] != kNoChild) sStk[sp++][lane] = ref(key[2]);
+        if (key[1] != kNoChild) sStk[sp++][lane] = ref(key[1]);
+        cur = key[0] != kNoChild ? ref(key[0]) : pop();
         if (pl == kDone && cur != kDone && (cur & kSearchLeafBit)) {
           pl = cur;
           cur = pop();

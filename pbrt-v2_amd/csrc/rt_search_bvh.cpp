@@ -339,7 +339,8 @@ class Collapser {
       }
       p[k] = make_uint4(h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16);
     }
-    p[3] = make_uint4(cells | (uint32_t)ni << 24, first, (kSearchLeafBit | tri) - (uint32_t)ni, 0u);
+    p[3] = make_uint4(cells | (uint32_t)ni << 24, first, (kSearchLeafBit | tri) - (uint32_t)ni,
+                      (uint32_t)n);
   }
 
   const std::vector<BNode>& B_;
