@@ -191,7 +191,7 @@ int rt_make_bounce_rays(rt_scene *scene, const rt_rays *in, const int32_t *id, c
                         void *stream);
 
 /* Launch-shape parameters (set by the autotuner; 0 restores the built-in choice).  None of
- * them changes any result.
+ * them changes any result, but for what is said at RT_PARAM_RAY_CLUSTERS_*.
  *   RT_PARAM_CLUSTERS_CLOSEST / RT_PARAM_CLUSTERS_OCCLUDED: passing triangle clusters (64
  *   triangles each) per rayhierarchy work unit for closest-hit / occlusion traces; smaller
  *   values split a block's work over more units of the persistent traversal kernel.
@@ -211,6 +211,13 @@ int rt_make_bounce_rays(rt_scene *scene, const rt_rays *in, const int32_t *id, c
  *   the block's (leaf, triangle) candidate pairs.  1 sends every block with work that way;
  *   2^29 keeps only the direction test; a value above 2^29 (at most 2^30) sends no block.
  *   Built-in (0): every block, without looking at its clusters.
+ *   Ray by ray, a strict hit of a ray within about a degree of a triangle's plane can be missed:
+ *   the strict test accepts such rays by its roundings, where no bounded search looks.  The
+ *   built-in form tests the triangles that a block's rays could graze beside the search, in blocks
+ *   of at most 1,024 rays and four levels whose leaves' directions spread by at most 0.25 on
+ *   average (every such block in a scene of at most 128 triangles), but for occlusion blocks that
+ *   pass 256 (rayhierarchy) or 64 (ray-bvh) clusters of four times as many; values from 1 on do
+ *   not.
  *   RT_PARAM_RAY_GRID_CLOSEST / RT_PARAM_RAY_GRID_OCCLUDED: work-groups (one wavefront each)
  *   of the per-ray kernel (batches only); 0 = one per resident slot.
  *   RT_PARAM_WALK_CLOSEST / RT_PARAM_WALK_OCCLUDED: v in 1..7: a round of the per-ray kernel

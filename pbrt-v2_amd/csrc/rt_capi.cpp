@@ -139,6 +139,13 @@ struct rt_scene {
   uint4* d_snode = nullptr;
   float4* d_tmts = nullptr;
   SearchFrame sframe{};
+  // grazing pass, in the order of the clusters' triangles (RhItem)
+  GrazeNormal* d_gnormal = nullptr;
+  GrazeTri* d_graze = nullptr;
+  float4* d_gtest = nullptr;
+  uint32_t* d_gfirst = nullptr; // ray-bvh: first record of every cluster of frontier roots
+  GrazeCluster* d_gcluster = nullptr;
+  float4* d_gbox = nullptr;     // boxes of every 64 clusters
   uint32_t* d_tleaf = nullptr;  // ray-bvh: reference BVH leaf of every original triangle
   uint32_t nclusters = 0;
   int clusters_closest = 0, clusters_occluded = 0;  // 0 = built-in choice
@@ -327,6 +334,52 @@ hipError_t upload(T*& d, const T* h, size_t n) {
   return e;
 }
 
+// Records of the grazing pass for the n triangles d_order (device), in clusters of the boxes cbox
+// (2 each) as s->d_gfirst cuts them.
+hipError_t graze_setup(rt_scene* s, const uint32_t* d_order, size_t n,
+                       const std::vector<float4>& cbox) {
+  const size_t nc = cbox.size() / 2, ng = (nc + 63) / 64;
+  std::vector<float4> gbox(2 * ng);
+  for (size_t c = 0; c < nc; ++c) {
+    float4 &lo = gbox[2 * (c / 64)], &hi = gbox[2 * (c / 64) + 1];
+    const float4 &a = cbox[2 * c], &b = cbox[2 * c + 1];
+    if (c % 64 == 0) {
+      lo = a;
+      hi = b;
+    }
+    lo = make_float4(std::min(lo.x, a.x), std::min(lo.y, a.y), std::min(lo.z, a.z), 0.f);
+    hi = make_float4(std::max(hi.x, b.x), std::max(hi.y, b.y), std::max(hi.z, b.z), 0.f);
+  }
+  hipError_t e = upload(s->d_gbox, gbox.data(), gbox.size());
+  if (e == hipSuccess)
+    e = hipMalloc((void**)&s->d_graze, sizeof(GrazeTri) * std::max<size_t>(n, 1));
+  if (e == hipSuccess)
+    e = hipMalloc((void**)&s->d_gnormal, sizeof(GrazeNormal) * std::max<size_t>(n, 1));
+  if (e == hipSuccess)
+    e = hipMalloc((void**)&s->d_gtest, 3 * sizeof(float4) * std::max<size_t>(n, 1));
+  if (e == hipSuccess)
+    e = hipMalloc((void**)&s->d_gcluster, sizeof(GrazeCluster) * std::max<size_t>(nc, 1));
+  if (e == hipSuccess)
+    e = launch_graze_records(s->d_v9, d_order, s->d_tleaf, (uint32_t)n, s->d_gfirst, (uint32_t)nc,
+                             s->sframe, s->d_gnormal, s->d_graze, s->d_gtest, s->d_gcluster,
+                             nullptr);
+  return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
+}
+void graze_free(rt_scene* s) {
+  (void)hipFree(s->d_gnormal);
+  (void)hipFree(s->d_graze);
+  (void)hipFree(s->d_gtest);
+  (void)hipFree(s->d_gfirst);
+  (void)hipFree(s->d_gcluster);
+  (void)hipFree(s->d_gbox);
+  s->d_gnormal = nullptr;
+  s->d_graze = nullptr;
+  s->d_gtest = nullptr;
+  s->d_gfirst = nullptr;
+  s->d_gcluster = nullptr;
+  s->d_gbox = nullptr;
+}
+
 // Launches `fn` bracketed by the timer's next event pair for `mode` (if timing is on).
 template <class F>
 hipError_t timed_launch(Timer& tm, int mode, hipStream_t st, F fn) {
@@ -368,6 +421,12 @@ int fill_item(const RhJob& jb, RhItem& it) {
   it.sframe = jb.s->sframe;
   it.tmts = jb.s->d_tmts;
   it.tleaf = jb.s->d_tleaf;
+  it.gnormal = jb.s->d_gnormal;
+  it.graze = jb.s->d_graze;
+  it.gtest = jb.s->d_gtest;
+  it.gfirst = jb.s->d_gfirst;
+  it.gcluster = jb.s->d_gcluster;
+  it.gbox = jb.s->d_gbox;
   it.ntri = jb.s->ntri;
   it.flags = jb.s->ctx->d_flags;
   it.nclusters = bvh ? (jb.s->ntri ? jb.s->nrclusters : 0) : jb.s->nclusters;
@@ -384,6 +443,11 @@ int fill_item(const RhJob& jb, RhItem& it) {
   it.occ = jb.occ;
   it.repair_run = (jb.mode == 0 && !bvh) ? jb.s->desc.repair_run : 0;
   return RT_OK;
+}
+
+// Whether the grazing pass of the job's blocks need not count their passing clusters first.
+bool graze_uncounted(const RhItem& it, int mode, bool bvh) {
+  return mode != 2 || it.nclusters < 4u * (bvh ? kHeavyBvh : kHeavy);
 }
 
 // Lays out the jobs as launch groups (one per mode and node type, in job order) in the
@@ -416,12 +480,12 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
   // geometry and sizes
   std::vector<RhItem> items(jobs.size());
   std::vector<size_t> off_nodes(jobs.size()), off_clist(jobs.size()), off_keys(jobs.size()),
-      off_rep(jobs.size());
+      off_rep(jobs.size()), off_gblock(jobs.size()), off_gseed(jobs.size());
   size_t total = 0;
   const size_t tables = align256(sizeof(RhItem) * std::max<size_t>(jobs.size(), 1));
   total += tables;
   struct GroupLayout {
-    size_t units, ustage, bunits, rq, ctr, replist, max_units, max_chunks;
+    size_t units, ustage, bunits, rq, heavy, ctr, replist, max_units, max_chunks;
     uint32_t ray;
     int rgrid, walk;
     uint32_t nblocks, nrays;
@@ -478,6 +542,12 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
       if (mode != 2 && !direct) total += align256(sizeof(uint64_t) * n);
       off_rep[j] = total;
       if (it.repair_run > 0 && !direct) total += align256(sizeof(uint32_t) * n);
+      off_gblock[j] = off_gseed[j] = total;
+      if (direct && graze_shape(it.g)) {
+        total += align256(sizeof(uint32_t) * (size_t)it.g.ntop);
+        off_gseed[j] = total;
+        if (mode != 2) total += align256(sizeof(uint64_t) * n);
+      }
     }
     if (blocks >= (1ull << 31) || rays >= (1ull << 31)) return RT_ERR_UNSUPPORTED;
     L.nblocks = (uint32_t)blocks;
@@ -496,6 +566,8 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
       L.rq = total;
       total += align256(sizeof(uint2) * std::max<size_t>(L.max_chunks, 1));
     }
+    L.heavy = total;
+    if (direct) total += align256(sizeof(uint32_t) * L.nblocks);
     L.ctr = total;
     total += align256(kCounterBytes);
     L.replist = total;
@@ -526,12 +598,21 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
     it.clist = direct ? nullptr : (uint32_t*)(A + off_clist[j]);
     it.keys = jobs[j].mode != 2 && !direct ? (uint64_t*)(A + off_keys[j]) : nullptr;
     it.repkeys = it.repair_run > 0 && !direct ? (uint32_t*)(A + off_rep[j]) : nullptr;
+    const bool graze = direct && graze_shape(it.g);
+    it.gblock = graze ? (uint32_t*)(A + off_gblock[j]) : nullptr;
+    it.gseed = graze && jobs[j].mode != 2 ? (uint64_t*)(A + off_gseed[j]) : nullptr;
   }
   // tables in group order
   std::vector<RhItem> table;
   table.reserve(jobs.size());
   for (size_t gi = 0; gi < keys.size(); ++gi) {
     RhGroup G{};
+    for (int j : members[gi])
+      if (items[j].gblock) G.graze = 1;
+    if (G.graze && gl[gi].nblocks <= kGrazeSmall) G.graze = 2;
+    for (int j : members[gi])
+      if (!graze_uncounted(items[j], keys[gi].first, (keys[gi].second >> 2) != 0)) G.graze &= 1;
+    for (int j : members[gi]) items[j].gsliced = G.graze == 2;
     G.items = (const RhItem*)A + table.size();
     for (int j : members[gi]) table.push_back(items[j]);
     G.nitems = (int)members[gi].size();
@@ -551,6 +632,7 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
     G.ray_grid = gl[gi].rgrid;
     G.walk = gl[gi].walk;
     G.ctr = (uint32_t*)(A + gl[gi].ctr);
+    G.heavy = (uint32_t*)(A + gl[gi].heavy);
     G.replist = gl[gi].repair ? (uint32_t*)(A + gl[gi].replist) : nullptr;
     G.per_unit = gl[gi].per;
     G.grid = gl[gi].grid;
@@ -724,6 +806,7 @@ int rt_scene_create(rt_ctx* ctx, const float* v9, const float* uv6, uint32_t ntr
         e = upload(s->d_tbox, tbox.data(), tbox.size());
       }
       s->nclusters = (uint32_t)(cbox.size() / 2);
+      if (e == hipSuccess) e = graze_setup(s, s->d_perm, ntri, cbox);
     }
   }
   if (e == hipSuccess && desc->kind == RT_ACCEL_RAYBVH && ntri) {
@@ -848,6 +931,24 @@ int rt_scene_set_bvh(rt_scene* s, const rt_gpu_node* nodes, uint32_t nnodes, con
     }
     s->nrclusters = nc;
   }
+  // Grazing pass: the triangles below every cluster's roots.
+  std::vector<uint32_t> gorder, gfirst(1, 0);
+  for (uint32_t k = 0; k < s->nrclusters; ++k) {
+    for (uint32_t r = k * kClusterSize; r < std::min(nroots, (k + 1) * kClusterSize); ++r) {
+      std::vector<uint32_t> stack{rsorted[r]};
+      while (!stack.empty()) {
+        const uint32_t n = stack.back();
+        stack.pop_back();
+        for (uint32_t f = 0; f < nodes[n].n_primitives; ++f)
+          gorder.push_back(prim_order[nodes[n].prim_offset + f]);
+        if (nodes[n].n_primitives) continue;
+        if (s->desc.node == RT_NODE_BOX_UV && nodes[n].prim_offset == 0) continue;
+        stack.push_back(nodes[n].prim_offset);
+        stack.push_back(nodes[n].prim_offset + 1);
+      }
+    }
+    gfirst.push_back((uint32_t)gorder.size());
+  }
   RT_TRY(hipSetDevice(s->ctx->device));
   if (s->d_rcbox) (void)hipFree(s->d_rcbox);
   s->d_rcbox = nullptr;
@@ -857,6 +958,7 @@ int rt_scene_set_bvh(rt_scene* s, const rt_gpu_node* nodes, uint32_t nnodes, con
   if (s->d_bvh_parent) (void)hipFree(s->d_bvh_parent);
   if (s->d_bvh_depth) (void)hipFree(s->d_bvh_depth);
   if (s->d_tleaf) (void)hipFree(s->d_tleaf);
+  graze_free(s);
   s->d_tleaf = nullptr;
   s->d_bvh = nullptr;
   s->d_roots = s->d_prim_order = s->d_bvh_parent = nullptr;
@@ -869,6 +971,15 @@ int rt_scene_set_bvh(rt_scene* s, const rt_gpu_node* nodes, uint32_t nnodes, con
   RT_TRY(upload(s->d_bvh_parent, parent.data(), parent.size()));
   RT_TRY(upload(s->d_bvh_depth, depth.data(), depth.size()));
   RT_TRY(upload(s->d_tleaf, tleaf.data(), tleaf.size()));
+  RT_TRY(upload(s->d_gfirst, gfirst.data(), gfirst.size()));
+  {
+    uint32_t* d_order = nullptr;
+    hipError_t e = upload(d_order, gorder.data(), gorder.size());
+    rcbox.resize(2 * (size_t)s->nrclusters);
+    if (e == hipSuccess) e = graze_setup(s, d_order, gorder.size(), rcbox);
+    (void)hipFree(d_order);
+    if (e != hipSuccess) return hip_status(e);
+  }
   RT_TRY(launch_set_tleaf(s->d_tmts, s->d_tleaf, s->ntri, nullptr));
   RT_TRY(hipStreamSynchronize(nullptr));
   s->nroots = nroots;
@@ -888,6 +999,7 @@ int rt_scene_destroy(rt_scene* s) {
   (void)hipFree(s->d_tmt);
   (void)hipFree(s->d_snode);
   (void)hipFree(s->d_tmts);
+  graze_free(s);
   (void)hipFree(s->d_tleaf);
   (void)hipFree(s->d_bvh);
   (void)hipFree(s->d_roots);
@@ -994,16 +1106,19 @@ int rt_trace_closest_noalloc(rt_scene* s, const rt_rays* rays, int32_t mode, con
   it.nodes = (float4*)take(sizeof(float4) * 4 * (size_t)it.g.nnodes);
   // reduction keys and queues, which this form once used and no longer does: the sizes that it
   // takes and refuses stay the ones its declaration promises
-  take(sizeof(uint64_t) * n);
+  uint64_t* const gseed = (uint64_t*)take(sizeof(uint64_t) * n);
   if (repair) take(sizeof(uint32_t) * n);
   take(sizeof(uint4));
-  take(sizeof(uint4) * (size_t)it.g.ntop);
-  take(sizeof(uint2) * (size_t)it.g.ntop * nch);
+  uint32_t* const gblock = (uint32_t*)take(sizeof(uint4) * (size_t)it.g.ntop);
+  uint32_t* const heavy = (uint32_t*)take(sizeof(uint2) * (size_t)it.g.ntop * nch);
   it.keys = nullptr;
   it.repkeys = nullptr;
   it.clist = nullptr;
+  it.gblock = graze_shape(it.g) ? gblock : nullptr;
+  it.gseed = graze_shape(it.g) ? gseed : nullptr;
   RhGroup G{};
   G.ctr = (uint32_t*)take(kCounterBytes);
+  G.heavy = heavy;
   G.replist = repair ? (uint32_t*)take(sizeof(uint32_t) * n) : nullptr;
   if (off > kNoAllocScratch || n >= (1ull << 31)) return RT_ERR_TOO_LARGE;
   it.block_base = 0;
@@ -1015,6 +1130,8 @@ int rt_trace_closest_noalloc(rt_scene* s, const rt_rays* rays, int32_t mode, con
   G.node = s->desc.node;
   G.bvh = kind == RT_ACCEL_RAYBVH ? 1 : 0;
   G.big = (it.g.rb > 256 || it.g.L > 3) ? 1 : 0;
+  G.graze = it.gblock == nullptr ? 0 : (uint32_t)it.g.ntop <= kGrazeSmall ? 2 : 1;
+  it.gsliced = G.graze == 2;
   G.one_ray = one_ray_leaves(it.g) ? 1 : 0;
   G.nblocks = (uint32_t)it.g.ntop;
   G.nrays = (uint32_t)n;

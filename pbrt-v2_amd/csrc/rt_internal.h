@@ -5,6 +5,8 @@
 
 #include <vector>
 
+#include "rt_search.h"
+
 struct rt_ctx {
   int device;
   uint32_t* d_flags;  // RT_FLAG_* recorded by the traversal kernels (rt_ctx_check)
@@ -67,15 +69,18 @@ int rh_geometry(int W, int H, int cx, int cy, int height, RHGeom* g);
 // Whether the leaf build has at most one ray for each of a leaf's lanes.
 inline bool one_ray_leaves(const RHGeom& g) { return g.g <= 64 && (g.g & (g.g - 1)) == 0; }
 
+// Blocks up to which a launch has several work-groups to each for the grazing pass: 16 blocks of a
+// 64 x 64 image leave most of the device idle.
+constexpr uint32_t kGrazeSmall = 64;
+// Clusters from which an occlusion block's number of passing ones is counted first (which one
+// work-group does).
+constexpr uint32_t kHeavy = 256, kHeavyBvh = 64;  // passing clusters, of four times as many
+// Whether blocks of this shape have the grazing pass.
+inline bool graze_shape(const RHGeom& g) { return g.L <= kUnitLevels && g.rb <= kMaxBlockRays; }
+
 struct HitOut {
   int32_t* id;
   float *t, *u, *v, *dpdu, *dpdv;
-};
-
-// Frame of a search tree's node planes: grid cell c of an axis starts at base + c * unit.
-struct SearchFrame {
-  float base[3];
-  float unit;
 };
 
 // One rayhierarchy traversal job: a resident scene, a ray image and its outputs, with the
@@ -101,6 +106,15 @@ struct RhItem {
   SearchFrame sframe;
   const float4* tmts;
   const uint32_t* tleaf;
+  // grazing pass: the records of the triangles of every cluster (cluster c's from gfirst[c] to
+  // gfirst[c + 1]; gfirst null: 64 each), their leaf tests' operands, index and tleaf entry (as
+  // tmts), the clusters' planes, and the boxes (as cbox) of every 64 clusters
+  const GrazeNormal* gnormal;
+  const GrazeTri* graze;
+  const float4* gtest;
+  const uint32_t* gfirst;
+  const GrazeCluster* gcluster;
+  const float4* gbox;
   uint32_t ntri;
   uint32_t nclusters;    // clusters of 64 triangles (rayhierarchy) or 64 frontier roots
   // ray-bvh: BVH nodes (2 float4 each), frontier roots (Morton-ordered; cbox holds the boxes
@@ -117,6 +131,11 @@ struct RhItem {
   uint64_t* keys;        // closest: one (t, id) key per ray
   uint32_t* repkeys;     // primary with repair: nearest repair-region t key per ray, else null
   uint8_t* occ;          // occlusion flags
+  // grazing pass: per block 0, 1 when it is looked at, kGrazeHit or kGrazeMark when any of its rays has a hit
+  // (null: no block of the job is looked at), and for closest hits the ray's nearest such hit in
+  // blocks with one
+  uint32_t* gblock;
+  uint64_t* gseed;
   HitOut out;            // closest-hit outputs
   uint32_t* flags;       // the context's RT_FLAG_* word
   uint32_t block_base, ray_base;
@@ -124,7 +143,11 @@ struct RhItem {
   uint32_t chunk_base;   // first per-ray chunk slot of the job (its blocks' slots follow)
   uint32_t unit_base;    // first staging slot of the job's work units (fixed per block)
   uint32_t unit_stride;  // staging slots per block: the most units a block can make
+  int32_t gsliced;       // the group's RhGroup::graze is 2
 };
+
+constexpr uint32_t kGrazeHit = 2;
+constexpr uint32_t kGrazeMark = 3;  // the same, and some ray has a repair-region hit at tmin
 
 // A launch group: `items` is the device copy of the job table; units, counters and the
 // repair list are shared by the group's jobs.
@@ -138,6 +161,9 @@ struct RhGroup {
   int node;  // 0 box_dir, 1 ia
   int big;   // some job has more than 256 rays per block or 4 levels
   int bvh;   // ray-bvh jobs (product traversal with the scene's BVH)
+  // some job has a grazing pass; 2: several work-groups take a block from the start (the build then
+  // clears its rays' results)
+  int graze;
   int one_ray;  // every job's leaves hold a power of two of at most 64 rays (one_ray_leaves)
   uint32_t nblocks, nrays;
   uint4* units;       // {item, block, first cluster, count}, compacted from ustage
@@ -150,6 +176,7 @@ struct RhGroup {
   uint32_t* ctr;      // [0] units, [2] rays flagged for repair, [4] set when any block goes
                       // per-ray; [64 + 32 q] and [64 + 32 q + 1]: next unit and next per-ray
                       // chunk slot of range q (kClaimQueues ranges)
+  uint32_t* heavy;    // grazing pass: queued blocks, their number in ctr[5]
   uint32_t* replist;  // global ray indices flagged for repair (primary with repair only)
   int per_unit;       // passing clusters per work unit
   int grid;           // work-groups of the persistent unit kernel; 0 = one per resident slot
@@ -199,6 +226,13 @@ constexpr size_t kNoAllocScratch = (size_t)64 << 20;
 constexpr int kMaxDevices = 64;
 int noalloc_setup(int device);
 void* noalloc_scratch(int device);
+// Records of the grazing pass for the triangles order[0 .. n) of v9 (original triangle order;
+// tleaf: RhItem::tleaf or null), and of the clusters that they make up: from first[c] to
+// first[c + 1], or 64 each (first null).
+hipError_t launch_graze_records(const float* v9, const uint32_t* order, const uint32_t* tleaf,
+                                uint32_t n, const uint32_t* first, uint32_t nclusters,
+                                const SearchFrame& frame, GrazeNormal* normal, GrazeTri* out,
+                                float4* test, GrazeCluster* cout, hipStream_t s);
 // Writes the tleaf entry of every triangle into its record in search order (RhItem::tmts).
 hipError_t launch_set_tleaf(float4* tmts, const uint32_t* tleaf, uint32_t ntri, hipStream_t s);
 

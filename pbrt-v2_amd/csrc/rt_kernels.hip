@@ -370,6 +370,17 @@ __device__ __forceinline__ uint32_t find_chunk_item_lane(const RhItem* __restric
   }
   return (uint32_t)lo;
 }
+// Job of a global block index, per lane.
+__device__ __forceinline__ uint32_t find_block_item_lane(const RhItem* __restrict__ items, int n,
+                                                         uint32_t gb) {
+  int lo = 0, hi = n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (items[mid].block_base <= gb) lo = mid;
+    else hi = mid - 1;
+  }
+  return (uint32_t)lo;
+}
 // Job of a global ray index (per lane).
 __device__ __forceinline__ int find_ray_item(const RhItem* __restrict__ items, int n,
                                              uint32_t gr) {
@@ -430,39 +441,6 @@ __device__ __forceinline__ void clear_counters(uint32_t* __restrict__ ctr, uint3
     ctr[kClaimBase + kClaimStride * i] = 0u;      // units
     ctr[kClaimBase + kClaimStride * i + 1] = 0u;  // per-ray chunk slots
   }
-}
-
-// ctr: the counters to clear for the kernels that follow (null: the init kernel does it).
-template <bool USE_VALID, bool UV, bool ONE>
-__device__ __forceinline__ void group_build(const RhItem& it, uint32_t* __restrict__ ctr) {
-  __shared__ float sBox[kMaxSub][12];
-  __shared__ int sVal[kMaxSub];
-  if (ctr != nullptr && blockIdx.x == 0) clear_counters(ctr, threadIdx.x);
-  const int b = (int)(blockIdx.x - it.block_base);
-  if (it.g.L > kUnitLevels)
-    build_block_deep<USE_VALID, UV, ONE>(it.g, it.r, it.nodes, b);
-  else
-    build_block<USE_VALID, UV, ONE>(it.g, it.r, it.nodes, b, sBox, sVal);
-}
-template <bool USE_VALID, bool UV, bool ONE>
-__global__ __launch_bounds__(256) void rh_group_build_kernel(const RhItem* __restrict__ items,
-                                                             int nitems,
-                                                             uint32_t* __restrict__ ctr) {
-  group_build<USE_VALID, UV, ONE>(items[find_block_item(items, nitems, blockIdx.x)], ctr);
-}
-// The same for a single job whose table entry comes with the launch; the first work-group leaves
-// it in `table` for the kernels that follow.  A renderer whose buffers change from call to call
-// thus uploads nothing: the copy (3.5 us), its event and the wait for the one before are gone.
-template <bool USE_VALID, bool UV, bool ONE>
-__global__ __launch_bounds__(256) void rh_single_build_kernel(const RhItem it,
-                                                              RhItem* __restrict__ table,
-                                                              uint32_t* __restrict__ ctr) {
-  if (blockIdx.x == 0) {
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(&it);
-    for (uint32_t i = threadIdx.x; i < sizeof(RhItem) / 4; i += kThreads)
-      reinterpret_cast<uint32_t*>(table)[i] = src[i];
-  }
-  group_build<USE_VALID, UV, ONE>(it, ctr);
 }
 
 // Clears the reduction state of every job: keys, repair keys, occlusion flags, counters.
@@ -540,6 +518,7 @@ __device__ __forceinline__ void load_subtree(const RHGeom& g, int K, int J, P no
 //            chain; the tests of verified pairs update the ray (LDS atomic min of the (t, id)
 //            key / occlusion bit).
 constexpr int kCluster = 64;     // triangles per cluster
+constexpr float kIncoherent = 0.25f;  // mean direction spread of an incoherent block's leaves
 constexpr uint32_t kNoUnit = 0xffffffffu;  // no unit left in the queue
 constexpr int kQ0Cap = 1024;     // root survivors held before expansion
 constexpr int kQCap = 1024;      // survivors of one expansion round
@@ -859,7 +838,6 @@ __device__ __forceinline__ void expand_queue(const RHGeom& g, PF v9s, P4 tbox, P
 // traced ray that way without scanning the clusters, and so does a block of more than
 // kMaxBlockRays rays or kUnitLevels levels (the unit kernels stage at most that much; the
 // reference's own scenes use such blocks, e.g. 100x4 leaves at height 3 or 4).
-constexpr float kIncoherent = 0.25f;
 template <int MODE, int NODE, bool BVH>
 __global__ __launch_bounds__(256) void rh_cluster_kernel(const RhItem* __restrict__ items,
                                                          int nitems, uint4* __restrict__ ustage,
@@ -1735,6 +1713,591 @@ __device__ __forceinline__ bool ray_chain_bvh(const RhItem& it, int x, int y, ui
   return true;
 }
 
+// ---------------------------------------------------------------------------------------
+// Grazing pass.  The per-ray path's tree does not find every strict hit of a ray that runs close
+// to a triangle's plane (rt_search.h).  For coherent blocks, where one plane can hold many rays
+// (a wall seen edge on, a light in the plane of a wall), a work-group therefore looks for the
+// triangles that a ray of the block may graze and tests them directly:
+//   - clusters are bounded against the block root as the cluster pass does (what the reference
+//     cannot reach through its cull chain is left out), 64 of them at a time by their common box
+//     first, and by the range of their triangles' planes;
+//   - the triangles of the clusters left are asked whether any ray of the block may graze them:
+//     by their angle, 16 bytes a triangle, and those left, compacted, by the distance of their
+//     plane and their place, with intervals over the block's origins, far ends and directions
+//     (camera rays have one origin, shadow rays toward a light nearly one far end), and bounded
+//     against the block root themselves;
+//   - every ray asks for its own angle (in a long list, every 16 rays all the questions first),
+//     and takes the strict test of what is left and then the exact cull chain.
+// A block whose rays lie far apart (the horizon of a ground plane) lists many triangles that
+// hardly any of its rays can graze, and the launch lasted as long as it: one work-group gives such
+// a block up and queues it, and a second launch takes it by kGrazeSlices work-groups, each with
+// its share of the clusters.
+// Hits found here are verified; they go into the ray's seed (closest) or its flag (occlusion),
+// and the per-ray kernel starts from them.
+// The build marks the blocks to look at (gblock 1): not incoherent ones (kIncoherent), whose
+// intervals exclude nothing, unless the scene is tiny (kGrazeAll), nor blocks of more than kMaxBlockRays rays or kUnitLevels levels.
+// Occlusion blocks whose root passes many clusters of a large scene (kHeavy) are left out here.
+constexpr int kGrazeSecond = 1024;  // work-groups of the second launch
+constexpr int kGrazeGrid = 4096;    // work-groups at most; each takes every kGrazeGrid-th block
+constexpr int kGrazeAhead = 2;      // chunks of 64 records loaded at a time
+constexpr int kGrazeRound = 128;    // records that a wavefront lists by angle before the next step
+constexpr int kGrazeBatch = 128;    // listed triangles tested at a time
+constexpr int kGrazeFew = 48;       // the length of a long list
+constexpr int kGrazeSlices = 16;    // work-groups to a queued block
+constexpr uint32_t kGrazeAll = 128;  // triangles that every ray can test: incoherent blocks too
+constexpr uint32_t kGrazeMany = 192;  // listed triangles that queue a block
+template <int WAVES>
+struct GrazeShared {
+  static constexpr int kNear = WAVES * (kGrazeRound + 64 * kGrazeAhead);
+  static constexpr int kList = 512 + kNear;
+  float box[kMaxBlockRays / 16][20];  // per 16 rays: ends of origin, far end, direction; dmin
+  GrazeRays rays[kMaxBlockRays / 16];
+  GrazeRays all;
+  uint32_t near[kNear];            // records that pass by their angle
+  uint32_t tri[kList];             // records that pass for the block
+  // the batch at hand: GrazeNormal, RhItem::gtest, and in a long list GrazeTri
+  float4 N[kGrazeBatch], T[kGrazeBatch][3], G[kGrazeBatch][3];
+  int nnear, ntri, any, passed, marked;
+};
+
+// A ray's seed: its key, bit 31 inverted when a repair-region hit lies at exactly tmin.
+__device__ __forceinline__ uint64_t seed_pack(uint64_t key, bool mark) {
+  return key ^ (mark ? 0x80000000ull : 0ull);
+}
+__device__ __forceinline__ void seed_unpack(uint64_t s, uint64_t& key, bool& mark) {
+  mark = ((s >> 31) & 1u) != ((uint32_t)(s >> 32) == 0xffffffffu ? 1u : 0u);
+  key = seed_pack(s, mark);
+}
+template <int M>
+__device__ __forceinline__ float min_group(float v) {
+  return fminf(v, __int_as_float(from_group<M>(__float_as_int(v))));
+}
+__device__ __forceinline__ float min_row(float v) {  // over the 16 lanes of a row
+  return min_group<8>(min_group<4>(min_group<2>(min_group<1>(v))));
+}
+__device__ __forceinline__ GrazeTri load_graze(const GrazeTri* p, size_t i) {
+  const auto q = (RT_GLOBAL const float4*)p;
+  const float4 a = ld4(q, 3 * i), b = ld4(q, 3 * i + 1), c = ld4(q, 3 * i + 2);
+  return GrazeTri{{a.x, a.y, a.z}, a.w, b.x, b.y, __float_as_uint(b.z), b.w, {c.x, c.y, c.z}, c.w};
+}
+
+template <int MODE, int NODE, bool BVH, int WAVES>
+__device__ __forceinline__ bool graze_block(const RhItem& it, int b, int slice, int slices,
+                                            GrazeShared<WAVES>& sh) {
+  constexpr int kWork = 64 * WAVES;
+  const uint32_t mates = (uint32_t)(WAVES * slices);  // wavefronts at the block
+  const RHGeom& g = it.g;
+  const RaysDev& r = it.r;
+  const SearchFrame frame = it.sframe;
+  const float4 *const cbox = it.cbox, *const gbox = it.gbox;
+  const GrazeCluster* const gcluster = it.gcluster;
+  const GrazeNormal* const gnormal = it.gnormal;
+  const uint32_t* const gfirst = it.gfirst;
+  const uint32_t ntri = it.ntri;
+  const float inf = __int_as_float(0x7f800000);
+  const int tid = threadIdx.x, lane = __lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int top = g.L - 1;
+  const int K = b % g.gw[top], J = b / g.gw[top];
+  const int rows = (g.rb + 15) / 16;
+  if (tid == 0) sh.nnear = sh.ntri = sh.any = sh.passed = sh.marked = 0;
+  // the boxes of every 16 rays, lower ends and negated upper ends
+#pragma unroll 1
+  for (int s0 = wave * 64; s0 < g.rb; s0 += kWork) {
+    float v[19];
+    int x = 0, y = 0, leaf = 0;
+    bool in = slot_xy(g, K, J, s0 + lane, x, y, leaf);
+    const size_t i = in ? (size_t)y * g.W + x : 0;
+    const V3 o = {glb(r.ox)[i], glb(r.oy)[i], glb(r.oz)[i]};
+    const V3 d = {glb(r.dx)[i], glb(r.dy)[i], glb(r.dz)[i]};
+    const float tm = glb(r.tmax)[i], s = tm < inf ? tm : 1.f;
+    if (MODE != 0 && r.valid != nullptr) in = in && glb(r.valid)[i] != 0;
+    // a ray that is not finite passes no test
+    in = in && fabsf(o.x) < inf && fabsf(o.y) < inf && fabsf(o.z) < inf && fabsf(d.x) < inf &&
+         fabsf(d.y) < inf && fabsf(d.z) < inf;
+    const float p[9] = {o.x, o.y, o.z, o.x + s * d.x, o.y + s * d.y, o.z + s * d.z,
+                        d.x, d.y, d.z};
+    for (int c = 0; c < 9; ++c) {
+      v[6 * (c / 3) + c % 3] = in ? p[c] : inf;
+      v[6 * (c / 3) + 3 + c % 3] = in ? -p[c] : inf;
+    }
+    v[18] = in ? fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z)) : inf;
+    for (int c = 0; c < 19; ++c) v[c] = min_row(v[c]);
+    if ((lane & 15) == 0)
+      for (int c = 0; c < 19; ++c) sh.box[(s0 + lane) / 16][c] = v[c];
+  }
+  __syncthreads();
+  auto rays_of = [&](const float* v) {
+    float hi[9];
+    for (int c = 0; c < 9; ++c) hi[c] = -v[6 * (c / 3) + 3 + c % 3];
+    return graze_rays(v, hi, v + 6, hi + 3, v + 12, hi + 6, v[18], frame);
+  };
+  if (wave == 0) {
+    float m = inf, v[19];
+    if (lane < 19)
+      for (int q = 0; q < rows; ++q) m = fminf(m, sh.box[q][lane]);
+    for (int c = 0; c < 19; ++c)
+      v[c] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m), c));
+    const GrazeRays a = rays_of(v);
+    if (lane == 0) sh.all = a;
+  }
+  const RT_GLOBAL float4* const p =
+      glb(it.nodes) + 4 * ((size_t)g.off[top] + (size_t)J * g.gw[top] + K);
+  Node root;
+  {
+    const float4 a0 = ld4(p, 0), a1 = ld4(p, 1), a2 = ld4(p, 2), a3 = ld4(p, 3);
+    root.dmin = {a0.x, a0.y, a0.z};
+    root.dmax = {a1.x, a1.y, a1.z};
+    root.omin = {a2.x, a2.y, a2.z};
+    root.omax = {a3.x, a3.y, a3.z};
+  }
+  __syncthreads();
+  GrazeRays all = sh.all;
+  {  // uniform: to scalar registers
+    auto scalar = [](float& q) { q = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(q))); };
+    for (F3* q : {&all.oc, &all.oh, &all.qc, &all.qh, &all.dc, &all.dh}) {
+      scalar(q->x);
+      scalar(q->y);
+      scalar(q->z);
+    }
+    for (float* q : {&all.dist, &all.far, &all.dir, &all.extra}) scalar(*q);
+    all.all = __builtin_amdgcn_readfirstlane((int)all.all) != 0;
+    for (V3* q : {&root.dmin, &root.dmax, &root.omin, &root.omax}) {
+      scalar(q->x);
+      scalar(q->y);
+      scalar(q->z);
+    }
+  }
+  // what a record's slope is multiplied by (GrazeNormal)
+  const float steep = graze_steep(all, frame);
+  auto box_passes = [&](const float4* box, uint32_t k) {
+    const float4 lo = ld4(glb(box), 2 * (size_t)k), hi = ld4(glb(box), 2 * (size_t)k + 1);
+    return cluster_bound<MODE, NODE, BVH>(root, V3{lo.x, lo.y, lo.z}, V3{hi.x, hi.y, hi.z});
+  };
+  // The same for one triangle.  ray-bvh: its reference BVH leaf meets the ray's hierarchy leaf,
+  // not the root; a cluster's bound over the root's rays holds for every node below it if its
+  // box covers the roundings of their centres and half widths.
+  auto root_passes = [&](uint32_t id) {
+    const Tri T = load_tri(glb(it.v9), id);
+    if constexpr (!BVH) {
+      return cull_bound<MODE, NODE>(root, T);
+    } else {
+      const uint32_t leaf = glb(it.tleaf)[id];
+      if (leaf == 0xffffffffu) return false;
+      V3 mn, mx;
+      uint32_t off, np;
+      bvh_box(glb(it.bvh), leaf & 0x7fffffffu, mn, mx, off, np);
+      if constexpr (NODE != 1) {
+        auto slack = [](float a0, float a1, float c0, float c1) {
+          return 0x1p-20f * (fmaxf(fabsf(a0), fabsf(a1)) + fmaxf(fabsf(c0), fabsf(c1)));
+        };
+        const V3 w = {slack(mn.x, mx.x, root.omin.x, root.omax.x),
+                      slack(mn.y, mx.y, root.omin.y, root.omax.y),
+                      slack(mn.z, mx.z, root.omin.z, root.omax.z)};
+        mn = sub(mn, w);
+        mx = add(mx, w);
+      }
+      return cluster_bound<MODE, NODE, BVH>(root, mn, mx);
+    }
+  };
+  // the wavefront's share of the clusters: one in `mates` of the groups of 64 that pass, or in
+  // small scenes of the clusters
+  const uint32_t nclusters = it.nclusters, ngroups = (nclusters + 63u) / 64u;
+  const uint32_t mate = (uint32_t)(slice * WAVES + wave);
+  const bool by_cluster = ngroups <= mates / 2;
+  uint32_t gbase = 0, group = 0, turn = 0, pos = 0, end = 0;
+  uint64_t gmask = 0, cmask = 0;
+  bool fresh = true;
+  // whether enough clusters pass decides first: a round that only counts
+  const uint32_t enough = BVH ? kHeavyBvh : kHeavy;
+  bool count = MODE == 2 && slices == 1 && nclusters >= 4u * enough;
+  int passed = 0;
+  auto next_chunk = [&]() {  // up to 64 records from pos
+#pragma unroll 1
+    for (;;) {
+      if (pos < end) return true;
+      if (cmask != 0) {
+        const uint32_t c = group * 64u + (uint32_t)__ffsll((unsigned long long)cmask) - 1u;
+        cmask &= cmask - 1;
+        if (by_cluster && turn++ % mates != mate) continue;
+        pos = gfirst ? glb(gfirst)[c] : c * (uint32_t)kCluster;
+        end = gfirst ? glb(gfirst)[c + 1]
+                        : min(c * (uint32_t)kCluster + (uint32_t)kCluster, ntri);
+        continue;
+      }
+      // the next group of clusters that passes, or (gmask empty) the next 64 groups
+      const bool inner = gmask != 0;
+      if (inner) {
+        group = gbase + (uint32_t)__ffsll((unsigned long long)gmask) - 1u;
+        gmask &= gmask - 1;
+        if (!by_cluster && turn++ % mates != mate) continue;
+      } else {
+        gbase = fresh ? 0u : gbase + 64u;
+        fresh = false;
+        if (gbase >= ngroups) return false;
+        if (ngroups == 1u) {  // its clusters say as much
+          gmask = 1u;
+          continue;
+        }
+      }
+      const uint32_t q = (inner ? group * 64u : gbase) + (uint32_t)lane;
+      const bool exists = q < (inner ? nclusters : ngroups);
+      float4 a0{}, a1{}, a2{};
+      if (exists && inner) {
+        const auto w = (RT_GLOBAL const float4*)gcluster;
+        a0 = ld4(w, 3 * (size_t)q);
+        a1 = ld4(w, 3 * (size_t)q + 1);
+        a2 = ld4(w, 3 * (size_t)q + 2);
+      }
+      const bool ok = exists && box_passes(inner ? cbox : gbox, q);
+      if (!inner) {
+        gmask = __ballot(ok);
+        continue;
+      }
+      if (count) {
+        passed += __popcll(__ballot(ok));
+        continue;
+      }
+      cmask = __ballot(ok && grazes_cluster(all, GrazeCluster{{a0.x, a0.y, a0.z}, a0.w,
+                                                              {a1.x, a1.y, a1.z}, a1.w, a2.x,
+                                                              a2.y, a2.z, 0.f}, frame));
+    }
+  };
+  bool first = true;
+  // the rays' tests against the listed triangles; empties the list
+  auto flush = [&]() {
+    const int n = sh.ntri;
+    const bool ask = n > kGrazeFew;
+    if (ask && tid < rows) sh.rays[tid] = rays_of(sh.box[tid]);
+    const bool init = first && slices == 1;
+    first = false;
+#pragma unroll 1
+    for (int base = 0; base < n; base += kGrazeBatch) {
+      const int m = min(n - base, kGrazeBatch);
+      for (int e = tid; e < 4 * m; e += kWork) {
+        const size_t rec = sh.tri[base + (e >> 2)];
+        if ((e & 3) == 3) sh.N[e >> 2] = ld4((RT_GLOBAL const float4*)gnormal, rec);
+        else sh.T[e >> 2][e & 3] = ld4((RT_GLOBAL const float4*)it.gtest, 3 * rec + (e & 3));
+        if (ask && (e & 3) != 3)
+          sh.G[e >> 2][e & 3] = ld4((RT_GLOBAL const float4*)it.graze, 3 * rec + (e & 3));
+      }
+      __syncthreads();
+      // 16 rays at a time, four lanes a ray
+#pragma unroll 1
+      for (int row = wave; row < rows; row += WAVES) {
+        const int slot = row * 16 + (lane & 15), sub = lane >> 4;
+        int x = 0, y = 0, hleaf = 0;
+        bool alive = slot_xy(g, K, J, slot, x, y, hleaf);
+        const size_t i = alive ? (size_t)y * g.W + x : 0;
+        const V3 o = {glb(r.ox)[i], glb(r.oy)[i], glb(r.oz)[i]};
+        const V3 d = {glb(r.dx)[i], glb(r.dy)[i], glb(r.dz)[i]};
+        const float tmin = glb(r.tmin)[i], tmax = MODE == 2 ? glb(r.tmax)[i] : inf;
+        if (MODE != 0 && r.valid != nullptr) alive = alive && glb(r.valid)[i] != 0;
+        const bool fresh_ray = init && base == 0;
+        uint64_t best = kMissKey;
+        bool mark = false, found = false;
+        if (alive && !fresh_ray) {
+          if (MODE == 2) found = glb(it.occ)[i] != 0;
+          else if (slices > 1) best = __hip_atomic_load(&it.gseed[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          else seed_unpack(glb(it.gseed)[i], best, mark);
+        }
+        const uint64_t best0 = best;
+        float len, dist;
+        graze_ray(F3{o.x, o.y, o.z}, F3{d.x, d.y, d.z}, frame, len, dist);
+#pragma unroll 1
+        for (int e0 = 0; e0 < m; e0 += 64) {
+          const int k = min(m - e0, 64);
+          uint64_t todo = k < 64 ? (1ull << k) - 1ull : ~0ull;
+          if (ask) {
+            bool ok = false;
+            if (lane < k) {
+              const float4 a = sh.G[e0 + lane][0], c1 = sh.G[e0 + lane][1], c2 = sh.G[e0 + lane][2];
+              ok = grazes(sh.rays[row],
+                          GrazeTri{{a.x, a.y, a.z}, a.w, c1.x, c1.y, __float_as_uint(c1.z), c1.w,
+                                   {c2.x, c2.y, c2.z}, c2.w}, frame);
+            }
+            todo &= __ballot(ok);
+          }
+          todo &= 0x1111111111111111ull << sub;
+          if (!alive || (MODE == 2 && found)) todo = 0;
+          // lanes go on to their next hit, whose chains are then evaluated together
+#pragma unroll 1
+          while (__any(todo != 0)) {
+            uint32_t id = 0, leaf = 0;
+            uint64_t key = kMissKey;
+            bool um = false, rp = false;
+#pragma unroll 1
+            for (; todo != 0 && !um && !rp; todo &= todo - 1) {
+              const int j = e0 + __ffsll((unsigned long long)todo) - 1;
+              const float4 q = sh.N[j], tc = sh.T[j][2];
+              // the ray's own angle
+              if (graze_clears(GrazeNormal{{q.x, q.y, q.z}, q.w}, tc.w, F3{d.x, d.y, d.z}, len,
+                               dist))
+                continue;
+              const float4 ta = sh.T[j][0], tb = sh.T[j][1];
+              Tri S;
+              S.v1 = {ta.x, ta.y, ta.z};
+              S.e1 = {ta.w, tb.x, tb.y};
+              S.e2 = {tb.z, tb.w, tc.x};
+              S.v2 = S.v3 = S.v1;
+              float t, b1, b2;
+              if (!mt_strict(o, d, S, t, b1, b2)) continue;
+              id = __float_as_uint(tc.y);
+              leaf = __float_as_uint(tc.z);
+              // in no leaf; or not its leaf's first primitive (6DB / IA secondary rays)
+              if (BVH && (leaf == 0xffffffffu ||
+                          (MODE == 1 && NODE != 2 && (leaf & 0x80000000u))))
+                continue;
+              key = hit_key(t, (int32_t)id);
+              um = t > tmin && t < tmax && (MODE == 2 || key < best);
+              rp = MODE == 0 && !BVH && it.repair_run > 0 && !mark && t == tmin &&
+                   repair_region(b1, b2);
+            }
+            bool ok = um || rp;
+            if (ok) {
+              // most that fail do so in the ray's leaf, which its bound tells for less
+              Node nd;
+              ok = chain_node(it.g, glb(it.nodes), x, y, 0, nd);
+              if constexpr (BVH) {
+                V3 mn, mx;
+                uint32_t off, np;
+                bvh_box(glb(it.bvh), leaf & 0x7fffffffu, mn, mx, off, np);
+                ok = ok && bvh_bound<NODE>(nd, mn, mx) &&
+                     ray_chain_bvh<NODE>(it, x, y, leaf & 0x7fffffffu);
+              } else {
+                ok = ok && cull_bound<MODE, NODE>(nd, load_tri(glb(it.v9), id)) &&
+                     ray_chain_rh<MODE, NODE>(it, x, y, id);
+              }
+            }
+            if (!ok) continue;
+            found = true;
+            if (MODE == 2) todo = 0;
+            if (um) best = key;
+            if (rp) mark = true;
+          }
+        }
+        // the four lanes' results together
+        for (int c = 16; c < 64; c <<= 1) {
+          const uint64_t q = ((uint64_t)(uint32_t)__shfl_xor((int)(uint32_t)(best >> 32), c) << 32) |
+                             (uint32_t)__shfl_xor((int)(uint32_t)best, c);
+          best = q < best ? q : best;
+          mark = __shfl_xor((int)mark, c) != 0 || mark;
+          found = __shfl_xor((int)found, c) != 0 || found;
+        }
+        if (slices > 1) {  // others are at the ray too
+          if (alive && sub == 0 && found) {
+            if (MODE == 2) glb(it.occ)[i] = 1;
+            else atomicMin((unsigned long long*)&it.gseed[i], (unsigned long long)best);
+            if (mark) sh.marked = 1;
+          }
+        } else if (alive && sub == 0 && (found || fresh_ray)) {
+          if (MODE == 2) glb(it.occ)[i] = found ? 1 : 0;
+          else glb(it.gseed)[i] = seed_pack(best, mark);
+        }
+        if (__any(found && (MODE == 2 || best != best0 || mark)) && lane == 0) sh.any = 1;
+      }
+      __syncthreads();
+    }
+    if (tid == 0) sh.ntri = 0;
+    __syncthreads();
+  };
+  uint32_t listed = 0, kept = 0;
+  // Rounds: the wavefronts list the records of their share by angle, up to kGrazeRound and one
+  // load each, and then share out the list for the other questions.
+  bool done = false;
+#pragma unroll 1
+  for (;;) {
+#pragma unroll 1
+    for (int added = 0; !done && added < kGrazeRound;) {
+      // chunk u's ends in lane u
+      uint32_t from = 0, to = 0;
+#pragma unroll 1
+      for (int u = 0; u < kGrazeAhead && !done; ++u) {
+        done = !next_chunk();
+        if (!done && lane == u) {
+          from = pos;
+          to = end;
+        }
+        pos += 64u;
+      }
+      float4 q[kGrazeAhead];
+      uint32_t at[kGrazeAhead];
+      uint64_t m[kGrazeAhead];
+      bool in[kGrazeAhead];
+#pragma unroll
+      for (int u = 0; u < kGrazeAhead; ++u) {
+        at[u] = __builtin_amdgcn_readlane(from, u) + (uint32_t)lane;
+        in[u] = at[u] < (uint32_t)__builtin_amdgcn_readlane(to, u);
+        if (in[u]) q[u] = ld4((RT_GLOBAL const float4*)gnormal, at[u]);
+      }
+      int cnt = 0;
+#pragma unroll
+      for (int u = 0; u < kGrazeAhead; ++u) {
+        m[u] = __ballot(in[u] && grazes_angle(all, steep, GrazeNormal{{q[u].x, q[u].y, q[u].z},
+                                                                      q[u].w}));
+        cnt += __popcll(m[u]);
+      }
+      if (cnt == 0) continue;
+      int base = 0;
+      if (lane == 0) base = atomicAdd(&sh.nnear, cnt);
+      base = __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+      for (int u = 0; u < kGrazeAhead; ++u) {
+        if ((m[u] >> lane) & 1u) sh.near[base + __popcll(m[u] & ((1ull << lane) - 1ull))] = at[u];
+        base += __popcll(m[u]);
+      }
+      added += cnt;
+    }
+    if (count) {  // uniform; by_cluster: every wavefront has counted all of them
+      if (lane == 0) atomicAdd(&sh.passed, passed);
+      __syncthreads();
+      if ((uint32_t)sh.passed >= enough * (by_cluster ? (uint32_t)WAVES : 1u)) break;
+      count = done = false;
+      fresh = true;
+      turn = 0;
+      continue;
+    }
+    const bool more = __syncthreads_or(!done) != 0;
+    const int nnear = sh.nnear;
+    listed += (uint32_t)nnear;
+#pragma unroll 1
+    for (int e = wave * 64; e < nnear; e += kWork) {
+      bool ok = false;
+      uint32_t k = 0;
+      if (e + lane < nnear) {
+        k = sh.near[e + lane];
+        const GrazeTri q = load_graze(it.graze, k);
+        ok = grazes(all, q, frame) && root_passes(q.id);
+      }
+      const uint64_t m = __ballot(ok);
+      if (m == 0) continue;
+      int base = 0;
+      if (lane == 0) base = atomicAdd(&sh.ntri, __popcll(m));
+      base = __builtin_amdgcn_readfirstlane(base);
+      if (ok) sh.tri[base + __popcll(m & ((1ull << lane) - 1ull))] = k;
+    }
+    __syncthreads();
+    if (tid == 0) sh.nnear = 0;
+    if (slices == 1) {  // uniform
+      kept += (uint32_t)sh.ntri;
+      if (kept > kGrazeMany || listed > kGrazeMany * 16u + 64u * ngroups) {
+        // to the second launch; no ray has a hit yet
+        for (int slot = tid; slot < g.rb; slot += kWork) {
+          int x = 0, y = 0, leaf = 0;
+          if (!slot_xy(g, K, J, slot, x, y, leaf)) continue;
+          const size_t i = (size_t)y * g.W + x;
+          if (MODE == 2) glb(it.occ)[i] = 0;
+          else glb(it.gseed)[i] = kMissKey;
+        }
+        if (tid == 0) glb(it.gblock)[b] = 1u;
+        return false;
+      }
+    }
+    if (sh.ntri > (more ? sh.kList - sh.kNear : 0)) flush();
+    if (!more) break;
+    __syncthreads();
+  }
+  // a repair-region hit of some ray in a slice: all rays of the block count as having one, which
+  // only sends them through the repair pass
+  if (tid == 0 && sh.any != 0) {
+    if (slices == 1) glb(it.gblock)[b] = kGrazeHit;
+    else atomicMax(&it.gblock[b], MODE == 0 && sh.marked != 0 ? kGrazeMark : kGrazeHit);
+  }
+  return true;
+}
+
+// heavy: the blocks queued for the second launch, their number in ctr[5].  slices: work-groups to a
+// block; 1 in the first launch.  queued: only the blocks in `heavy`.
+template <int MODE, int NODE, bool BVH, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4))) void
+rh_graze_kernel(const RhItem* __restrict__ items, int nitems, uint32_t nblocks,
+                uint32_t* __restrict__ ctr, uint32_t* __restrict__ heavy, uint32_t slices,
+                bool queued) {
+  __shared__ GrazeShared<WAVES> sh;
+  const uint32_t n = (queued ? __builtin_amdgcn_readfirstlane(ctr[5]) : nblocks) * slices;
+  for (uint32_t i0 = 0; i0 * gridDim.x + blockIdx.x < n; i0 += 64) {
+    // lane u: the work-group's block (or slice) number i0 + u
+    const uint64_t at = (uint64_t)(i0 + (uint32_t)__lane_id()) * gridDim.x + blockIdx.x;
+    bool look = at < n;
+    if (look && !queued) {
+      const uint32_t gb = (uint32_t)at / slices;
+      const RhItem& it = items[find_block_item_lane(items, nitems, gb)];
+      look = it.gblock != nullptr && glb(it.gblock)[gb - it.block_base] != 0u;
+    }
+    for (uint64_t m = __ballot(look); m != 0; m &= m - 1) {
+      const uint32_t u =
+          (i0 + (uint32_t)__ffsll((unsigned long long)m) - 1u) * gridDim.x + blockIdx.x;
+      const uint32_t gb = queued ? __builtin_amdgcn_readfirstlane(heavy[u / slices]) : u / slices;
+      const RhItem& it = items[nitems == 1 ? 0 : find_block_item(items, nitems, gb)];
+      if (!graze_block<MODE, NODE, BVH, WAVES>(it, (int)(gb - it.block_base), (int)(u % slices),
+                                               (int)slices, sh)) {
+        if (threadIdx.x == 0) heavy[atomicAdd(&ctr[5], 1u)] = gb;
+      }
+      __syncthreads();
+    }
+  }
+}
+
+// ctr: the counters to clear for the kernels that follow (null: the init kernel does it).
+template <bool USE_VALID, bool UV, bool ONE>
+__device__ __forceinline__ void group_build(const RhItem& it, uint32_t* __restrict__ ctr) {
+  __shared__ float sBox[kMaxSub][12];
+  __shared__ int sVal[kMaxSub];
+  if (ctr != nullptr && blockIdx.x == 0) clear_counters(ctr, threadIdx.x);
+  const int b = (int)(blockIdx.x - it.block_base);
+  if (it.g.L > kUnitLevels) {
+    build_block_deep<USE_VALID, UV, ONE>(it.g, it.r, it.nodes, b);
+    return;
+  }
+  build_block<USE_VALID, UV, ONE>(it.g, it.r, it.nodes, b, sBox, sVal);
+  if (it.gblock != nullptr && threadIdx.x < 64) {
+    // whether the grazing pass looks at the block: the mean direction spread of its leaves, as in
+    // the cluster pass
+    const int lane = threadIdx.x, nleaf = it.g.nlx * it.g.nlx;
+    float sp = 0.f;
+    const bool have = lane < nleaf && sVal[it.g.nsub - nleaf + lane] != 0;
+    if (have) {
+      const float* v = sBox[it.g.nsub - nleaf + lane];
+      sp = UV ? v[4] - v[1] : fmaxf(fmaxf(v[3] - v[0], v[4] - v[1]), v[5] - v[2]);
+    }
+    for (int m = 32; m > 0; m >>= 1) sp += __shfl_xor(sp, m);
+    const int n = __popcll(__ballot(have));
+    const bool look =
+        n > 0 && it.ntri > 0 && (it.ntri <= kGrazeAll || !(sp > kIncoherent * (float)n));
+    if (lane == 0) glb(it.gblock)[b] = look ? 1u : 0u;
+    if (look && it.gsliced) {  // no ray has a hit yet
+      const int top = it.g.L - 1;
+      for (int slot = lane; slot < it.g.rb; slot += 64) {
+        int x = 0, y = 0, leaf = 0;
+        if (!slot_xy(it.g, b % it.g.gw[top], b / it.g.gw[top], slot, x, y, leaf)) continue;
+        const size_t i = (size_t)y * it.g.W + x;
+        if (it.occ != nullptr) glb(it.occ)[i] = 0;
+        else glb(it.gseed)[i] = kMissKey;
+      }
+    }
+  }
+}
+template <bool USE_VALID, bool UV, bool ONE>
+__global__ __launch_bounds__(256) void rh_group_build_kernel(const RhItem* __restrict__ items,
+                                                             int nitems,
+                                                             uint32_t* __restrict__ ctr) {
+  group_build<USE_VALID, UV, ONE>(items[find_block_item(items, nitems, blockIdx.x)], ctr);
+}
+// The same for a single job whose table entry comes with the launch; the first work-group leaves
+// it in `table` for the kernels that follow.  A renderer whose buffers change from call to call
+// thus uploads nothing: the copy (3.5 us), its event and the wait for the one before are gone.
+template <bool USE_VALID, bool UV, bool ONE>
+__global__ __launch_bounds__(256) void rh_single_build_kernel(const RhItem it,
+                                                              RhItem* __restrict__ table,
+                                                              uint32_t* __restrict__ ctr) {
+  if (blockIdx.x == 0) {
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(&it);
+    for (uint32_t i = threadIdx.x; i < sizeof(RhItem) / 4; i += kThreads)
+      reinterpret_cast<uint32_t*>(table)[i] = src[i];
+  }
+  group_build<USE_VALID, UV, ONE>(it, ctr);
+}
+
 // Compare-exchange of two sort keys.
 __device__ __forceinline__ void key_swap(uint32_t& a, uint32_t& b) {
   const uint32_t lo = min(a, b);
@@ -1864,7 +2427,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     careful = true;
     best = kMissKey;
     mark = false;
-    thi = MODE == 2 ? widened(tmax) : kInf;
+    if constexpr (MODE != 2) {  // the grazing pass's hit, which is verified
+      const RhItem& it = item(jk);
+      if (it.gblock != nullptr) {
+        const RHGeom& g = it.g;
+        const uint32_t y = idx / (uint32_t)g.W, x = idx - y * (uint32_t)g.W;
+        const uint32_t blk = y / (uint32_t)g.bh * (uint32_t)g.gw[g.L - 1] + x / (uint32_t)g.bw;
+        const uint32_t hit = glb(it.gblock)[blk];
+        if (hit == kGrazeHit) seed_unpack(glb(it.gseed)[idx], best, mark);
+        if (hit == kGrazeMark) {
+          best = glb(it.gseed)[idx];
+          mark = MODE == 0 && !BVH && it.repair_run > 0;
+        }
+      }
+    }
+    thi = MODE == 2 ? widened(tmax)
+                    : best == kMissKey ? kInf : widened(fkey_inv((uint32_t)(best >> 32)));
     sp = sb = 0;
     cur = 0u;  // interior node 0 (the root)
     pl = kDone;
@@ -1990,6 +2568,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
             got = it.ntri > 0 &&
                   (MODE == 0 || it.r.valid == nullptr || glb(it.r.valid)[idx] != 0);
             if (direct && !got) write_miss(it, idx);
+            // occluded by the grazing pass
+            if (MODE == 2 && got && it.gblock != nullptr && glb(it.gblock)[blk] == kGrazeHit)
+              got = glb(it.occ)[idx] == 0;
           }
         }
       }
@@ -2000,10 +2581,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
         d = {glb(r.dx)[idx], glb(r.dy)[idx], glb(r.dz)[idx]};
         tmin = glb(r.tmin)[idx];
         tmax = glb(r.tmax)[idx];
-        const SearchFrame& f = it.sframe;
-        slab_axis(o.x, d.x, f.base[0], f.unit, sr.ih.x, sr.cn.x, sr.cf.x);
-        slab_axis(o.y, d.y, f.base[1], f.unit, sr.ih.y, sr.cn.y, sr.cf.y);
-        slab_axis(o.z, d.z, f.base[2], f.unit, sr.ih.z, sr.cn.z, sr.cf.z);
+        sr = slab_ray(F3{o.x, o.y, o.z}, F3{d.x, d.y, d.z}, it.sframe);
         tlo = tmin - fabsf(tmin) * kSlack;
         track_rep = MODE == 0 && !BVH && it.repair_run > 0;
         const bool again = careful;
@@ -2751,6 +3329,22 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
     build(rh_group_build_kernel<MODE != 0, NODE == 2, false>,
           rh_single_build_kernel<MODE != 0, NODE == 2, false>);
   if (direct) {
+    if (G.graze) {
+      const dim3 grid(std::min<uint32_t>(G.nblocks, kGrazeGrid));
+      auto launch = [&](auto kernel, int waves) {
+        if (G.graze == 2) {  // few blocks
+          hipLaunchKernelGGL(kernel, dim3(G.nblocks * kGrazeSlices), dim3(64 * waves), 0, s, G.items,
+                             G.nitems, G.nblocks, G.ctr, G.heavy, (uint32_t)kGrazeSlices, false);
+          return;
+        }
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, s, G.items, G.nitems, G.nblocks,
+                           G.ctr, G.heavy, 1u, false);
+        hipLaunchKernelGGL(kernel, dim3(kGrazeSecond), dim3(64 * waves), 0, s, G.items, G.nitems,
+                           G.nblocks, G.ctr, G.heavy, (uint32_t)kGrazeSlices, true);
+      };
+      if (G.bvh) launch(rh_graze_kernel<MODE, NODE, true, 4>, 4);
+      else launch(rh_graze_kernel<MODE, NODE, false, 4>, 4);
+    }
   } else if (G.bvh)
     hipLaunchKernelGGL((rh_cluster_kernel<MODE, NODE, true>), dim3(G.nblocks), dim3(kThreads), 0,
                        s, G.items, G.nitems, G.ustage, G.bunits, G.rq, G.ctr, G.per_unit,
@@ -2830,6 +3424,36 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
   return hipGetLastError();
 }
 
+// See launch_graze_records.
+__global__ __launch_bounds__(256) void graze_records_kernel(
+    const float* __restrict__ v9, const uint32_t* __restrict__ order,
+    const uint32_t* __restrict__ tleaf, uint32_t n, SearchFrame frame,
+    GrazeNormal* __restrict__ normal, GrazeTri* __restrict__ out, float4* __restrict__ test) {
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t id = order[i];
+  float p[9];
+  for (int k = 0; k < 9; ++k) p[k] = v9[9 * (size_t)id + k];
+  out[i] = graze_record(p, id, frame);
+  normal[i] = graze_normal(out[i], frame);
+  const Tri T = load_tri(v9, id);
+  test[3 * (size_t)i] = make_float4(T.v1.x, T.v1.y, T.v1.z, T.e1.x);
+  test[3 * (size_t)i + 1] = make_float4(T.e1.y, T.e1.z, T.e2.x, T.e2.y);
+  test[3 * (size_t)i + 2] = make_float4(T.e2.z, __uint_as_float(id),
+                                        __uint_as_float(tleaf ? tleaf[id] : 0u),
+                                        graze_near_slope(out[i], normal[i]));
+}
+__global__ __launch_bounds__(256) void graze_clusters_kernel(const GrazeTri* __restrict__ rec,
+                                                             const uint32_t* __restrict__ first,
+                                                             uint32_t n, uint32_t nclusters,
+                                                             GrazeCluster* __restrict__ out) {
+  const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
+  if (c >= nclusters) return;
+  const uint32_t a = first ? first[c] : c * (uint32_t)kCluster;
+  const uint32_t z = first ? first[c + 1] : min(n, a + (uint32_t)kCluster);
+  out[c] = graze_cluster(rec + a, z - a);
+}
+
 // See launch_set_tleaf.
 __global__ __launch_bounds__(256) void set_tleaf_kernel(float4* __restrict__ tmts,
                                                         const uint32_t* __restrict__ tleaf,
@@ -2866,6 +3490,19 @@ void* noalloc_scratch(int device) {
   if (device < 0 || device >= kMaxDevices) return nullptr;
   std::lock_guard<std::mutex> lk(g_scratch_mu);
   return g_scratch_ptr[device];
+}
+
+hipError_t launch_graze_records(const float* v9, const uint32_t* order, const uint32_t* tleaf,
+                                uint32_t n, const uint32_t* first, uint32_t nclusters,
+                                const SearchFrame& frame, GrazeNormal* normal, GrazeTri* out,
+                                float4* test, GrazeCluster* cout, hipStream_t s) {
+  if (n)
+    hipLaunchKernelGGL(graze_records_kernel, grid1(n), dim3(kThreads), 0, s, v9, order, tleaf, n,
+                       frame, normal, out, test);
+  if (nclusters)
+    hipLaunchKernelGGL(graze_clusters_kernel, grid1(nclusters), dim3(kThreads), 0, s, out, first,
+                       n, nclusters, cout);
+  return hipGetLastError();
 }
 
 hipError_t launch_set_tleaf(float4* tmts, const uint32_t* tleaf, uint32_t ntri, hipStream_t s) {

@@ -19,7 +19,8 @@
 // centroid extent.  Binning every axis in place of the widest one alone made the per-ray kernels
 // about 4% faster on a batch of 64 cluster scenes.  Every box is the FP32 min/max of its
 // triangles' vertices grown outward by pad = 2^-11 * max(1, largest vertex coordinate
-// magnitude), which covers the rounding of the strict leaf test's hit point and of the slab test.
+// magnitude), more for thin triangles, which covers the rounding of the strict leaf test's hit
+// point and of the slab test unless the ray grazes the triangle's plane (rt_search.h).
 //
 // Collapse: a wide node starts from a binary node's two children and replaces its interior child
 // of largest area by that child's two children until it has four.  A ray loads about half as
@@ -356,35 +357,57 @@ void build_search_bvh(const float* v9, uint32_t ntri, std::vector<uint4>& nodes,
                       std::vector<uint32_t>& order, SearchFrame& frame) {
   nodes.clear();
   order.clear();
-  frame = SearchFrame{{0.f, 0.f, 0.f}, 1.f};
+  frame = SearchFrame{};
+  frame.unit = 1.f;
   if (ntri == 0) return;
   std::vector<uint32_t> bin_order(ntri);
   for (uint32_t i = 0; i < ntri; ++i) bin_order[i] = i;
   float big = 1.f;
   double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-  std::vector<Prim> prims(ntri);
   for (uint32_t i = 0; i < ntri; ++i) {
     const float* p = v9 + 9 * (size_t)i;
-    for (int k = 0; k < 3; ++k) {
-      for (int v = 0; v < 3; ++v) {
-        const float x = p[3 * v + k];
-        if (!std::isfinite(x)) continue;
-        big = std::max(big, std::fabs(x));
-        lo[k] = std::min(lo[k], (double)x);
-        hi[k] = std::max(hi[k], (double)x);
-      }
-      prims[i].box.lo[k] = std::min(std::min(p[k], p[3 + k]), p[6 + k]);
-      prims[i].box.hi[k] = std::max(std::max(p[k], p[3 + k]), p[6 + k]);
-      prims[i].c[k] = (prims[i].box.lo[k] + prims[i].box.hi[k]) * 0.5f;
+    for (int q = 0; q < 9; ++q) {
+      if (!std::isfinite(p[q])) continue;
+      big = std::max(big, std::fabs(p[q]));
+      lo[q % 3] = std::min(lo[q % 3], (double)p[q]);
+      hi[q % 3] = std::max(hi[q % 3], (double)p[q]);
     }
   }
   const float pad = std::ldexp(big, -11);
+  frame.pad = pad;
+  frame.huge = big > kGrazeHuge;
+  double half2 = 0.0;
+  for (int k = 0; k < 3; ++k) {
+    if (!(lo[k] <= hi[k])) lo[k] = hi[k] = 0.0;
+    frame.center[k] = (float)(0.5 * (lo[k] + hi[k]));
+    const double h = std::max(hi[k] - frame.center[k], frame.center[k] - lo[k]);
+    half2 += h * h;
+  }
+  std::vector<Prim> prims(ntri);
+  float widest = pad;
+  double edge2 = 0.0;
+  for (uint32_t i = 0; i < ntri; ++i) {
+    const float* p = v9 + 9 * (size_t)i;
+    const float kappa = graze_record(p, i, frame).kappa;
+    const float wide = pad * (pad_grow(kappa) - 1.f);  // what nodes add to `pad` for this one
+    widest = std::max(widest, pad + wide);
+    double s1 = 0.0, s2 = 0.0;
+    for (int k = 0; k < 3; ++k) {
+      prims[i].box.lo[k] = std::min(std::min(p[k], p[3 + k]), p[6 + k]) - wide;
+      prims[i].box.hi[k] = std::max(std::max(p[k], p[3 + k]), p[6 + k]) + wide;
+      prims[i].c[k] = (prims[i].box.lo[k] + prims[i].box.hi[k]) * 0.5f;
+      s1 += ((double)p[3 + k] - p[k]) * ((double)p[3 + k] - p[k]);
+      s2 += ((double)p[6 + k] - p[k]) * ((double)p[6 + k] - p[k]);
+    }
+    if (std::isfinite(s1)) edge2 = std::max(edge2, s1);
+    if (std::isfinite(s2)) edge2 = std::max(edge2, s2);
+  }
+  frame.reach = (float)((std::sqrt(half2) + std::sqrt(edge2)) * (1.0 + 1e-6));
   // 255 units of a power of two span the padded scene from `base` on every axis
   double ext = 0.0;
   for (int k = 0; k < 3; ++k) {
-    if (!(lo[k] <= hi[k])) lo[k] = hi[k] = 0.0;
-    frame.base[k] = (float)(lo[k] - 2.0 * pad);
-    ext = std::max(ext, hi[k] - lo[k] + 4.0 * pad);
+    frame.base[k] = (float)(lo[k] - 2.0 * widest);
+    ext = std::max(ext, hi[k] - lo[k] + 4.0 * widest);
   }
   int e;
   std::frexp(ext / 255.0, &e);

@@ -14,7 +14,34 @@ struct Tree {
   std::vector<uint4> nodes;
   std::vector<uint32_t> order;
   SearchFrame frame;
+  std::vector<float> v9;
+  std::vector<GrazeTri> graze;
+  std::vector<GrazeNormal> normal;
+  std::vector<GrazeCluster> cluster;  // of 64 triangles each
 };
+
+F3 sub(F3 a, F3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
+F3 cross(F3 a, F3 b) {
+  return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
+}
+float dot(F3 a, F3 b) { return (a.x * b.x + a.y * b.y) + a.z * b.z; }
+// The strict leaf test in FP32 (intersectAllLeaves.cl:40-55), as the kernels evaluate it.
+bool strict(F3 o, F3 d, const float* p, float& t) {
+  const F3 v1 = {p[0], p[1], p[2]}, e1 = sub({p[3], p[4], p[5]}, v1),
+           e2 = sub({p[6], p[7], p[8]}, v1);
+  const F3 s = cross(d, e2);
+  const float det = dot(s, e1);
+  if (det == 0.f) return false;
+  const float inv = 1.0f / det;
+  const F3 ov = sub(o, v1);
+  const float b1 = dot(ov, s) * inv;
+  if (!(b1 > 0.f && b1 < 1.f)) return false;
+  const F3 s2 = cross(ov, e1);
+  const float b2 = dot(d, s2) * inv;
+  if (!(b2 > 0.f && (b1 + b2) < 1.f)) return false;
+  t = dot(e2, s2) * inv;
+  return true;
+}
 }  // namespace
 
 extern "C" {
@@ -22,6 +49,11 @@ extern "C" {
 void* sw_build(const float* v9, uint32_t ntri) {
   Tree* t = new Tree();
   build_search_bvh(v9, ntri, t->nodes, t->order, t->frame);
+  t->v9.assign(v9, v9 + 9 * (size_t)ntri);
+  for (uint32_t i = 0; i < ntri; ++i) t->graze.push_back(graze_record(v9 + 9 * (size_t)i, i, t->frame));
+  for (const GrazeTri& g : t->graze) t->normal.push_back(graze_normal(g, t->frame));
+  for (uint32_t i = 0; i < ntri; i += 64)
+    t->cluster.push_back(graze_cluster(&t->graze[i], std::min(64u, ntri - i)));
   return t;
 }
 void sw_free(void* h) { delete (Tree*)h; }
@@ -36,10 +68,7 @@ void sw_walk(void* h, const float* rays, uint32_t n, int all, int32_t* depth, ui
   const Tree& T = *(const Tree*)h;
   for (uint32_t i = 0; i < n; ++i) {
     const float* r = rays + 8 * (size_t)i;
-    SlabRay sr;
-    slab_axis(r[0], r[3], T.frame.base[0], T.frame.unit, sr.ih.x, sr.cn.x, sr.cf.x);
-    slab_axis(r[1], r[4], T.frame.base[1], T.frame.unit, sr.ih.y, sr.cn.y, sr.cf.y);
-    slab_axis(r[2], r[5], T.frame.base[2], T.frame.unit, sr.ih.z, sr.cn.z, sr.cf.z);
+    const SlabRay sr = slab_ray(F3{r[0], r[1], r[2]}, F3{r[3], r[4], r[5]}, T.frame);
     const float tlo = r[6] - fabsf(r[6]) * kSlack, thi = r[7] + fabsf(r[7]) * kSlack;
     if (reached) std::fill(reached, reached + T.order.size(), 0);
     std::vector<uint32_t> stack;
@@ -76,6 +105,68 @@ void sw_walk(void* h, const float* rays, uint32_t n, int all, int32_t* depth, ui
     depth[i] = (int32_t)most;
     visits[i] = nv;
     leaves[i] = nl;
+  }
+}
+
+// Every ray against every triangle.  out: strict hits inside the ray's interval; those of them
+// that the walk does not reach; those neither reached nor taken for grazing by the ray itself;
+// the same by the boxes of `group` consecutive rays; (ray, triangle) pairs taken for grazing by
+// the ray; by its group.
+void sw_grazing(void* h, const float* rays, uint32_t n, uint32_t group, uint64_t* out) {
+  const Tree& T = *(const Tree*)h;
+  const uint32_t ntri = (uint32_t)T.order.size();
+  std::vector<uint8_t> reached(ntri);
+  GrazeRays gr{};
+  for (int k = 0; k < 6; ++k) out[k] = 0;
+  auto boxes = [&](uint32_t a, uint32_t b) {
+    float lo[9], hi[9], dmin = INFINITY;
+    for (int k = 0; k < 9; ++k) {
+      lo[k] = INFINITY;
+      hi[k] = -INFINITY;
+    }
+    for (uint32_t i = a; i < b; ++i) {
+      const float* r = rays + 8 * (size_t)i;
+      const float s = r[7] < INFINITY ? r[7] : 1.f;
+      const float v[9] = {r[0], r[1], r[2], r[0] + s * r[3], r[1] + s * r[4], r[2] + s * r[5],
+                          r[3], r[4], r[5]};
+      for (int k = 0; k < 9; ++k) {
+        lo[k] = fminf(lo[k], v[k]);
+        hi[k] = fmaxf(hi[k], v[k]);
+      }
+      dmin = fminf(dmin, fmaxf(fmaxf(fabsf(r[3]), fabsf(r[4])), fabsf(r[5])));
+    }
+    return graze_rays(lo, hi, lo + 3, hi + 3, lo + 6, hi + 6, dmin, T.frame);
+  };
+  for (uint32_t i = 0; i < n; ++i) {
+    const float* r = rays + 8 * (size_t)i;
+    int32_t depth;
+    uint32_t nv, nl;
+    sw_walk(h, r, 1, 0, &depth, &nv, &nl, reached.data());
+    const GrazeRays own = boxes(i, i + 1);
+    if (i % group == 0) gr = boxes(i, std::min(i + group, n));
+    for (uint32_t j = 0; j < ntri; ++j) {
+      const bool a = grazes(own, T.graze[j], T.frame), b = grazes(gr, T.graze[j], T.frame);
+      out[4] += a;
+      out[5] += b;
+      // the quicker questions that come before: by angle, and by the cluster's planes
+      float len, dist;
+      const F3 o = {r[0], r[1], r[2]}, d = {r[3], r[4], r[5]};
+      graze_ray(o, d, T.frame, len, dist);
+      const bool qa =
+          a && grazes_angle(own, graze_steep(own, T.frame), T.normal[j]) &&
+          !graze_clears(T.normal[j], graze_near_slope(T.graze[j], T.normal[j]), d, len, dist) &&
+          grazes_cluster(own, T.cluster[j / 64], T.frame);
+      const bool qb = b && grazes_angle(gr, graze_steep(gr, T.frame), T.normal[j]) &&
+                      grazes_cluster(gr, T.cluster[j / 64], T.frame);
+      float t;
+      if (!strict(o, d, &T.v9[9 * (size_t)j], t)) continue;
+      if (!(t > r[6] && t < r[7])) continue;
+      ++out[0];
+      if (reached[j]) continue;
+      ++out[1];
+      out[2] += !qa;
+      out[3] += !qb;
+    }
   }
 }
 
