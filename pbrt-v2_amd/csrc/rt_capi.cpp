@@ -129,6 +129,7 @@ struct rt_scene {
   uint32_t ntri = 0;
   float* d_v9 = nullptr;
   float* d_uv6 = nullptr;
+  uint64_t* d_merge = nullptr;  // naive: scratch of calls that share out the triangles
   // traversal copy for rayhierarchy: Morton-sorted triangles in clusters of 64
   float* d_v9s = nullptr;
   uint32_t* d_perm = nullptr;
@@ -809,6 +810,8 @@ int rt_scene_create(rt_ctx* ctx, const float* v9, const float* uv6, uint32_t ntr
       if (e == hipSuccess) e = graze_setup(s, s->d_perm, ntri, cbox);
     }
   }
+  if (e == hipSuccess && desc->kind == RT_ACCEL_NAIVE && ntri >= kNaiveSplit)
+    e = hipMalloc((void**)&s->d_merge, sizeof(uint64_t) * kNaiveMerge);
   if (e == hipSuccess && desc->kind == RT_ACCEL_RAYBVH && ntri) {
     const std::vector<float4> mt = mt_operands(v9, ntri);  // original order
     e = upload(s->d_tmt, mt.data(), mt.size());
@@ -992,6 +995,7 @@ int rt_scene_destroy(rt_scene* s) {
   (void)hipSetDevice(s->ctx->device);
   (void)hipFree(s->d_v9);
   (void)hipFree(s->d_uv6);
+  (void)hipFree(s->d_merge);
   (void)hipFree(s->d_v9s);
   (void)hipFree(s->d_perm);
   (void)hipFree(s->d_cbox);
@@ -1049,8 +1053,8 @@ static int trace_impl(rt_scene* s, const rt_rays* rays, int mode, const rt_hits*
   }
   // naive brute force, or an empty scene, where every ray misses
   const auto launch = [&] {
-    return launch_naive_trace(r, mode, s->d_v9, s->d_uv6, ntri, kind == RT_ACCEL_NAIVE, out, occ,
-                              hs);
+    return launch_naive_trace(r, mode, s->d_v9, s->d_uv6, ntri, kind == RT_ACCEL_NAIVE,
+                              s->d_merge, out, occ, hs);
   };
   RT_TRY(ntri > 0 ? timed_launch(s->timer, mode, hs, launch) : launch());
   return RT_OK;
@@ -1083,10 +1087,11 @@ int rt_trace_closest_noalloc(rt_scene* s, const rt_rays* rays, int32_t mode, con
   const HitOut out{hits->id, hits->t, hits->u, hits->v, hits->dpdu, hits->dpdv};
   const int kind = s->desc.kind;
   if (kind == RT_ACCEL_NAIVE || s->ntri == 0) {
-    // naive brute force (or an empty scene) needs no scratch; the bound is the call's own
+    // naive brute force (or an empty scene) needs no more scratch than the scene's own words;
+    // the bound is the call's own
     if (align256(sizeof(uint64_t) * n) > kNoAllocScratch) return RT_ERR_TOO_LARGE;
-    RT_TRY(launch_naive_trace(r, mode, s->d_v9, s->d_uv6, s->ntri, kind == RT_ACCEL_NAIVE, out,
-                              nullptr, hs));
+    RT_TRY(launch_naive_trace(r, mode, s->d_v9, s->d_uv6, s->ntri, kind == RT_ACCEL_NAIVE,
+                              s->d_merge, out, nullptr, hs));
     return RT_OK;
   }
   // rayhierarchy / ray-bvh: one job whose blocks all take the per-ray path (the same result as

@@ -246,9 +246,14 @@ hipError_t launch_rh_group(const RhGroup& G, hipStream_t s, hipEvent_t t0, hipEv
                            hipEvent_t t1);
 // Naive brute force from rays to hit records (mode 0, 1) or occlusion flags (mode 2); without
 // triangles every ray misses.  naive_rule: shading frames as the naive kernels take them.
+// merge: kNaiveMerge keys of scratch, used where several work-groups share out the triangles;
+// scenes of under kNaiveSplit triangles need none.
+constexpr uint32_t kNaiveSplit = 6144;
+constexpr uint32_t kNaiveGroups = 1024;  // work-groups that a launch should have
+constexpr size_t kNaiveMerge = (size_t)kNaiveGroups * 8;  // fewer have 8 rays each at most
 hipError_t launch_naive_trace(const RaysDev& r, int mode, const float* v9, const float* uv6,
-                              uint32_t ntri, bool naive_rule, HitOut out, uint8_t* occ,
-                              hipStream_t s);
+                              uint32_t ntri, bool naive_rule, uint64_t* merge, HitOut out,
+                              uint8_t* occ, hipStream_t s);
 hipError_t launch_camera_rays(int W, int H, int spp, const float origin[3], float tan_half,
                               float aspect, uint32_t seed, float* ox, float* oy, float* oz,
                               float* dx, float* dy, float* dz, float* tmin, float* tmax,

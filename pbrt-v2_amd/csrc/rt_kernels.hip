@@ -24,7 +24,8 @@
 //             traverses (phases below); per-ray results are reduced in LDS and merged with
 //             global atomics;
 //   finalize  turns each ray's (t, id) key into id / t / u / v (+ dpdu, dpdv).
-// naive is one launch: a work-group has its rays' whole answer.
+// naive is one launch, in which a work-group has its rays' whole answer, or three where few rays
+// meet many triangles and several work-groups share those out (naive_shape).
 // The nearest hit is the smallest (t, id) key, so the result is deterministic (ties -> smallest
 // id).
 #include <algorithm>
@@ -2919,6 +2920,8 @@ __global__ __launch_bounds__(kNaiveThreads) void naive_kernel(RaysDev r,
                                                               const float* __restrict__ v9,
                                                               const float* __restrict__ uv6,
                                                               uint32_t ntri, int shift,
+                                                              uint32_t chunk,
+                                                              uint64_t* __restrict__ merge,
                                                               HitOut out, bool naive_rule,
                                                               uint8_t* __restrict__ occ_out) {
   constexpr bool P = MODE == 2;
@@ -2955,8 +2958,9 @@ __global__ __launch_bounds__(kNaiveThreads) void naive_kernel(RaysDev r,
     m[j] = cross(o[j], d[j]);
     dn[j] = norm_bound(norm1(d[j]));
   }
-  for (uint32_t base = 0; base < ntri; base += kNaiveTris) {
-    const uint32_t cnt = min(ntri - base, (uint32_t)kNaiveTris);
+  const uint32_t tend = min(ntri, (blockIdx.y + 1) * chunk);
+  for (uint32_t base = blockIdx.y * chunk; base < tend; base += kNaiveTris) {
+    const uint32_t cnt = min(tend - base, (uint32_t)kNaiveTris);
     __syncthreads();
     const float omax = __uint_as_float(sFar);
     for (uint32_t k = tid; k < cnt; k += kNaiveThreads)
@@ -3005,11 +3009,32 @@ __global__ __launch_bounds__(kNaiveThreads) void naive_kernel(RaysDev r,
       atomicMin((unsigned long long*)&sBest[slot + j * lanes], (unsigned long long)best[j]);
   __syncthreads();
   const size_t i = first + tid;
+  if (gridDim.y > 1) {  // naive_finish_kernel has the rest
+    if (tid < 2 * lanes && sBest[tid] != kMissKey)
+      atomicMin((unsigned long long*)&merge[i], (unsigned long long)sBest[tid]);
+    return;
+  }
   if (tid >= 2 * lanes || i >= n) return;
   if (P)
     occ_out[i] = sBest[tid] == 0 ? 1 : 0;
   else
     finalize_ray(r, v9, uv6, sBest[tid], i, out, naive_rule);
+}
+
+// Results of a naive launch whose triangles several work-groups shared out.
+template <bool P>
+__global__ __launch_bounds__(kThreads) void naive_finish_kernel(RaysDev r,
+                                                                const float* __restrict__ v9,
+                                                                const float* __restrict__ uv6,
+                                                                const uint64_t* __restrict__ merge,
+                                                                HitOut out, bool naive_rule,
+                                                                uint8_t* __restrict__ occ_out) {
+  const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x;
+  if (i >= (size_t)r.W * r.H) return;
+  if (P)
+    occ_out[i] = merge[i] == 0 ? 1 : 0;
+  else
+    finalize_ray(r, v9, uv6, merge[i], i, out, naive_rule);
 }
 
 // Hit records of every job of a closest-hit group.  Rays whose nearest repair-region
@@ -3584,24 +3609,61 @@ hipError_t launch_rh_group(const RhGroup& G, hipStream_t s, hipEvent_t t0, hipEv
 #undef RT_CALL
 }
 
-hipError_t launch_naive_trace(const RaysDev& r, int mode, const float* v9, const float* uv6,
-                              uint32_t ntri, bool naive_rule, HitOut out, uint8_t* occ,
-                              hipStream_t s) {
-  const size_t n = (size_t)r.W * r.H;
+// How a naive launch shares out rays and triangles.
+struct NaiveShape {
+  int shift = kNaiveShift;          // rays to a work-group: 2 << shift
+  uint32_t groups = 1, parts = 1;   // work-groups over the rays, over the triangles
+  uint32_t chunk = 0;               // triangles to a part
+};
+static NaiveShape naive_shape(size_t n, uint32_t ntri) {
+  NaiveShape g;
+  const auto groups = [&] { return (uint32_t)(((n - 1) >> (g.shift + 1)) + 1); };
   // Rays to a work-group: as many as leave 1,024 work-groups, four to a CU (three are resident
   // at once), and 8 at least.  4,096 triangles, 250 x 200 rays, both kernels: 512 work-groups
   // 266 us, 1,024 240, 2,048 254, 4,096 335 (every work-group stages all triangles); 128 x 128
   // rays equal.  With 128 rays always, 33 x 40 rays would leave 245 CUs idle.
-  int shift = kNaiveShift;
-  while (shift > 2 && ((n - 1) >> (shift + 1)) + 1 < 1024) --shift;
-  const dim3 grid((unsigned)(((n - 1) >> (shift + 1)) + 1));
+  while (g.shift > 2 && groups() < kNaiveGroups) --g.shift;
+  // Fewer than that, and enough triangles to pay for two launches more and the keys: as many
+  // rays to a work-group again as leave 1,024 with the triangles shared out, since a triangle
+  // is staged once for all of them.  Whole calls, shared by one work-group -> by several: 64
+  // rays, 4,500 triangles 24 -> 27 us, 6,000 28 -> 27, 20,000 76 -> 27, 200,000 767 -> 27;
+  // 1,024 rays, 20,000 triangles 80 -> 30, 200,000 724 -> 142 (with 8 rays each 224); 8,000
+  // rays, 6,000 triangles 60 -> 50, 200,000 1,548 -> 1,032 (8 rays each 1,358).  The last to
+  // arrive writing the results in the same launch took a fence a work-group, 300 us in all.
+  uint32_t parts = 1;
+  if (groups() < kNaiveGroups && ntri >= kNaiveSplit) {
+    const uint32_t most = ntri / kNaiveTris;
+    g.shift = kNaiveShift;
+    while (g.shift > 2 && (size_t)groups() * most < kNaiveGroups) --g.shift;
+    parts = std::min(most, (kNaiveGroups + groups() - 1) / groups());
+  }
+  while (g.shift > 0 && n <= ((size_t)1 << g.shift)) --g.shift;  // one group
+  g.groups = groups();
+  g.chunk = std::max((ntri + parts - 1) / parts, 1u);
+  g.parts = std::max((ntri + g.chunk - 1) / g.chunk, 1u);
+  return g;
+}
+
+hipError_t launch_naive_trace(const RaysDev& r, int mode, const float* v9, const float* uv6,
+                              uint32_t ntri, bool naive_rule, uint64_t* merge, HitOut out,
+                              uint8_t* occ, hipStream_t s) {
+  const size_t n = (size_t)r.W * r.H;
+  const NaiveShape g = naive_shape(n, ntri);
+  if (g.parts > 1)
+    hipLaunchKernelGGL(fill_kernel<uint64_t>, grid1(n), dim3(kThreads), 0, s, merge,
+                       (uint64_t)kMissKey, n);
   auto run = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(kNaiveThreads), 0, s, r, v9, uv6, ntri, shift, out,
-                       naive_rule, occ);
+    hipLaunchKernelGGL(kernel, dim3(g.groups, g.parts), dim3(kNaiveThreads), 0, s, r, v9, uv6,
+                       ntri, g.shift, g.chunk, merge, out, naive_rule, occ);
   };
   if (mode == 0) run(naive_kernel<0>);
   else if (mode == 1) run(naive_kernel<1>);
   else run(naive_kernel<2>);
+  if (g.parts > 1) {
+    auto finish = mode == 2 ? naive_finish_kernel<true> : naive_finish_kernel<false>;
+    hipLaunchKernelGGL(finish, grid1(n), dim3(kThreads), 0, s, r, v9, uv6, merge, out, naive_rule,
+                       occ);
+  }
   return hipGetLastError();
 }
 
