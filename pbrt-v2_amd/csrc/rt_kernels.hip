@@ -2364,6 +2364,11 @@ constexpr uint32_t kSplitLanes = 48;
 // triangles: any idle lane 801 us, 4 lanes 769, 8 765, 16 761, 24 781; twelve scenes 561, 523,
 // 507, 499, 494).
 constexpr uint32_t kDealLanes = 16;
+// A word of LDS that other lanes of the wavefront change by atomics.
+template <class T>
+__device__ __forceinline__ T lds_load(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
 // State of a split ray (sRay): lanes at work in bits 0..7, then a hit at exactly tmin that the
 // repair pass must see (primary), or the candidate found (occlusion).
 constexpr uint32_t kRayLanes = 255u, kRayMark = 256u;
@@ -2754,10 +2759,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
       bool last = true;
       if (split && !careful) {
         if (MODE != 2 && mark) atomicOr(&sRay[own], kRayMark);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         const uint32_t was = atomicAdd(&sRay[own], 0xffffffffu);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         last = (was & kRayLanes) == 1u && !(MODE == 2 && (was & kRayMark));
         if constexpr (MODE != 2) {
-          best = sBest[own];
+          best = lds_load(&sBest[own]);
           mark = (was & kRayMark) != 0u;
         }
       }
@@ -2816,9 +2823,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     // the other lanes' news of a split ray
     if (split && act && !careful) {
       if constexpr (MODE == 2) {
-        if (sRay[own] & kRayMark) act = false;
+        if (lds_load(&sRay[own]) & kRayMark) act = false;
       } else {
-        const uint64_t b = sBest[own];
+        const uint64_t b = lds_load(&sBest[own]);
         if (b < best) {
           best = b;
           thi = widened(fkey_inv((uint32_t)(b >> 32)));
