@@ -1590,11 +1590,11 @@ __global__ __launch_bounds__(256) void bvh_unit_kernel(const RhItem* __restrict_
 // Hit record: id, t, (u, v) and optionally dpdu/dpdv of computeDpTuTv.cl:8-91.
 // Hit record of ray i (computeDpTuTv.cl:8-91).  naive_rule: the naive kernels' inline copy of
 // that code takes the coordinate-system fallback for |det| < EPS (naive.cl:60-61,153-154)
-// where computeDpTuTv.cl:57 takes it for det == 0 only.  write_t: false leaves t as it is.
+// where computeDpTuTv.cl:57 takes it for det == 0 only.  find_t: t is the strict test's, not given.
 __device__ void write_hit(const RaysDev& r, const float* __restrict__ v9,
                           const float* __restrict__ uv6, size_t i, int32_t id, float t,
                           const HitOut& out, bool naive_rule = false,
-                          bool write_t = true) {
+                          bool find_t = false) {
   if (id < 0) {
     out.id[i] = -1;
     out.t[i] = __int_as_float(0x7f800000);
@@ -1610,13 +1610,14 @@ __device__ void write_hit(const RaysDev& r, const float* __restrict__ v9,
   const V3 o = {r.ox[i], r.oy[i], r.oz[i]};
   const V3 d = {r.dx[i], r.dy[i], r.dz[i]};
   float b1, b2;
+  if (find_t && mt_strict(o, d, T, t, b1, b2)) t = fkey_inv((uint32_t)(hit_key(t, id) >> 32));
   bary(o, d, T, b1, b2);
   float uv[6] = {0.f, 0.f, 1.f, 0.f, 1.f, 1.f};
   if (uv6)
     for (int k = 0; k < 6; ++k) uv[k] = uv6[6 * (size_t)id + k];
   const float b0 = 1 - b1 - b2;
   out.id[i] = id;
-  if (write_t) out.t[i] = t;
+  out.t[i] = t;
   out.u[i] = (b0 * uv[0] + b1 * uv[2]) + b2 * uv[4];
   out.v[i] = (b0 * uv[1] + b1 * uv[3]) + b2 * uv[5];
   if (out.dpdu || out.dpdv) {
@@ -2424,7 +2425,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     else
       return ray_chain_rh<MODE, NODE>(it, x, y, ref);
   };
-  // direct: the record of a ray that hits nothing / has hit triangle id (its t is written apart)
+  // direct: the record of a ray that hits nothing / has hit triangle id
   auto write_miss = [&](const RhItem& it, uint32_t ri) {
     if constexpr (MODE == 2) glb(it.occ)[ri] = 0;
     else write_hit(it.r, it.v9, it.uv6, ri, -1, 0.f, it.out);
@@ -2468,7 +2469,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
       if constexpr (MODE == 2) {
         if (ok) glb(it.occ)[ri] = 1;
       } else if (direct) {
-        if (ok) write_hit(it.r, it.v9, it.uv6, ri, (int32_t)ref, 0.f, it.out, false, false);
+        if (ok) write_hit(it.r, it.v9, it.uv6, ri, (int32_t)ref, 0.f, it.out, false, true);
       } else {
         // stores of one wavefront to one address keep their order
         if (!ok) glb(it.keys)[ri] = kMissKey;
@@ -2808,8 +2809,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
           sQRef[e] = MODE == 2 ? cand : (uint32_t)best;
           sQJob[e] = (uint16_t)jk;
           if constexpr (MODE != 2) {
-            if (direct) glb(it.out.t)[idx] = fkey_inv((uint32_t)(best >> 32));
-            else glb(it.keys)[idx] = best;
+            if (!direct) glb(it.keys)[idx] = best;
           }
           act = false;
         } else {

@@ -111,3 +111,22 @@ def test_trees(rt, scenes, gpu_ctx, name, accel):
         hits += int((block[0] >= 0).sum())
     assert hits > 0
     sc.close()
+
+
+@pytest.mark.parametrize("array", ["ox", "dz", "tmin", "tmax"])
+@pytest.mark.parametrize("accel", ["rayhierarchy", "ray-bvh"])
+def test_distances_over_the_rays(rt, scenes, gpu_ctx, accel, array):
+    """A ray's record is written when nothing of the ray is needed any more, so distances may
+    replace one of the rays' own arrays."""
+    v9, rays = _failing(scenes, 0.3, 64, 48)
+    dev = rt.DeviceRays.from_numpy(rays)
+    sc = rt.Scene(gpu_ctx, v9, desc=rt.default_desc(accel, node="box_uv"))
+    mode = rt.RT_CLOSEST_SECONDARY
+    apart = sc.trace_closest(dev, mode)
+    over = rt.DeviceHits.empty(dev.count)
+    over.t = getattr(dev, array)
+    sc.trace_closest(dev, mode, hits=over)
+    _same([getattr(over, k).cpu().numpy() for k in ("id", "t", "u", "v")],
+          [getattr(apart, k).cpu().numpy() for k in ("id", "t", "u", "v")], array)
+    assert (apart.id.cpu().numpy() >= 0).sum() > 100
+    sc.close()
