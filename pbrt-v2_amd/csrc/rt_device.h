@@ -86,6 +86,13 @@ __device__ __forceinline__ bool repair_region(float b1, float b2) {
   return !(b1 < kEps || b1 > kRepHi1) && !(b2 < kEps || (b1 + b2) > kRepHi2);
 }
 
+// Whether a repair-region hit of a primary ray is to be kept apart for the repair pass.  One
+// beyond tmin is a main hit too, so the nearest of them is never below the answer; only hits at
+// exactly tmin, or at an infinite distance (all that a ray of tiny direction may have), are not.
+__device__ __forceinline__ bool repair_kept(float t, float tmin) {
+  return t == tmin || t == __int_as_float(0x7f800000);
+}
+
 // Half the width of the leaf test's interval of b1, which lies around 1/2, with a margin for the
 // roundings of b1 = fl(n1 * fl(1 / div)) (2^-22 of it at most).
 template <bool P>

@@ -2052,7 +2052,7 @@ __device__ __forceinline__ bool graze_block(const RhItem& it, int b, int slice, 
                 continue;
               key = hit_key(t, (int32_t)id);
               um = t > tmin && t < tmax && (MODE == 2 || key < best);
-              rp = MODE == 0 && !BVH && it.repair_run > 0 && !mark && t == tmin &&
+              rp = MODE == 0 && !BVH && it.repair_run > 0 && !mark && repair_kept(t, tmin) &&
                    repair_region(b1, b2);
             }
             bool ok = um || rp;
@@ -2370,8 +2370,8 @@ template <class T>
 __device__ __forceinline__ T lds_load(const T* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
-// State of a split ray (sRay): lanes at work in bits 0..7, then a hit at exactly tmin that the
-// repair pass must see (primary), or the candidate found (occlusion).
+// State of a split ray (sRay): lanes at work in bits 0..7, then a hit that the repair pass must
+// see (primary, repair_kept), or the candidate found (occlusion).
 constexpr uint32_t kRayLanes = 255u, kRayMark = 256u;
 // Registers for four wavefronts per SIMD (128 VGPRs) and LDS for as many, see kSearchStack; with
 // registers for five (96, 15-30 spilled) the room task's secondary rays took 1,315 us, the torus
@@ -2405,7 +2405,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
   // tlo, thi: the interval's ends, widened; thi follows the closest bound
   float tmin = 0.f, tmax = 0.f, tlo = 0.f, thi = 0.f;
   uint64_t best = kMissKey;   // closest: the nearest hit (verified when careful)
-  bool mark = false;          // primary: a repair-region hit at exactly tmin (likewise)
+  bool mark = false;          // primary: a repair-region hit kept apart (likewise)
   uint32_t cand = 0;          // occlusion: the candidate triangle, for ray-bvh its BVH leaf
   bool track_rep = false;
   int sp = 0, sb = 0;         // the lane's stack entries [sb, sp)
@@ -2733,9 +2733,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
           }
         } else {
           const bool main = t > tmin && t < kInf;
-          // A repair-region hit beyond tmin is a main hit too, so the nearest of them is never
-          // below the answer; only one at tmin is kept apart.
-          const bool rp = track_rep && t == tmin && repair_region(b1, b2);
+          const bool rp = track_rep && repair_kept(t, tmin) && repair_region(b1, b2);
           const uint64_t key = hit_key(t, (int32_t)id);
           const bool um = main && key < best;
           if ((um || (rp && !mark)) && (!careful || chain(it, idx, id))) {

@@ -130,3 +130,25 @@ def test_distances_over_the_rays(rt, scenes, gpu_ctx, accel, array):
           [getattr(apart, k).cpu().numpy() for k in ("id", "t", "u", "v")], array)
     assert (apart.id.cpu().numpy() >= 0).sum() > 100
     sc.close()
+
+
+@pytest.mark.parametrize("scale", [1e-20, 1e-37, 2e-38])
+@pytest.mark.parametrize("node", ["box_dir", "box_uv", "ia"])
+def test_infinite_distances(rt, scenes, gpu_ctx, node, scale):
+    """Directions so short that the distance of a hit overflows: the leaf test passes, the hit is
+    no nearest one, but the repair pass takes it where a primary ray has no other."""
+    v9 = (scenes.random_triangles(300, seed=3, size=0.6) * 4).astype(np.float32)
+    rays = scenes.pinhole_rays(48, 32, origin=(0, 0, -12.0))
+    for k in ("dx", "dy", "dz"):
+        rays[k] = (rays[k] * np.float32(scale)).astype(np.float32)
+    rays["dz"][::3] *= np.float32(50)       # with scale 2e-38, some whose distances are finite
+    dev = rt.DeviceRays.from_numpy(rays)
+    sc = rt.Scene(gpu_ctx, v9, desc=rt.default_desc("rayhierarchy", node=node))
+    for mode in (0, 1):
+        print(f"[direct] infinite distances {node} {scale} mode {mode}", flush=True)
+        block = _run(rt, gpu_ctx, sc, dev, mode, rt.RAY_PATH_OFF)[0]
+        far = int(((block[0] >= 0) & np.isinf(block[1])).sum())
+        print(f"[direct] {far} at an infinite distance, {int((block[0] >= 0).sum())} hits", flush=True)
+        assert (far > 0) == (mode == 0 and scale == 2e-38)
+        _same(_run(rt, gpu_ctx, sc, dev, mode, 0)[0], block, node)
+    sc.close()
