@@ -221,8 +221,8 @@ int rt_make_bounce_rays(rt_scene *scene, const rt_rays *in, const int32_t *id, c
  *   RT_PARAM_RAY_GRID_CLOSEST / RT_PARAM_RAY_GRID_OCCLUDED: work-groups (one wavefront each)
  *   of the per-ray kernel (batches only); 0 = one per resident slot.
  *   RT_PARAM_WALK_CLOSEST / RT_PARAM_WALK_OCCLUDED: v in 1..7: a round of the per-ray kernel
- *   walks the search tree until at most 7/8, 3/4, 3/8, 1/4, 1/8, 1/16 or none (v = 1 .. 7) of
- *   its lanes still look for a leaf; 0 = the built-in 3.
+ *   walks the search tree until at most 1/2^v of its lanes still look for a leaf (7: until
+ *   none does); 0 = the built-in choice, 3/8 of the lanes, which a batch reports as 3.
  *   RT_PARAM_TILE_CLOSEST / RT_PARAM_TILE_OCCLUDED: LDS tile of the block path's unit kernel:
  *   0 = by block size (256 rays and three levels where every block fits, else 1,024 rays and
  *   four levels); 1 = the 1,024-ray tile for every block (more LDS per work-group, fewer

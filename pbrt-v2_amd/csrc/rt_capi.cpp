@@ -504,7 +504,7 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
     L.ray = (uint32_t)prm.ray[mi];
     const bool direct = L.ray == 0;  // no cluster lists, queues or keys
     L.rgrid = prm.rgrid[mi];
-    L.walk = prm.walk[mi] > 0 ? prm.walk[mi] : kDefaultWalk;
+    L.walk = prm.walk[mi];
     L.max_units = 0;
     L.max_chunks = 0;
     L.nblocks = 0;
@@ -1146,7 +1146,7 @@ int rt_trace_closest_noalloc(rt_scene* s, const rt_rays* rays, int32_t mode, con
   G.max_chunks = (uint32_t)it.g.ntop * nch;
   G.ray_clusters = 0;
   G.ray_grid = 0;
-  G.walk = kDefaultWalk;
+  G.walk = 0;
   G.single = &it;
   RT_TRY(launch_rh_group(G, hs, nullptr, nullptr, nullptr));
   return RT_OK;
@@ -1501,7 +1501,7 @@ int rt_batch_autotune(rt_batch* b, void* stream, int32_t reps) {
   };
   int st = routing();
   // stage 2: how far a round of the per-ray kernel walks before its leaf tests
-  static const int kWalk[] = {1, 2, 3, 7};
+  static const int kWalk[] = {0, 1, 2, 7};
   if (!st)
     st = autotune_stage(
         b, hs, reps, 4, [&](int c, RhParams& p) { p.walk[0] = p.walk[1] = kWalk[c]; },

@@ -186,9 +186,9 @@ struct RhGroup {
   // block with a traced ray that way without the cluster scan (job cluster lists unused)
   uint32_t ray_clusters;
   int ray_grid;  // work-groups (one wavefront each) of the per-ray kernel; 0 = resident slots
-  int walk;      // per-ray walk rounds, RT_PARAM_WALK_* 1..7
+  int walk;      // per-ray walk rounds, RT_PARAM_WALK_* (0: built-in)
 };
-constexpr int kDefaultWalk = 3;
+constexpr int kDefaultWalk = 3;  // what the built-in walk reads as, the v that it once was
 
 // Search tree of the per-ray path (see rt_search_bvh.cpp): a 4-wide tree over the triangles in
 // their own search order.  A node is one 64-byte line, 4 uint4:

@@ -2381,7 +2381,7 @@ template <int MODE, int NODE, bool BVH, bool ONE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void ray_path_kernel(
     const RhItem* __restrict__ items, int nitems, const uint2* __restrict__ rq,
     uint32_t* __restrict__ ctr, uint32_t* __restrict__ replist, uint32_t nchunks, uint32_t spread,
-    uint32_t walk16) {
+    uint32_t walk64) {
   __shared__ uint32_t sStk[kSearchStack][64];
   // candidates [0, qn) and, from the far end, rays to trace again [kChainQ - nf, kChainQ)
   __shared__ uint32_t sQIdx[kChainQ], sQRef[kChainQ];
@@ -2693,13 +2693,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
           cur = pop();
         }
       }
-      // walk on while more than walk16 / 16 of the lanes holding a ray have neither a postponed
+      // walk on while more than walk64 / 64 of the lanes holding a ray have neither a postponed
       // leaf nor finished (fewer lanes idle behind the longest walk); the others go on from
       // their node in the next round (every round walks at least one step, so each lane
       // advances)
       const uint32_t searching = (uint32_t)__popcll(
           __ballot(act && pl == kDone && cur != kDone && !(cur & kSearchLeafBit)));
-      if (16u * searching <= walk16 * (uint32_t)__popcll(__ballot(act))) break;
+      if (64u * searching <= walk64 * (uint32_t)__popcll(__ballot(act))) break;
     }
     // leaf phase: the triangle each lane holds
     bool push = false;
@@ -3330,11 +3330,11 @@ unsigned resident_grid(F kernel, uint32_t cap, int threads = kThreads) {
   return std::max(1u, std::min(n, std::max(cap, 1u)));
 }
 
-// RT_PARAM_WALK_* 1..7 as sixteenths of the lanes holding a ray.  The built-in 3 was the
+// RT_PARAM_WALK_* as 64ths of the lanes holding a ray: 1/2^v, none for 7.  The built-in 3/8 was the
 // fastest or within 2% of it on every workload measured (1 M segments: 7/8 of the lanes 856 us,
 // 3/4 775, 1/2 688, 1/4 688, 1/8 770; with the lanes of a wavefront better filled, camera rays of
 // twelve scenes 555 us at 1/2, 538 at 3/8, 527 at 1/4).
-constexpr uint32_t kWalk16[7] = {14, 12, 6, 4, 2, 1, 0};
+constexpr uint32_t kWalk64[8] = {24, 32, 16, 8, 4, 2, 1, 0};
 
 // Launch sequence of one rayhierarchy group with the mode and node type fixed.
 template <int MODE, int NODE>
@@ -3428,7 +3428,7 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
     }();
     hipLaunchKernelGGL(kernel, grid, dim3(64), 0, s, G.items, G.nitems,
                        direct ? nullptr : G.rq, G.ctr, G.replist, G.max_chunks, spread,
-                       kWalk16[std::min(std::max(G.walk, 1), 7) - 1]);
+                       kWalk64[std::min(std::max(G.walk, 0), 7)]);
   };
   if (G.nitems == 1) {
     if (G.bvh) launch_rays(ray_path_kernel<MODE, NODE, true, true>);
