@@ -633,7 +633,9 @@ def bench_plain(args, rt, scenes, torch, orc, name):
         if cnt:
             km[key] = ms / cnt
             if accel != "naive":
-                km[key + "_unit"] = sc.kernel_time(m + rt.RT_TIME_UNIT)[0] / cnt
+                unit, nu = sc.kernel_time(m + rt.RT_TIME_UNIT)
+                if nu:
+                    km[key + "_unit"] = unit / cnt
                 km[key + "_per_ray"] = sc.kernel_time(m + rt.RT_TIME_PER_RAY)[0] / cnt
     sc.set_timing(False)
     gpu_ids = hits.id.cpu().numpy()

@@ -247,8 +247,9 @@ int rt_scene_set_param(rt_scene *scene, int32_t param, int32_t value);
 /* HIP-event timing of the traversal kernels.  rt_scene_set_timing(scene, 1) starts recording
  * events around every traversal launch (and clears earlier records); rt_scene_kernel_time
  * sums the recorded launches of one mode (RT_CLOSEST_PRIMARY, RT_CLOSEST_SECONDARY, or 2 for
- * occlusion), waiting for them to finish.  mode + 3 gives only the per-ray kernel of those
- * launches, mode + 6 only the unit (block) kernel.  This is the counterpart of the reference's
+ * occlusion), waiting for them to finish: the unit (block) kernel or, with the built-in routing,
+ * the grazing pass, and the per-ray kernel.  mode + 3 gives only the per-ray kernel of those
+ * launches, mode + 6 only the unit kernel, 0 ms of 0 launches where none was launched.  This is the counterpart of the reference's
  * GPU_TIMES accounting (GPUparallel.h:18-27,528-539). */
 int rt_scene_set_timing(rt_scene *scene, int32_t enable);
 int rt_scene_kernel_time(rt_scene *scene, int32_t mode, float *total_ms, int32_t *launches);

@@ -23,6 +23,7 @@ struct Timer {
   struct Slot {
     int mode;
     bool split;  // m was recorded (rayhierarchy / ray-bvh launches)
+    bool unit;   // the unit kernel runs between a and m
     hipEvent_t a, m, b;
   };
   bool on = false;
@@ -36,10 +37,10 @@ struct Timer {
     }
   }
   // The events for the next launch of `mode`, or null when timing is off.
-  Slot* next(int mode, bool split) {
+  Slot* next(int mode, bool split, bool unit = false) {
     if (!on) return nullptr;
     if (used == slots.size()) {
-      Slot t{mode, split, nullptr, nullptr, nullptr};
+      Slot t{mode, split, unit, nullptr, nullptr, nullptr};
       if (hipEventCreate(&t.a) != hipSuccess) return nullptr;
       if (hipEventCreate(&t.m) != hipSuccess) {
         (void)hipEventDestroy(t.a);
@@ -55,6 +56,7 @@ struct Timer {
     Slot& t = slots[used++];
     t.mode = mode;
     t.split = split;
+    t.unit = unit;
     return &t;
   }
   // part 0: whole traversal, 1: the unit (block) kernel, 2: the per-ray kernel.
@@ -63,7 +65,7 @@ struct Timer {
     int32_t n = 0;
     for (size_t i = 0; i < used; ++i) {
       const Slot& t = slots[i];
-      if (t.mode != mode) continue;
+      if (t.mode != mode || (part == 1 && t.split && !t.unit)) continue;
       if (hipEventSynchronize(t.b) != hipSuccess) return RT_ERR_HIP;
       float ms = 0.f;
       hipEvent_t from = t.a, to = t.b;
@@ -392,6 +394,16 @@ hipError_t timed_launch(Timer& tm, int mode, hipStream_t st, F fn) {
   hipError_t e = fn();
   if (e == hipSuccess && t) e = hipEventRecord(t->b, st);
   return e;
+}
+
+hipError_t timed_group(Timer& tm, const RhGroup& G, hipStream_t st) {
+  RhEvents ev;
+  if (const Timer::Slot* t = tm.next(G.mode, true, G.ray_clusters > 0)) {
+    ev.trace = t->a;
+    ev.ray = t->m;
+    ev.ray_end = t->b;
+  }
+  return launch_rh_group(G, st, ev);
 }
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -1046,9 +1058,7 @@ static int trace_impl(rt_scene* s, const rt_rays* rays, int mode, const rt_hits*
     RhItem single;
     st = rh_prepare(s->ws[mode], jobs, prm, hs, groups, &changed, &single);
     if (st) return st;
-    Timer::Slot* t = s->timer.next(mode, true);
-    RT_TRY(launch_rh_group(groups[0], hs, t ? t->a : nullptr, t ? t->m : nullptr,
-                           t ? t->b : nullptr));
+    RT_TRY(timed_group(s->timer, groups[0], hs));
     return RT_OK;
   }
   // naive brute force, or an empty scene, where every ray misses
@@ -1148,7 +1158,7 @@ int rt_trace_closest_noalloc(rt_scene* s, const rt_rays* rays, int32_t mode, con
   G.ray_grid = 0;
   G.walk = 0;
   G.single = &it;
-  RT_TRY(launch_rh_group(G, hs, nullptr, nullptr, nullptr));
+  RT_TRY(launch_rh_group(G, hs, RhEvents{}));
   return RT_OK;
 }
 
@@ -1270,8 +1280,8 @@ int rt_batch_add_occluded(rt_batch* b, rt_scene* s, const rt_rays* rays, uint8_t
 static int batch_launch(rt_batch* b, const std::vector<RhGroup>& groups, hipStream_t hs,
                         bool timed) {
   for (const RhGroup& G : groups) {
-    Timer::Slot* t = timed ? b->timer.next(G.mode, true) : nullptr;
-    RT_TRY(launch_rh_group(G, hs, t ? t->a : nullptr, t ? t->m : nullptr, t ? t->b : nullptr));
+    if (timed) RT_TRY(timed_group(b->timer, G, hs));
+    else RT_TRY(launch_rh_group(G, hs, RhEvents{}));
   }
   return RT_OK;
 }
@@ -1286,17 +1296,17 @@ constexpr uint32_t kForkLateChunks = 4096;  // 64-ray chunks: 16 wavefronts on e
 static int batch_launch_forked(rt_batch* b, const std::vector<RhGroup>& groups, hipStream_t hs) {
   const size_t nside = std::min(groups.size() - 1, b->side.size());
   if (groups.size() < 2 || nside == 0) return batch_launch(b, groups, hs, false);
-  // A first group that fills the device forks after its build (the point of the event that
-  // launch_rh_group records before the traversal), so that its traversal takes the device first
+  // A first group that fills the device forks after its build and grazing pass, so that its traversal takes the device first
   // and the others' fill in behind it; forked at the start, two such traversals split the
   // device between them (twelve scenes: 838 us a step against 738).
   const bool late = groups[0].max_chunks > kForkLateChunks;
+  RhEvents fork;
+  fork.ready = b->forks[0];
   if (!late) RT_TRY(hipEventRecord(b->forks[0], hs));
-  else RT_TRY(launch_rh_group(groups[0], hs, b->forks[0], nullptr, nullptr));
+  else RT_TRY(launch_rh_group(groups[0], hs, fork));
   for (size_t k = 0; k < nside; ++k) RT_TRY(hipStreamWaitEvent(b->side[k], b->forks[0], 0));
   for (size_t gi = late ? 1 : 0; gi < groups.size(); ++gi)
-    RT_TRY(launch_rh_group(groups[gi], gi == 0 ? hs : b->side[(gi - 1) % nside], nullptr,
-                           nullptr, nullptr));
+    RT_TRY(launch_rh_group(groups[gi], gi == 0 ? hs : b->side[(gi - 1) % nside], RhEvents{}));
   for (size_t k = 0; k < nside; ++k) {
     RT_TRY(hipEventRecord(b->forks[k + 1], b->side[k]));
     RT_TRY(hipStreamWaitEvent(hs, b->forks[k + 1], 0));

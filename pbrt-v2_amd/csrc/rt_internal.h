@@ -238,12 +238,17 @@ hipError_t launch_set_tleaf(float4* tmts, const uint32_t* tleaf, uint32_t ntri, 
 
 // Launchers (all asynchronous on `s`).
 hipError_t launch_fill_u8(uint8_t* p, uint8_t v, size_t n, hipStream_t s);
-// rayhierarchy / ray-bvh group: init, fused build, cluster (root) pass, persistent unit
-// kernel, per-ray kernel and, for closest hits, finalize and (rayhierarchy) repair.  When
-// given, t0 is recorded before the unit kernel, tm between the unit and per-ray kernels and
-// t1 after the per-ray kernel.
-hipError_t launch_rh_group(const RhGroup& G, hipStream_t s, hipEvent_t t0, hipEvent_t tm,
-                           hipEvent_t t1);
+// rayhierarchy / ray-bvh group: fused build, grazing pass, per-ray kernel and, for primary
+// rayhierarchy rays, repair.  With ray_clusters above 0: init, build, cluster (root) pass, with
+// ray_clusters above 1 the units' scan and pack, persistent unit kernel, per-ray kernel and, for
+// closest hits, finalize and repair.  Events that are given are recorded between.
+struct RhEvents {
+  hipEvent_t trace = nullptr;     // before the first traversal kernel: grazing pass or unit kernel
+  hipEvent_t ready = nullptr;     // before the unit or, without one, the per-ray kernel
+  hipEvent_t ray = nullptr;       // before the per-ray kernel
+  hipEvent_t ray_end = nullptr;   // after it
+};
+hipError_t launch_rh_group(const RhGroup& G, hipStream_t s, const RhEvents& ev);
 // Naive brute force from rays to hit records (mode 0, 1) or occlusion flags (mode 2); without
 // triangles every ray misses.  naive_rule: shading frames as the naive kernels take them.
 // merge: kNaiveMerge keys of scratch, used where several work-groups share out the triangles;

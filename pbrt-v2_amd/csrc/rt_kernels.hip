@@ -3338,8 +3338,8 @@ constexpr uint32_t kWalk64[8] = {24, 32, 16, 8, 4, 2, 1, 0};
 
 // Launch sequence of one rayhierarchy group with the mode and node type fixed.
 template <int MODE, int NODE>
-hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hipEvent_t tm,
-                             hipEvent_t t1) {
+hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, const RhEvents& ev) {
+  auto record = [&](hipEvent_t e) { return e ? hipEventRecord(e, s) : hipSuccess; };
   const bool direct = G.ray_clusters == 0;  // every block ray by ray, results written there
   if (!direct)
     hipLaunchKernelGGL((rh_init_kernel<MODE>), grid1(std::max<uint32_t>(G.nrays, kClaimQueues)),
@@ -3358,6 +3358,9 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
   else
     build(rh_group_build_kernel<MODE != 0, NODE == 2, false>,
           rh_single_build_kernel<MODE != 0, NODE == 2, false>);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess && direct) e = record(ev.trace);
+  if (e != hipSuccess) return e;
   if (direct) {
     if (G.graze) {
       const dim3 grid(std::min<uint32_t>(G.nblocks, kGrazeGrid));
@@ -3390,12 +3393,10 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
                                                  (kPackThreads / 64)),
                        dim3(kPackThreads), 0, s, G.bunits, G.nblocks, G.ustage, G.units, G.ctr);
   }
-  hipError_t e = hipGetLastError();
+  e = hipGetLastError();
+  if (e == hipSuccess && !direct) e = record(ev.trace);
+  if (e == hipSuccess) e = record(ev.ready);
   if (e != hipSuccess) return e;
-  if (t0) {
-    e = hipEventRecord(t0, s);
-    if (e != hipSuccess) return e;
-  }
   auto launch = [&](auto kernel) {
     const dim3 grid(G.grid > 0 ? (unsigned)G.grid : resident_grid(kernel, G.max_units));
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, s, G.items, G.units, G.ctr);
@@ -3410,11 +3411,8 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
   else
     launch(rh_unit_kernel<MODE, NODE, 256, 3>);
   e = hipGetLastError();
+  if (e == hipSuccess) e = record(ev.ray);
   if (e != hipSuccess) return e;
-  if (tm) {
-    e = hipEventRecord(tm, s);
-    if (e != hipSuccess) return e;
-  }
   auto launch_rays = [&](auto kernel) {
     unsigned spread = 0;
     const unsigned slots = resident_grid(kernel, 0x7fffffffu, 64);
@@ -3438,11 +3436,8 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, hipEvent_t t0, hip
     else launch_rays(ray_path_kernel<MODE, NODE, false, false>);
   }
   e = hipGetLastError();
+  if (e == hipSuccess) e = record(ev.ray_end);
   if (e != hipSuccess) return e;
-  if (t1) {
-    e = hipEventRecord(t1, s);
-    if (e != hipSuccess) return e;
-  }
   if (MODE != 2) {
     if (!direct)
       hipLaunchKernelGGL(rh_finalize_kernel, grid1(G.nrays), dim3(kThreads), 0, s, G.items,
@@ -3594,10 +3589,9 @@ hipError_t launch_fill_u8(uint8_t* p, uint8_t v, size_t n, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_rh_group(const RhGroup& G, hipStream_t s, hipEvent_t t0, hipEvent_t tm,
-                           hipEvent_t t1) {
+hipError_t launch_rh_group(const RhGroup& G, hipStream_t s, const RhEvents& ev) {
   if (G.nitems <= 0 || G.nrays == 0) return hipSuccess;
-#define RT_CALL(M, N) rh_group_dispatch<M, N>(G, s, t0, tm, t1)
+#define RT_CALL(M, N) rh_group_dispatch<M, N>(G, s, ev)
   if (G.node == 1) {
     if (G.mode == 0) return RT_CALL(0, 1);
     if (G.mode == 1) return RT_CALL(1, 1);
