@@ -277,9 +277,10 @@ int rt_batch_run(rt_batch *batch, void *stream);
 int rt_batch_set_param(rt_batch *batch, int32_t param, int32_t value);
 int rt_batch_get_param(rt_batch *batch, int32_t param, int32_t *value);
 /* Autotuner: times the batch's current jobs over the launch-shape candidates, `reps` runs
- * each, and keeps the fastest per mode: first the per-ray routing threshold x per-ray grid,
- * then clusters per work unit x persistent grid of the unit kernel.  No candidate changes a
- * result. */
+ * each, and keeps the fastest per mode: the routing (built-in or block path) with the per-ray
+ * grid, the per-ray walk, then clusters per work unit x persistent grid of the unit kernel and
+ * its tile.  A launch group is timed from its first launch to its last.  No candidate changes a
+ * result, but that the block path also finds what is said at RT_PARAM_RAY_CLUSTERS_*. */
 int rt_batch_autotune(rt_batch *batch, void *stream, int32_t reps);
 /* Event timing of the batch's traversal kernels, as rt_scene_set_timing / kernel_time. */
 int rt_batch_set_timing(rt_batch *batch, int32_t enable);

@@ -27,6 +27,7 @@ struct Timer {
     hipEvent_t a, m, b;
   };
   bool on = false;
+  bool whole = false;  // a and b around the whole launch group, m not recorded
   std::vector<Slot> slots;
   size_t used = 0;
   ~Timer() {
@@ -398,10 +399,15 @@ hipError_t timed_launch(Timer& tm, int mode, hipStream_t st, F fn) {
 
 hipError_t timed_group(Timer& tm, const RhGroup& G, hipStream_t st) {
   RhEvents ev;
-  if (const Timer::Slot* t = tm.next(G.mode, true, G.ray_clusters > 0)) {
-    ev.trace = t->a;
-    ev.ray = t->m;
-    ev.ray_end = t->b;
+  if (const Timer::Slot* t = tm.next(G.mode, !tm.whole, G.ray_clusters > 0)) {
+    if (tm.whole) {
+      ev.first = t->a;
+      ev.last = t->b;
+    } else {
+      ev.trace = t->a;
+      ev.ray = t->m;
+      ev.ray_end = t->b;
+    }
   }
   return launch_rh_group(G, st, ev);
 }
@@ -1444,7 +1450,9 @@ int rt_batch_get_param(rt_batch* b, int32_t param, int32_t* value) {
 }  // extern "C"
 
 // Times the batch over `cands` launch-shape candidates (each applies itself to b->prm for
-// both modes) and keeps, per mode, the fields `keep` copies from the fastest candidate.
+// both modes) and keeps, per mode, the fields `keep` copies from the fastest candidate.  Launch
+// groups are timed whole, from the first launch to the last, since candidates differ in which
+// launches they need.
 template <class Apply, class Keep>
 static int autotune_stage(rt_batch* b, hipStream_t hs, int reps, int ncand, Apply apply,
                           Keep keep) {
@@ -1493,16 +1501,18 @@ int rt_batch_autotune(rt_batch* b, void* stream, int32_t reps) {
   const bool was_graph = b->use_graph;
   b->use_graph = false;
   b->timer.on = true;
-  // stage 1: which blocks take the per-ray path (0: all, 2^30: none) and the per-ray grid
-  // (one wavefront per work-group: 8 or 16 per CU, or every resident slot)
-  static const int kRay[] = {0, 64, 256, 1 << 29, 1 << 30};
-  static const int kRGrid[] = {0, 2048, 4096};
+  b->timer.whole = true;
+  // stage 1: whether blocks take the per-ray path (0: all, 2^30: none) and the per-ray grid (one
+  // wavefront per work-group: 8 or 16 per CU, or every resident slot).  Thresholds between would
+  // send blocks that way without the grazing pass, whose hits a tuned batch must not lose.
+  static const int kRay[] = {0, 0, 0, 1 << 30};
+  static const int kRGrid[] = {0, 2048, 4096, 0};
   auto routing = [&]() {
     return autotune_stage(
-        b, hs, reps, 5 * 3,
+        b, hs, reps, 4,
         [&](int c, RhParams& p) {
-          p.ray[0] = p.ray[1] = kRay[c / 3];
-          p.rgrid[0] = p.rgrid[1] = kRGrid[c % 3];
+          p.ray[0] = p.ray[1] = kRay[c];
+          p.rgrid[0] = p.rgrid[1] = kRGrid[c];
         },
         [](int m, const RhParams& p, RhParams& o) {
           o.ray[m] = p.ray[m];
@@ -1516,9 +1526,7 @@ int rt_batch_autotune(rt_batch* b, void* stream, int32_t reps) {
     st = autotune_stage(
         b, hs, reps, 4, [&](int c, RhParams& p) { p.walk[0] = p.walk[1] = kWalk[c]; },
         [](int m, const RhParams& p, RhParams& o) { o.walk[m] = p.walk[m]; });
-  // stage 1 again with the walk just chosen: a faster per-ray kernel can move the best split
-  // between the two paths (on a batch of 64 cluster scenes it then sent every camera block
-  // per-ray: 7.65 ms per step against 7.73)
+  // stage 1 again with the walk just chosen, which can make the per-ray path the faster one
   if (!st) st = routing();
   // stage 3: passing clusters per work unit x persistent grid of the unit kernel
   static const int kPer[] = {2, 4, 8, 16, 32};
@@ -1540,6 +1548,7 @@ int rt_batch_autotune(rt_batch* b, void* stream, int32_t reps) {
         b, hs, reps, 2, [&](int c, RhParams& p) { p.tile[0] = p.tile[1] = c; },
         [](int m, const RhParams& p, RhParams& o) { o.tile[m] = p.tile[m]; });
   b->timer.on = was_on;
+  b->timer.whole = false;
   b->timer.used = 0;
   b->use_graph = was_graph;
   b->graph_valid = false;

@@ -243,10 +243,12 @@ hipError_t launch_fill_u8(uint8_t* p, uint8_t v, size_t n, hipStream_t s);
 // ray_clusters above 1 the units' scan and pack, persistent unit kernel, per-ray kernel and, for
 // closest hits, finalize and repair.  Events that are given are recorded between.
 struct RhEvents {
+  hipEvent_t first = nullptr;     // before the group's first launch
   hipEvent_t trace = nullptr;     // before the first traversal kernel: grazing pass or unit kernel
   hipEvent_t ready = nullptr;     // before the unit or, without one, the per-ray kernel
   hipEvent_t ray = nullptr;       // before the per-ray kernel
   hipEvent_t ray_end = nullptr;   // after it
+  hipEvent_t last = nullptr;      // after the group's last launch
 };
 hipError_t launch_rh_group(const RhGroup& G, hipStream_t s, const RhEvents& ev);
 // Naive brute force from rays to hit records (mode 0, 1) or occlusion flags (mode 2); without

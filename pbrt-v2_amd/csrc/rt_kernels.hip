@@ -3340,6 +3340,8 @@ constexpr uint32_t kWalk64[8] = {24, 32, 16, 8, 4, 2, 1, 0};
 template <int MODE, int NODE>
 hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, const RhEvents& ev) {
   auto record = [&](hipEvent_t e) { return e ? hipEventRecord(e, s) : hipSuccess; };
+  hipError_t e = record(ev.first);
+  if (e != hipSuccess) return e;
   const bool direct = G.ray_clusters == 0;  // every block ray by ray, results written there
   if (!direct)
     hipLaunchKernelGGL((rh_init_kernel<MODE>), grid1(std::max<uint32_t>(G.nrays, kClaimQueues)),
@@ -3358,7 +3360,7 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, const RhEvents& ev
   else
     build(rh_group_build_kernel<MODE != 0, NODE == 2, false>,
           rh_single_build_kernel<MODE != 0, NODE == 2, false>);
-  hipError_t e = hipGetLastError();
+  e = hipGetLastError();
   if (e == hipSuccess && direct) e = record(ev.trace);
   if (e != hipSuccess) return e;
   if (direct) {
@@ -3446,7 +3448,8 @@ hipError_t rh_group_dispatch(const RhGroup& G, hipStream_t s, const RhEvents& ev
       hipLaunchKernelGGL((rh_repair_kernel<NODE>), dim3(64), dim3(kThreads), 0, s, G.items,
                          G.nitems, G.ctr, G.replist);
   }
-  return hipGetLastError();
+  e = hipGetLastError();
+  return e == hipSuccess ? record(ev.last) : e;
 }
 
 // See launch_graze_records.
