@@ -692,9 +692,6 @@ int rh_prepare(RhWorkspace& ws, const std::vector<RhJob>& jobs, const RhParams& 
 }  // namespace
 
 namespace rti {
-uint32_t scene_nclusters(const rt_scene* s) {
-  return s->desc.kind == RT_ACCEL_RAYBVH ? s->nrclusters : s->nclusters;
-}
 int scene_check_image(const rt_scene* s, int W, int H) {
   if (s->desc.kind != RT_ACCEL_RAYHIERARCHY && s->desc.kind != RT_ACCEL_RAYBVH)
     return RT_ERR_UNSUPPORTED;
@@ -704,6 +701,18 @@ int scene_check_image(const rt_scene* s, int W, int H) {
     return RT_ERR_UNSUPPORTED;
   if (s->ntri >= (1u << 26)) return RT_ERR_UNSUPPORTED;
   return RT_OK;
+}
+uint64_t scene_scratch(const rt_scene* s, int W, int H) {
+  RHGeom g;
+  if (rh_geometry(W, H, s->desc.chunk_x, s->desc.chunk_y, s->desc.height, &g)) return 0;
+  // per trace the hierarchy, a word per block for the list of those the grazing pass slices and,
+  // where it takes them, one for what it found; closest hits a seed a ray, primary ones of a
+  // rayhierarchy the list of rays to repair (rh_prepare)
+  const uint64_t n = (uint64_t)W * H, ntop = (uint64_t)g.ntop;
+  const bool graze = graze_shape(g);
+  const uint64_t both = sizeof(float4) * 4 * (uint64_t)g.nnodes + sizeof(uint32_t) * ntop * (graze ? 2 : 1);
+  return 2 * both + (graze ? sizeof(uint64_t) * n : 0) +
+         (s->desc.kind == RT_ACCEL_RAYHIERARCHY && s->desc.repair_run > 0 ? sizeof(uint32_t) * n : 0);
 }
 }  // namespace rti
 

@@ -15,9 +15,9 @@ struct rt_scene;
 
 namespace rti {
 
-// Clusters a block's cluster pass tests: Morton clusters of triangles (rayhierarchy) or of
-// frontier roots (ray-bvh); 0 for naive scenes.
-uint32_t scene_nclusters(const rt_scene* s);
+// Scratch in bytes of tracing a W x H image of primary rays and one of shadow rays on `s` with the
+// built-in routing, where scene_check_image accepts it.
+uint64_t scene_scratch(const rt_scene* s, int W, int H);
 // RT_OK when `s` can trace a W x H ray image through the batched form (a rayhierarchy or
 // ray-bvh scene with its BVH, a hierarchy shape the kernels support), else the status the
 // batch would return.

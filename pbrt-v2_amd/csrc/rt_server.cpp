@@ -434,11 +434,10 @@ int rt_server_submit(rt_server* S, const rt_request* q, uint64_t* ticket) {
   r->q = *q;
   r->n = (size_t)n;
   r->block = block_bytes(r->n);
-  // traversal scratch in the batch: keys and repair keys (12 B/ray), hierarchy nodes
-  // (< 64 B per 12 rays), passing-cluster lists (4 B per block and cluster), work units
-  const uint64_t blocks = (n + 255) / 256;
-  const uint64_t ncl = rti::scene_nclusters(S->scenes[q->scene]);
-  r->charge = r->block + 12 * n + 6 * n + blocks * ncl * 4 + blocks * (ncl / 2 + 1) * 16;
+  // traversal scratch in the two batches, whose arenas grow by a quarter more than they need
+  const uint64_t scratch =
+      rti::scene_scratch(S->scenes[q->scene], q->width * q->spp, q->height);
+  r->charge = r->block + scratch + scratch / 4;
   r->st.primary_rays = n;
   r->st.submit_s = now_s();
   {
