@@ -100,10 +100,13 @@ def timed(fn, steps, warmup, stream, label):
 def bound_of(facts, hbm_meas, hbm_alg, valu_frac):
     """The roof that limits the kernel.  From the profiled counters when they are recorded:
     HBM when the measured DRAM traffic uses a larger share of its peak than the VALU is busy,
-    else VALU.  Without them, the same comparison of the algorithmic model's shares."""
+    else VALU.  Without them, the same comparison of the algorithmic model's shares; None where
+    the model has no count of operations."""
     busy = facts.get("valu-busy")
     if busy is not None and hbm_meas is not None:
         return "hbm" if hbm_meas >= busy else "valu"
+    if valu_frac is None:
+        return None
     return "hbm" if hbm_alg >= valu_frac else "valu"
 
 
@@ -122,14 +125,15 @@ def per_ray_roofline(name, t_ms, rays, ntri, mode, workload, st=None):
     hbm_meas = None if traffic is None else traffic / (t_ms * 1e-3) / 1e9 / HBM_PEAK_GBS
     valu = {"busy_measured": facts.get("valu-busy"),
             "lane_utilisation_measured": facts.get("lane-utilisation")}
-    out = {"bound": bound_of(facts, hbm_meas, achieved / HBM_PEAK_GBS, 1.0), "kernel": name,
+    flops = None if st is None else 24 * st.visits + 45 * st.tests + 60 * st.culls
+    tflops = None if st is None else flops / (t_ms * 1e-3) / 1e12
+    valu_frac = None if st is None else tflops / FP32_UNPACKED_TFLOPS
+    out = {"bound": bound_of(facts, hbm_meas, achieved / HBM_PEAK_GBS, valu_frac), "kernel": name,
            "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
            "frac": round(achieved / HBM_PEAK_GBS, 4),
            "traffic": None if traffic is None else int(traffic),
            "bytes_per_launch": int(b), "ms_per_launch": round(t_ms, 4), "valu": valu}
     if st is not None:
-        flops = 24 * st.visits + 45 * st.tests + 60 * st.culls
-        tflops = flops / (t_ms * 1e-3) / 1e12
         out["counts_binary_tree"] = {"rays": int(st.rays), "node_loads": int(st.visits),
                                      "leaf_tests": int(st.tests), "chain_culls": int(st.culls),
                                      "chains": int(st.chains)}
