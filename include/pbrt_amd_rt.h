@@ -11,7 +11,7 @@
  *
  * Memory: scenes (triangles, UVs, the ray-bvh BVH) are copied once into device memory and
  * stay resident until rt_scene_destroy.  Ray and hit arrays passed to the trace calls are
- * DEVICE pointers owned by the caller; scratch (the ray hierarchy, reduction keys) is owned
+ * DEVICE pointers owned by the caller; scratch (the ray hierarchy, keys, seeds) is owned
  * by the scene and grows on demand.  Calls on one scene must not overlap in time.
  */
 #ifndef PBRT_AMD_RT_H
@@ -161,7 +161,7 @@ int rt_trace_occluded(rt_scene *scene, const rt_rays *rays, uint8_t *occluded, v
 /* rt_trace_closest without any device allocation.  No counterpart in the reference: it is for
  * callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  Same arguments and the same results as rt_trace_closest; its
- * scratch (hierarchy, reduction keys, work queue, job table) lives in a static device array of
+ * scratch (hierarchy, the grazing pass's seeds and block words, job table) lives in a static device array of
  * 64 MiB per device, set up by rt_ctx_create and held until the process ends.  A call needs
  * at most about 22 bytes per ray, its hierarchy included, so up to about 3 million rays; a
  * larger one returns RT_ERR_TOO_LARGE (naive, which uses none of it: beyond 8 bytes per ray).

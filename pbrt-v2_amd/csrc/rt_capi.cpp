@@ -1119,8 +1119,7 @@ int rt_trace_closest_noalloc(rt_scene* s, const rt_rays* rays, int32_t mode, con
                               s->d_merge, out, nullptr, hs));
     return RT_OK;
   }
-  // rayhierarchy / ray-bvh: one job whose blocks all take the per-ray path (the same result as
-  // the block path), so no cluster lists are needed
+  // rayhierarchy / ray-bvh: one job in the built-in routing, so no cluster lists are needed
   RhItem it;
   st = fill_item(RhJob{s, r, mode, out, nullptr}, it);
   if (st) return st;
@@ -1134,8 +1133,8 @@ int rt_trace_closest_noalloc(rt_scene* s, const rt_rays* rays, int32_t mode, con
   };
   RhItem* table = (RhItem*)take(sizeof(RhItem));
   it.nodes = (float4*)take(sizeof(float4) * 4 * (size_t)it.g.nnodes);
-  // reduction keys and queues, which this form once used and no longer does: the sizes that it
-  // takes and refuses stay the ones its declaration promises
+  // the grazing pass's seeds; what else is taken keeps the sizes that this form accepts and
+  // refuses the ones its declaration promises
   uint64_t* const gseed = (uint64_t*)take(sizeof(uint64_t) * n);
   if (repair) take(sizeof(uint32_t) * n);
   take(sizeof(uint4));
@@ -1313,7 +1312,8 @@ static int batch_launch_forked(rt_batch* b, const std::vector<RhGroup>& groups, 
   if (groups.size() < 2 || nside == 0) return batch_launch(b, groups, hs, false);
   // A first group that fills the device forks after its build and grazing pass, so that its traversal takes the device first
   // and the others' fill in behind it; forked at the start, two such traversals split the
-  // device between them (twelve scenes: 838 us a step against 738).
+  // device between them (twelve scenes, before the grazing pass: 778 us a step
+  // against 738).
   const bool late = groups[0].max_chunks > kForkLateChunks;
   RhEvents fork;
   fork.ready = b->forks[0];

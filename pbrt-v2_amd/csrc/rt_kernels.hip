@@ -11,6 +11,8 @@
 // Work decomposition of a rayhierarchy / ray-bvh trace (a launch group of one or more jobs):
 //   build     one 256-thread work-group per top-level hierarchy node ("block") builds the
 //             block's leaves and levels from its rays and clears the group's counters;
+//   graze     in coherent blocks, work-groups list the triangles that a ray of the block may
+//             graze, where the search tree finds no hits that only rounding gives, and test them;
 //   ray path  wavefronts take 64-ray chunks of every block, walk each ray through a search tree
 //             of the triangles and write its hit record or occlusion flag;
 //   repair    the reference's repairRun pass for the rays that were listed for it.
